@@ -11,8 +11,10 @@
 //
 // The candidate loop of one cell is sequential in the reference: the running
 // (sigma g w)_max is updated before every acceptance test, and particles
-// created by a split become candidates of the same loop.  Each cell is
-// therefore one lane; cells run in parallel.  Draw order per cell stream:
+// created by a split become candidates of the same loop.  Cells run in
+// parallel, a cell with several candidates on a wavefront that evaluates them
+// ahead (ntc_windows), other cells and replayed draws one lane each.  Draw
+// order per cell stream:
 // [n_coll], then per candidate [i, k (, k redraws)], [accept] if g > eps,
 // [phi, cos theta] if accepted.
 //
@@ -208,6 +210,54 @@ __device__ __forceinline__ bool ntc_candidate(const NtcArgs &A, const int c, con
     return true;
 }
 
+// One candidate of cell c's swpm! loop (collision_swpm.jl:201-288); false
+// when a replay row ran out.  S.sgwm is (sigma g)_max, S.ca the created.
+template <class Draw>
+__device__ __forceinline__ bool swpm_candidate(const NtcArgs &A, const int c, const NtcCell &C, NtcState &S, Draw &dr,
+                                               const double wtf, const double inv_w_max) {
+    const int32_t i = (int32_t)floor(dr.next() * (double)S.na);
+    int32_t k = (int32_t)floor(dr.next() * (double)S.na);
+    while (i == k) {
+        k = (int32_t)floor(dr.next() * (double)S.na);
+        if (dr.exhausted()) return false;   // replay row exhausted
+    }
+    const PRef pi = ntc_ref_a(A, c, C, i), pk = ntc_ref_a(A, c, C, k);
+    const double vi0 = pi.v0[pi.i], vi1 = pi.v1[pi.i], vi2 = pi.v2[pi.i];
+    const double vk0 = pk.v0[pk.i], vk1 = pk.v1[pk.i], vk2 = pk.v2[pk.i];
+    double g0, g1, g2;
+    const double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
+    if (!(g > MZ_G_EPS)) return true;
+    const double sgm = mz_vhs_sgw(A.factor, A.expo, g, 1.0, 1.0);   // sigma g
+    S.sgwm = sgm > S.sgwm ? sgm : S.sgwm;
+    const double wi = pi.w[pi.i], wk = pk.w[pk.i];
+    if (!(dr.next() < sgm * (wi > wk ? wi : wk) * inv_w_max / S.sgwm)) return true;
+    ++S.performed;
+    double vc0, vc1, vc2;
+    mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
+    const double dw = (wi < wk ? wi : wk) * wtf;
+    pi.w[pi.i] = wi - dw;
+    pk.w[pk.i] = wk - dw;
+    if (S.ca + 1 >= 2 * C.n_coll) {
+        atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
+        return true;
+    }
+    const PRef n_i = pref_scratch(A, 0, C.s_base + S.ca), n_k = pref_scratch(A, 0, C.s_base + S.ca + 1);
+    n_i.x0[n_i.i] = pi.x0[pi.i]; n_i.x1[n_i.i] = pi.x1[pi.i]; n_i.x2[n_i.i] = pi.x2[pi.i];
+    n_k.x0[n_k.i] = pk.x0[pk.i]; n_k.x1[n_k.i] = pk.x1[pk.i]; n_k.x2[n_k.i] = pk.x2[pk.i];
+    n_i.w[n_i.i] = dw;
+    n_k.w[n_k.i] = dw;
+    S.ca += 2;
+    S.na += 2;
+    // scatter_vhs! on the two new particles: phi first, then cos(theta)
+    const double R_phi = dr.next();
+    const double R_ct = dr.next();
+    double ui0, ui1, ui2, uk0, uk1, uk2;
+    mz_vhs_post(A.mu1, A.mu2, g, vc0, vc1, vc2, R_phi, R_ct, ui0, ui1, ui2, uk0, uk1, uk2);
+    n_i.v0[n_i.i] = ui0; n_i.v1[n_i.i] = ui1; n_i.v2[n_i.i] = ui2;
+    n_k.v0[n_k.i] = uk0; n_k.v1[n_k.i] = uk1; n_k.v2[n_k.i] = uk2;
+    return true;
+}
+
 // The end of a cell's loop: (sigma g w)_max, the counters, created counts.
 __device__ __forceinline__ void ntc_finish_cell(const NtcArgs &A, const int c, const NtcCell &C,
                                                 const NtcState &S) {
@@ -222,18 +272,6 @@ __device__ __forceinline__ void ntc_finish_cell(const NtcArgs &A, const int c, c
         A.created[c] = A.single ? S.ca + S.cb : S.ca;
         A.created[(int64_t)(A.cell_hi + 1) + c] = A.single ? 0 : S.cb;
     }
-}
-
-// The candidate loop of cell c with the draws of its stream from dr (next(),
-// seek(k), exhausted()).
-template <class Draw>
-__device__ __forceinline__ void ntc_cell(const NtcArgs &A, const int c, Draw &dr) {
-    NtcCell C;
-    NtcState S;
-    ntc_setup(A, c, dr, C, S);
-    for (int64_t cc = 0; cc < C.n_coll; ++cc)
-        if (!ntc_candidate(A, c, C, S, dr)) return;
-    ntc_finish_cell(A, c, C, S);
 }
 
 // Draws of a cell's stream for one lane: mz_rand.
@@ -266,151 +304,316 @@ struct NtcWaveDraw {
     }
     __device__ bool exhausted() const { return false; }
     __device__ void seek(uint64_t kk) { k = kk; }
-    // the block holds draws D .. D + 67 afterwards
-    __device__ void cover(uint64_t D) {
-        if (D < base || D + 68 > base + 128) {
+    // the block holds draws D .. D + span - 1 afterwards (span <= 127)
+    __device__ void cover(uint64_t D, int span) {
+        if (D < base || D + (uint64_t)span > base + 128) {
             base = D & ~(uint64_t)1;
             mz_philox_pair(rp, stream, (base >> 1) + (uint64_t)(threadIdx.x & 63), h0, h1);
         }
     }
-    // draw s for this lane (s may differ between lanes; base <= s < base + 128)
-    __device__ double at(uint64_t s) const {
-        const uint64_t idx = s - base;
-        const int l = (int)(idx >> 1);
+    // draw base + idx for this lane (idx may differ between lanes; idx < 128)
+    __device__ double at(int idx) const {
+        const int l = idx >> 1;
         const double a = __shfl(h0, l, 64), b = __shfl(h1, l, 64);
         return (idx & 1) ? b : a;
     }
 };
 
-// ntc_cell for a single-species cell on a whole wavefront with Philox
-// draws, with the candidates evaluated ahead: at a window's start at draw D,
-// lane L evaluates the candidate that would start at draw D + L (pair,
-// relative speed, (sigma g w), the acceptance test under the window's
-// (sigma g w)_max, post-collision velocities); the wave then walks the
-// candidates in the reference's order on uniform values.  Each starts where
-// the previous one ended, (sigma g w)_max is updated before its acceptance
-// test, and a lane's test is taken only while (sigma g w)_max is unchanged
-// (the same operands, so the same result).  A candidate whose k is redrawn,
-// or that shares a particle with a collision earlier in the window, is
-// evaluated directly and a new window starts after it; so does a split,
-// which changes n_local and with it every later pair.  The results are
-// ntc_cell's.
-__device__ void ntc_cell_spec(const NtcArgs &A, const int c, NtcWaveDraw &dr) {
+// A cell's candidate loop on a whole wavefront (Philox draws), candidates
+// evaluated ahead.  A candidate that is rejected takes three draws and one
+// that collides takes five, and a collision of unequal weights adds a known
+// number of particles to the cell, so the candidate reached after `a`
+// collisions and `r` rejections of a window that starts at draw D begins at
+// draw D + 5 a + 3 r and picks from na0 + inc a particles.  A window
+// evaluates that lattice: lane a M + j takes the candidate after a
+// collisions and j rejections (T tracks of M candidates, T M <= 64) -- pair,
+// relative speed, collision rate, acceptance test, post-collision
+// velocities.  The wave then walks it in the reference's order, jumping from
+// event to event with ballots: rejections in between need no work, a
+// collision moves to the next track, a new (sigma g w)_max renews every
+// lane's acceptance test.  The window ends, and the next one starts at that
+// draw, at a candidate that shares a particle with a collision of the window
+// or picks one created in it, where the particle count is not the predicted
+// one, and where a track or the tracks run out; T follows the acceptance
+// rate (doubled when the tracks run out, halved when a track does).  A
+// candidate whose k must be drawn again runs on its own.  Same draws, same
+// operands, same order of updates as the loop over ntc_candidate: the results
+// are equal.
+//
+// What bounds it: the latency of one window (draw exchange, the two gathers,
+// the power chain; about 4 us) times the windows of the cell with the most.
+// Few acceptances make windows of 40 candidates, many make eight tracks of
+// eight.  Measured against one lane per cell, and against windows that ended
+// at every split: 8,192 boxes of 90 particles with 130 candidates, 8% accepted,
+// 4,030 -> 330 us a call; 2,048 boxes with 580 candidates (up to 3,500), 4%
+// accepted, SWPM, 5,560 -> 285 us; 4,096 boxes with 150 candidates, 39%
+// accepted, SWPM, 1,220 -> 190 us; 1,024 cells of up to 30,000 particles, 290
+// candidates (up to 2,900), 40% accepted, 3,250 -> 1,320 us; 500 cells of 35
+// candidates, 5% accepted, 46 -> 22 us.
+#define NTC_T1_LEN 40   // candidates of a single track (its draws fit the 128 held)
+
+enum { NTC_PLAIN = 0, NTC_SPLIT = 1, NTC_SWPM = 2 };   // no particles created; ntc! with splitting; swpm!
+
+template <int KIND>
+__device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const NtcCell &C, NtcState &S,
+                                            NtcWaveDraw &dr, const double wtf, const double inv_w_max) {
+    constexpr bool SWPM = KIND == NTC_SWPM, CREATES = KIND != NTC_PLAIN;
     const int lane = threadIdx.x & 63;
-    NtcCell C;
-    NtcState S;
-    ntc_setup(A, c, dr, C, S);
+    const bool single = SWPM || A.single;
+    const int32_t st1a = A.a.pia.start1[c] - 1, st2a = A.a.pia.start2[c] - 1;
+    const int32_t st1b = A.b.pia.start1[c] - 1, st2b = A.b.pia.start2[c] - 1;
+    const int64_t sc_b = !CREATES || single ? 0 : A.sc_cap;   // species half 1 of the scratch
+    int T = 4;
+    int32_t inc = SWPM ? 2 : (CREATES && single ? 1 : 0);
     int64_t cc = 0;
-    uint64_t o = dr.k;   // the next draw of the stream
+    uint64_t o = dr.k;
     while (cc < C.n_coll) {
         const uint64_t D = o;
-        dr.cover(D);
-        const int32_t na0 = S.na;
-        const double sgwm0 = S.sgwm;
-        const uint64_t sL = D + (uint64_t)lane;
-        const double d0 = dr.at(sL), d1 = dr.at(sL + 1), d2 = dr.at(sL + 2), d3 = dr.at(sL + 3), d4 = dr.at(sL + 4);
-        const int32_t si = (int32_t)floor(d0 * (double)na0), sk = (int32_t)floor(d1 * (double)na0);
-        double swi, swk, sgw, vi0, vi1, vi2, vk0, vk1, vk2, ui0, ui1, ui2, uk0, uk1, uk2;
-        int32_t f;
-        {
-            const PRef pi = ntc_ref_a(A, c, C, si), pk = ntc_ref_a(A, c, C, sk);
-            vi0 = pi.v0[pi.i]; vi1 = pi.v1[pi.i]; vi2 = pi.v2[pi.i];
-            vk0 = pk.v0[pk.i]; vk1 = pk.v1[pk.i]; vk2 = pk.v2[pk.i];
-            swi = pi.w[pi.i];
-            swk = pk.w[pk.i];
+        const int M = T == 1 ? NTC_T1_LEN : 64 / T;
+        dr.cover(D, 5 * (T - 1) + 3 * (M - 1) + 5);
+        const int32_t na0 = S.na, nb0 = single ? S.na : S.nb;
+        const int a_l = T == 1 ? 0 : lane / M;
+        const int j_l = lane - a_l * M;
+        const int64_t cand = cc + a_l + j_l;
+        const bool live = j_l < M && cand < C.n_coll;
+        const int idx = min((int)(D - dr.base) + 5 * a_l + 3 * j_l, 123);
+        const double d0 = dr.at(idx), d1 = dr.at(idx + 1), d2 = dr.at(idx + 2), d3 = dr.at(idx + 3),
+                     d4 = dr.at(idx + 4);
+        const int32_t si = (int32_t)floor(d0 * (double)(na0 + inc * a_l));
+        const int32_t sk = (int32_t)floor(d1 * (double)(nb0 + inc * a_l));
+        const bool fresh = si >= na0 || sk >= nb0;   // created in this window (or out of range by rounding)
+        const bool same = single && si == sk;
+        bool slow = false;                            // g <= eps: no acceptance draw
+        double vi0 = 0.0, vi1 = 0.0, vi2 = 0.0, vk0 = 0.0, vk1 = 0.0, vk2 = 0.0, wi = 0.0, wk = 0.0;
+        double sg = 0.0, t = 0.0;                     // rate entering the running maximum; acceptance numerator
+        double ui0 = 0.0, ui1 = 0.0, ui2 = 0.0, uk0 = 0.0, uk1 = 0.0, uk2 = 0.0;
+        double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0, xk0 = 0.0, xk1 = 0.0, xk2 = 0.0;
+        const bool in_i = !CREATES || si < C.nla, in_k = !CREATES || sk < C.nlb;
+        const int64_t pi = in_i ? (int64_t)(si < C.n1a ? st1a + si : st2a + (si - C.n1a)) : C.s_base + (si - C.nla);
+        const int64_t pk = in_k ? (int64_t)(sk < C.n1b ? st1b + sk : st2b + (sk - C.n1b))
+                                : sc_b + C.s_base + (sk - C.nlb);
+        double sgwm = S.sgwm;
+        bool acc = false;
+        if (live && !fresh && !same) {
+            vi0 = (in_i ? A.a.v0 : A.sc[3])[pi]; vk0 = (in_k ? A.b.v0 : A.sc[3])[pk];
+            vi1 = (in_i ? A.a.v1 : A.sc[4])[pi]; vk1 = (in_k ? A.b.v1 : A.sc[4])[pk];
+            vi2 = (in_i ? A.a.v2 : A.sc[5])[pi]; vk2 = (in_k ? A.b.v2 : A.sc[5])[pk];
+            wi = (in_i ? A.a.w : A.sc[6])[pi];
+            wk = (in_k ? A.b.w : A.sc[6])[pk];
+            // the direction needs the draws only: it is worked out while the
+            // loads are in flight, for every candidate
+            double e0, e1, e2;
+            mz_vhs_dir(d3, d4, e0, e1, e2);
             double g0, g1, g2;
             const double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
-            sgw = mz_vhs_sgw(A.factor, A.expo, g, swi, swk);
-            f = (si == sk ? 1 : 0) | (g > MZ_G_EPS ? 2 : 0) | (sgw > sgwm0 ? 4 : 0) | (d2 < sgw / sgwm0 ? 8 : 0);
-            double vc0, vc1, vc2;
-            mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
-            mz_vhs_post(A.mu1, A.mu2, g, vc0, vc1, vc2, d3, d4, ui0, ui1, ui2, uk0, uk1, uk2);
+            slow = !(g > MZ_G_EPS);
+            if (SWPM) {
+                sg = mz_vhs_sgw(A.factor, A.expo, g, 1.0, 1.0);
+                t = sg * (wi > wk ? wi : wk) * inv_w_max;
+            } else {
+                sg = mz_vhs_sgw(A.factor, A.expo, g, wi, wk);
+                t = sg;
+            }
+            // every candidate that can be accepted: a larger maximum only
+            // lowers t / (sigma g w)_max
+            acc = d2 < t / sgwm;
+            if (acc) {
+                if (SWPM || (CREATES && wi > wk)) {
+                    xi0 = (in_i ? A.a.x0 : A.sc[0])[pi]; xi1 = (in_i ? A.a.x1 : A.sc[1])[pi];
+                    xi2 = (in_i ? A.a.x2 : A.sc[2])[pi];
+                }
+                if (SWPM || (CREATES && wk > wi)) {
+                    xk0 = (in_k ? A.b.x0 : A.sc[0])[pk]; xk1 = (in_k ? A.b.x1 : A.sc[1])[pk];
+                    xk2 = (in_k ? A.b.x2 : A.sc[2])[pk];
+                }
+                double vc0, vc1, vc2;
+                mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
+                mz_vhs_along(A.mu1, A.mu2, g, vc0, vc1, vc2, e0, e1, e2, ui0, ui1, ui2, uk0, uk1, uk2);
+            }
         }
-        // walk the window; lane j < nd holds a particle that collided in it
-        int32_t dirty = -1;
-        int nd = 0;
-        bool direct = false;
-        while (cc < C.n_coll) {
-            const int L = (int)(o - D);
-            if (L >= 60 || nd >= 62) break;
-            const int32_t i = __builtin_amdgcn_readlane(si, L), k = __builtin_amdgcn_readlane(sk, L);
-            const int32_t fl = __builtin_amdgcn_readlane(f, L);
-            if ((fl & 1) || __ballot(lane < nd && (dirty == i || dirty == k))) {
+        // lanes at which the window ends before their candidate
+        uint64_t stop = __ballot(live && fresh);
+        const uint64_t end = __ballot(!live), samem = __ballot(live && same && !fresh), slowm = __ballot(slow);
+        const uint64_t eqm = __ballot(A.equal_weight || fabs(wi - wk) < A.dw_tol), heavym = __ballot(wi > wk);
+        uint64_t accm = __ballot(acc), maxm = __ballot(sg > sgwm);
+        int a = 0, j = 0;
+        bool direct = false, at_o = false, ran_out = false;
+        for (;;) {
+            if (j >= M) {   // the track ran out
+                ran_out = true;
+                break;
+            }
+            const int at0 = a * M + j;
+            uint64_t track = ~0ull << at0;
+            if (a * M + M < 64) track &= (1ull << (a * M + M)) - 1;
+            const uint64_t hit = (stop | end | samem | slowm | accm | maxm) & track;
+            if (!hit) {
+                cc += M - j;
+                j = M;
+                continue;
+            }
+            const int L = __ffsll((unsigned long long)hit) - 1;
+            const uint64_t bit = 1ull << L;
+            cc += L - at0;
+            j += L - at0;
+            if ((stop | end) & bit) break;
+            if (samem & bit) {
                 direct = true;
                 break;
             }
-            if (!(fl & 2)) {   // g <= eps: no acceptance draw
-                o += 2;
-                ++cc;
-                continue;
-            }
-            bool acc;
-            if (!(fl & 4) && S.sgwm == sgwm0) {
-                acc = (fl & 8) != 0;
-            } else {
-                const double sl = mz_readlane_d(sgw, L);
-                S.sgwm = sl > S.sgwm ? sl : S.sgwm;
-                acc = mz_readlane_d(d2, L) < sl / S.sgwm;
-            }
-            if (!acc) {
-                o += 3;
-                ++cc;
-                continue;
-            }
-            const double wi = mz_readlane_d(swi, L), wk = mz_readlane_d(swk, L);
-            if (!ntc_split_room(A, C, S, wi, wk)) {
-                ++S.performed;
-                o += 3;
-                ++cc;
-                continue;
-            }
-            const int32_t na_before = S.na;
-            ntc_collide(A, C, S, ntc_ref_a(A, c, C, i), ntc_ref_a(A, c, C, k), mz_readlane_d(vi0, L),
-                        mz_readlane_d(vi1, L), mz_readlane_d(vi2, L), mz_readlane_d(vk0, L), mz_readlane_d(vk1, L),
-                        mz_readlane_d(vk2, L), wi, wk, mz_readlane_d(ui0, L), mz_readlane_d(ui1, L),
-                        mz_readlane_d(ui2, L), mz_readlane_d(uk0, L), mz_readlane_d(uk1, L), mz_readlane_d(uk2, L));
-            if (lane == nd) dirty = i;
-            if (lane == nd + 1) dirty = k;
-            nd += 2;
-            o += 5;
             ++cc;
-            if (S.na != na_before) break;   // a split changed n_local
+            if (slowm & bit) {
+                o = D + (uint64_t)(5 * a + 3 * j + 2);
+                at_o = true;
+                break;
+            }
+            if (maxm & bit) {
+                sgwm = mz_readlane_d(sg, L);   // above the running maximum
+                accm = __ballot(acc && d2 < t / sgwm);
+                maxm = __ballot(sg > sgwm);
+            }
+            if (!(accm & bit)) {
+                ++j;
+                continue;
+            }
+            if (SWPM) {
+                ++S.performed;
+                const double dw = (wi < wk ? wi : wk) * wtf;
+                if (lane == L) {
+                    (in_i ? A.a.w : A.sc[6])[pi] = wi - dw;
+                    (in_k ? A.b.w : A.sc[6])[pk] = wk - dw;
+                }
+                if (S.ca + 1 >= 2 * C.n_coll) {
+                    if (lane == 0) atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
+                    o = D + (uint64_t)(5 * a + 3 * j + 3);
+                    at_o = true;
+                    break;
+                }
+                if (lane == L) {
+                    const int64_t e = C.s_base + S.ca;
+                    A.sc[0][e] = xi0; A.sc[1][e] = xi1; A.sc[2][e] = xi2;
+                    A.sc[3][e] = ui0; A.sc[4][e] = ui1; A.sc[5][e] = ui2; A.sc[6][e] = dw;
+                    A.sc[0][e + 1] = xk0; A.sc[1][e + 1] = xk1; A.sc[2][e + 1] = xk2;
+                    A.sc[3][e + 1] = uk0; A.sc[4][e + 1] = uk1; A.sc[5][e + 1] = uk2; A.sc[6][e + 1] = dw;
+                }
+                S.ca += 2;
+                S.na += 2;
+            } else {
+                const bool eq = (eqm & bit) != 0, heavy_i = (heavym & bit) != 0;
+                const bool split = CREATES && !eq;
+                const bool on_a = heavy_i || single;
+                const int32_t q = on_a ? (single ? S.ca + S.cb : S.ca) : S.cb;
+                ++S.performed;
+                if (split && q >= C.n_coll) {   // no room for the split: ends before its scattering draws
+                    if (lane == 0) atomicOr(&(on_a ? A.a : A.b).ctr->err, MZ_ERR_SCRATCH);
+                    ++j;
+                    continue;
+                }
+                if (eq) {
+                    ++S.eqw;
+                } else if (!CREATES) {
+                    if (lane == 0) atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
+                }
+                if (lane == L) {
+                    if (split) {
+                        const int64_t e = (on_a ? 0 : sc_b) + C.s_base + q;
+                        A.sc[0][e] = heavy_i ? xi0 : xk0; A.sc[1][e] = heavy_i ? xi1 : xk1;
+                        A.sc[2][e] = heavy_i ? xi2 : xk2;
+                        A.sc[3][e] = heavy_i ? vi0 : vk0; A.sc[4][e] = heavy_i ? vi1 : vk1;
+                        A.sc[5][e] = heavy_i ? vi2 : vk2;
+                        A.sc[6][e] = heavy_i ? wi - wk : wk - wi;
+                        if (heavy_i) (in_i ? A.a.w : A.sc[6])[pi] = wk;
+                        else (in_k ? A.b.w : A.sc[6])[pk] = wi;
+                    }
+                    (in_i ? A.a.v0 : A.sc[3])[pi] = ui0; (in_i ? A.a.v1 : A.sc[4])[pi] = ui1;
+                    (in_i ? A.a.v2 : A.sc[5])[pi] = ui2;
+                    (in_k ? A.b.v0 : A.sc[3])[pk] = uk0; (in_k ? A.b.v1 : A.sc[4])[pk] = uk1;
+                    (in_k ? A.b.v2 : A.sc[5])[pk] = uk2;
+                }
+                if (split) {
+                    if (on_a) {
+                        ++S.ca;
+                        ++S.na;
+                    } else {
+                        ++S.cb;
+                        ++S.nb;
+                    }
+                }
+            }
+            const int32_t i = __builtin_amdgcn_readlane(si, L), k = __builtin_amdgcn_readlane(sk, L);
+            stop |= single ? __ballot(si == i || sk == i || si == k || sk == k) : __ballot(si == i || sk == k);
+            ++a;
+            if (single ? S.na != na0 + inc * a : (S.na != na0 || S.nb != nb0)) {
+                if (single && KIND == NTC_SPLIT) inc = S.na - na0 == inc * (a - 1) ? 0 : 1;
+                break;
+            }
+            if (a == T) {
+                T = min(8, 2 * T);
+                break;
+            }
         }
-        // the stores of the window before the loads that follow
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        if (!at_o) o = D + (uint64_t)(5 * a + 3 * j);
+        if (ran_out && 2 * a < T) T = max(1, T / 2);
+        if (a + j == 0 && !at_o) direct = true;   // a first pick out of range by rounding: taken as the loop takes it
+        S.sgwm = sgwm;
+        // the window's stores before the loads that follow: one wave's vector
+        // memory operations stay in order, so this only holds the compiler
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         if (direct) {
             dr.seek(o);
-            ntc_candidate(A, c, C, S, dr);   // Philox draws: never exhausted
+            if (SWPM) swpm_candidate(A, c, C, S, dr, wtf, inv_w_max);
+            else ntc_candidate(A, c, C, S, dr);   // Philox draws: never exhausted
             o = dr.k;
             ++cc;
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
     }
-    ntc_finish_cell(A, c, C, S);
 }
 
-// One lane per cell; cells run in parallel (64-lane workgroups, so the
-// loop keeps its state in registers).
-__global__ void __launch_bounds__(64) k_ntc(NtcArgs A) {
+// Calls over more cells than this first run the cells of at most
+// NTC_LANE_MAX candidates one lane each (k_ntc), then the others one wavefront
+// each; calls over fewer run every cell on a wavefront.  A window costs about
+// 4 us however few of its lanes hold a candidate, and some 3,000 wavefronts
+// run at once: 16,000 cells of one candidate take 45 us on wavefronts and
+// 16 us on lanes, 2,000 cells of seven 21 us on wavefronts against 4 us per
+// candidate on lanes; 65,536 cells of 20 to 20,000 particles 14.0 ms on lanes
+// and 9.4 ms on wavefronts.
+#define NTC_WAVE_MAX_CELLS 4096
+#define NTC_LANE_MAX 4
+
+// One lane per cell; cells run in parallel (64-lane workgroups, so the loop
+// keeps its state in registers).  Cells of more than max_coll candidates are
+// left, their count noted, for k_ntc_wave.
+__global__ void __launch_bounds__(64) k_ntc(NtcArgs A, int64_t max_coll) {
     const int c = A.cell_lo + blockIdx.x * blockDim.x + threadIdx.x;
     if (c > A.cell_hi) return;
     A.rp = mz_rng_resolve(A.rp);
     NtcLaneDraw dr{A.rp, mz_stream((uint64_t)c)};
-    ntc_cell(A, c, dr);
+    NtcCell C;
+    NtcState S;
+    ntc_setup(A, c, dr, C, S);
+    if (C.n_coll > max_coll) {
+        A.cnt[(int64_t)c * 5 + 2] = (int32_t)C.n_coll;
+        return;
+    }
+    for (int64_t cc = 0; cc < C.n_coll; ++cc)
+        if (!ntc_candidate(A, c, C, S, dr)) return;
+    ntc_finish_cell(A, c, C, S);
 }
 
-// One wavefront per cell (Philox draws): single-species cells take their
-// candidates a window at a time (ntc_cell_spec), two-species cells run the
-// loop on every lane on the same values; the draws come from registers.  For
-// calls over few cells, which one lane per cell would spread over a handful
-// of wavefronts.
-__global__ void __launch_bounds__(64) k_ntc_wave(NtcArgs A) {
+// One wavefront per cell (Philox draws), candidates a window at a time; cells
+// of at most min_coll candidates (after k_ntc) are done already.
+template <int KIND>
+__global__ void __launch_bounds__(64) k_ntc_wave(NtcArgs A, int32_t min_coll) {
     const int c = A.cell_lo + blockIdx.x;
-    if (c > A.cell_hi) return;
+    if (c > A.cell_hi || (min_coll > 0 && A.cnt[(int64_t)c * 5 + 2] <= min_coll)) return;
     A.rp = mz_rng_resolve(A.rp);
     NtcWaveDraw dr{A.rp, (uint64_t)c, 0, ~(uint64_t)0, 0.0, 0.0};
-    if (A.single) ntc_cell_spec(A, c, dr);
-    else ntc_cell(A, c, dr);
+    NtcCell C;
+    NtcState S;
+    ntc_setup(A, c, dr, C, S);
+    ntc_windows<KIND>(A, c, C, S, dr, 0.0, 0.0);
+    if ((threadIdx.x & 63) == 0) ntc_finish_cell(A, c, C, S);
 }
 
 // Count pass of the split path: n_coll of every cell (draw 0 of its stream).
@@ -562,14 +765,16 @@ static NtcArgs base_args(mz_store *h, int s1, int s2, double dt, const double *d
     return A;
 }
 
-// The candidate loops over ncells cells: a wavefront per cell for calls over
-// few cells (Philox draws), one lane per cell otherwise.
-#define NTC_WAVE_MAX_CELLS 4096
+// The candidate loops over ncells cells; replayed draws run one lane per cell.
 static void launch_k_ntc(mz_store *h, const NtcArgs &A, int ncells) {
-    if (ncells <= NTC_WAVE_MAX_CELLS && A.rp.mode == 0)
-        hipLaunchKernelGGL(k_ntc_wave, dim3(ncells), dim3(64), 0, h->stream, A);
-    else
-        hipLaunchKernelGGL(k_ntc, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A);
+    const bool wave = A.rp.mode == 0, few = ncells <= NTC_WAVE_MAX_CELLS;
+    if (!wave || !few)
+        hipLaunchKernelGGL(k_ntc, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A,
+                           wave ? (int64_t)NTC_LANE_MAX : INT64_MAX);
+    if (wave && A.may_split)
+        hipLaunchKernelGGL(k_ntc_wave<NTC_SPLIT>, dim3(ncells), dim3(64), 0, h->stream, A, few ? 0 : NTC_LANE_MAX);
+    else if (wave)
+        hipLaunchKernelGGL(k_ntc_wave<NTC_PLAIN>, dim3(ncells), dim3(64), 0, h->stream, A, few ? 0 : NTC_LANE_MAX);
 }
 
 int mz_launch_ntc_equal(mz_store *h, int s1, int s2, double dt, const double *dV, double dw_tol, int equal_weight,
@@ -743,69 +948,56 @@ __global__ void __launch_bounds__(256) k_swpm_count(NtcArgs A, double G, int32_t
     wmax[c] = w_max;
 }
 
+__device__ __forceinline__ void swpm_setup(const NtcArgs &A, const int c, NtcCell &C, NtcState &S) {
+    C.n1a = C.n1b = A.a.pia.n1[c];
+    C.n2a = C.n2b = A.a.pia.n2[c] > 0 ? A.a.pia.n2[c] : 0;
+    C.nla = C.nlb = A.a.pia.nloc[c];
+    C.n_coll = A.ncoll_in[c];
+    C.s_base = A.soff[c];
+    S.na = S.nb = C.nla;
+    S.ca = S.cb = 0;
+    S.performed = S.eqw = 0;
+    S.sgwm = A.sgwm[c];
+}
+
+__device__ __forceinline__ void swpm_finish(const NtcArgs &A, const int c, const NtcCell &C, const NtcState &S) {
+    A.sgwm[c] = S.sgwm;
+    int32_t *cn = A.cnt + (int64_t)c * 5;
+    cn[0] = C.nla;
+    cn[1] = C.nla;
+    cn[2] = (int32_t)C.n_coll;
+    cn[3] = S.performed;
+    cn[4] = 0;
+    A.created[c] = S.ca;
+}
+
+// One lane per cell, for replayed draws.
 __global__ void __launch_bounds__(64) k_swpm(NtcArgs A, double G, const double *__restrict__ wmax) {
     const int c = A.cell_lo + blockIdx.x * blockDim.x + threadIdx.x;
     if (c > A.cell_hi) return;
     A.rp = mz_rng_resolve(A.rp);
-    const int32_t n1 = A.a.pia.n1[c], n2 = A.a.pia.n2[c] > 0 ? A.a.pia.n2[c] : 0;
-    const int32_t nl = A.a.pia.nloc[c];
-    const double wtf = 1.0 / (1.0 + G);
-    const double inv_w_max = 1.0 / wmax[c];
-    double sgmax = A.sgwm[c];
-    MzStream st = mz_stream((uint64_t)c);
-    st.k = 1;
-    const int64_t n_coll = A.ncoll_in[c];
-    const int64_t s_base = A.soff[c];
-    int32_t na = nl, created = 0, performed = 0;
-    for (int64_t cc = 0; cc < n_coll; ++cc) {
-        const int32_t i = (int32_t)floor(mz_rand(A.rp, st) * (double)na);
-        int32_t k = (int32_t)floor(mz_rand(A.rp, st) * (double)na);
-        while (i == k) {
-            k = (int32_t)floor(mz_rand(A.rp, st) * (double)na);
-            if (A.rp.mode == 1 && (int64_t)st.k > A.rp.cols) return;   // replay row exhausted
-        }
-        PRef pi = i < nl ? pref_slot(A.a, slot_of(A.a, c, i, n1, n2)) : pref_scratch(A, 0, s_base + (i - nl));
-        PRef pk = k < nl ? pref_slot(A.a, slot_of(A.a, c, k, n1, n2)) : pref_scratch(A, 0, s_base + (k - nl));
-        const double vi0 = pi.v0[pi.i], vi1 = pi.v1[pi.i], vi2 = pi.v2[pi.i];
-        const double vk0 = pk.v0[pk.i], vk1 = pk.v1[pk.i], vk2 = pk.v2[pk.i];
-        double g0, g1, g2;
-        const double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
-        if (!(g > MZ_G_EPS)) continue;
-        const double sgm = mz_vhs_sgw(A.factor, A.expo, g, 1.0, 1.0);   // sigma g
-        sgmax = sgm > sgmax ? sgm : sgmax;
-        const double wi = pi.w[pi.i], wk = pk.w[pk.i];
-        if (!(mz_rand(A.rp, st) < sgm * (wi > wk ? wi : wk) * inv_w_max / sgmax)) continue;
-        ++performed;
-        double vc0, vc1, vc2;
-        mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
-        const double dw = (wi < wk ? wi : wk) * wtf;
-        pi.w[pi.i] = wi - dw;
-        pk.w[pk.i] = wk - dw;
-        if (created + 1 >= 2 * n_coll) {
-            atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
-            continue;
-        }
-        PRef n_i = pref_scratch(A, 0, s_base + created), n_k = pref_scratch(A, 0, s_base + created + 1);
-        n_i.x0[n_i.i] = pi.x0[pi.i]; n_i.x1[n_i.i] = pi.x1[pi.i]; n_i.x2[n_i.i] = pi.x2[pi.i];
-        n_k.x0[n_k.i] = pk.x0[pk.i]; n_k.x1[n_k.i] = pk.x1[pk.i]; n_k.x2[n_k.i] = pk.x2[pk.i];
-        n_i.w[n_i.i] = dw;
-        n_k.w[n_k.i] = dw;
-        created += 2;
-        na += 2;
-        // scatter_vhs! on the two new particles: phi first, then cos(theta)
-        double ui0, ui1, ui2, uk0, uk1, uk2;
-        mz_vhs_scatter(A.rp, st, A.mu1, A.mu2, g, vc0, vc1, vc2, ui0, ui1, ui2, uk0, uk1, uk2);
-        n_i.v0[n_i.i] = ui0; n_i.v1[n_i.i] = ui1; n_i.v2[n_i.i] = ui2;
-        n_k.v0[n_k.i] = uk0; n_k.v1[n_k.i] = uk1; n_k.v2[n_k.i] = uk2;
-    }
-    A.sgwm[c] = sgmax;
-    int32_t *cn = A.cnt + (int64_t)c * 5;
-    cn[0] = nl;
-    cn[1] = nl;
-    cn[2] = (int32_t)n_coll;
-    cn[3] = performed;
-    cn[4] = 0;
-    A.created[c] = created;
+    NtcLaneDraw dr{A.rp, mz_stream((uint64_t)c)};
+    dr.seek(1);
+    NtcCell C;
+    NtcState S;
+    swpm_setup(A, c, C, S);
+    const double wtf = 1.0 / (1.0 + G), inv_w_max = 1.0 / wmax[c];
+    for (int64_t cc = 0; cc < C.n_coll; ++cc)
+        if (!swpm_candidate(A, c, C, S, dr, wtf, inv_w_max)) return;
+    swpm_finish(A, c, C, S);
+}
+
+// One wavefront per cell (Philox draws), candidates a window at a time.
+__global__ void __launch_bounds__(64) k_swpm_wave(NtcArgs A, double G, const double *__restrict__ wmax) {
+    const int c = A.cell_lo + blockIdx.x;
+    if (c > A.cell_hi) return;
+    A.rp = mz_rng_resolve(A.rp);
+    NtcWaveDraw dr{A.rp, (uint64_t)c, 1, ~(uint64_t)0, 0.0, 0.0};
+    NtcCell C;
+    NtcState S;
+    swpm_setup(A, c, C, S);
+    ntc_windows<NTC_SWPM>(A, c, C, S, dr, 1.0 / (1.0 + G), 1.0 / wmax[c]);
+    if ((threadIdx.x & 63) == 0) swpm_finish(A, c, C, S);
 }
 
 extern "C" int mz_swpm(mz_store *h, int32_t species, double G, double dt, const double *V, uint64_t tag,
@@ -853,7 +1045,10 @@ extern "C" int mz_swpm(mz_store *h, int32_t species, double G, double dt, const 
         A.ncoll_in = ncoll;
         A.soff = soff;
         A.created = created;
-        hipLaunchKernelGGL(k_swpm, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A, G, (const double *)wmax);
+        if (rng_mode == 0)
+            hipLaunchKernelGGL(k_swpm_wave, dim3(ncells), dim3(64), 0, h->stream, A, G, (const double *)wmax);
+        else
+            hipLaunchKernelGGL(k_swpm, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A, G, (const double *)wmax);
         MZ_HIP(hipGetLastError());
         double **scp = (double **)mz_scratch(h, "ntc_scp", 7 * sizeof(double *));
         MZ_CHECK(scp != nullptr, "swpm: scratch allocation failed");

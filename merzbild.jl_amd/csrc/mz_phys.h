@@ -53,23 +53,41 @@ __device__ inline void mz_com(double mu1, double mu2, double vi0, double vi1, do
     vc2 = fma(mu1, vi2, mu2 * vk2);
 }
 
-// scatter_vhs! from its two draws (R_phi drawn first, then R_ct): isotropic
-// post-collision relative velocity of magnitude g about the centre of mass.
-__device__ inline void mz_vhs_post(double mu1, double mu2, double g, double vc0, double vc1, double vc2,
-                                   double R_phi, double R_ct, double &vi0, double &vi1, double &vi2, double &vk0,
-                                   double &vk1, double &vk2) {
+// The isotropic direction of scatter_vhs! from its two draws (R_phi drawn
+// first, then R_ct).
+__device__ inline void mz_vhs_dir(double R_phi, double R_ct, double &e0, double &e1, double &e2) {
     double phi = 6.283185307179586 * R_phi;
     double sphi, cphi;
     mz_sincos(phi, &sphi, &cphi);
     double ct = 2.0 * R_ct - 1.0;
     double stt = sqrt(1.0 - ct * ct);
-    double gn0 = g * (stt * cphi), gn1 = g * (stt * sphi), gn2 = g * ct;
+    e0 = stt * cphi;
+    e1 = stt * sphi;
+    e2 = ct;
+}
+
+// The post-collision velocities: the relative velocity of magnitude g along
+// (e0, e1, e2) about the centre of mass.
+__device__ inline void mz_vhs_along(double mu1, double mu2, double g, double vc0, double vc1, double vc2, double e0,
+                                    double e1, double e2, double &vi0, double &vi1, double &vi2, double &vk0,
+                                    double &vk1, double &vk2) {
+    double gn0 = g * e0, gn1 = g * e1, gn2 = g * e2;
     vi0 = fma(mu2, gn0, vc0);
     vi1 = fma(mu2, gn1, vc1);
     vi2 = fma(mu2, gn2, vc2);
     vk0 = fma(-mu1, gn0, vc0);
     vk1 = fma(-mu1, gn1, vc1);
     vk2 = fma(-mu1, gn2, vc2);
+}
+
+// scatter_vhs! from its two draws (R_phi drawn first, then R_ct): isotropic
+// post-collision relative velocity of magnitude g about the centre of mass.
+__device__ inline void mz_vhs_post(double mu1, double mu2, double g, double vc0, double vc1, double vc2,
+                                   double R_phi, double R_ct, double &vi0, double &vi1, double &vi2, double &vk0,
+                                   double &vk1, double &vk2) {
+    double e0, e1, e2;
+    mz_vhs_dir(R_phi, R_ct, e0, e1, e2);
+    mz_vhs_along(mu1, mu2, g, vc0, vc1, vc2, e0, e1, e2, vi0, vi1, vi2, vk0, vk1, vk2);
 }
 
 // scatter_vhs!: two draws, phi first, then cos(theta)
