@@ -167,6 +167,7 @@ struct MzSpecies {
     int32_t *idb;
     int32_t *key;       // cell key per slot before the last sort (reference pv.cell)
     int32_t *keyb;      // second key buffer (squash moves keys with the data)
+    int2 *krange;       // smallest and largest cell key of each chunk of slots (during a sort)
     int32_t *buffer;    // free-id LIFO (reference pv.buffer), capacity bufcap
     int64_t bufcap;
     MzPia pia;

@@ -11,7 +11,7 @@
 
 #define MZ_MAX_SPECIES 4
 #define MZ_SORT_CHUNK 1024
-#define MZ_SORT_MAX_CELLS 14336   // LDS: 8 KB per chunk + 4 B per cell within 64 KB
+#define MZ_SORT_MAX_CELLS 14336   // of the count-matrix sort where a caller asks for it
 #define MZ_MAX_BOUNCES 64
 #define MZ_MAX_MOMENTS 8   // total-moment powers per compute_props_with_total_moments! call
 #define MZ_NTC_MAX_CANDIDATES 100000000  // per cell and call; larger counts flag an error
@@ -73,7 +73,8 @@ struct mz_store {
     double *d_replay[3] = {nullptr, nullptr, nullptr};
     int64_t replay_rows[3] = {0, 0, 0}, replay_cols[3] = {0, 0, 0};
     int32_t *d_err = nullptr;
-    uint32_t *d_ticket = nullptr;  // last-block counter of k_sort_rows (left at 0 by every launch)
+    // of the count-matrix sort: the cells' totals (left at 0 by every sort) and starts
+    int32_t *d_ccount = nullptr, *d_cstart = nullptr;
     double *d_np = nullptr, *d_n = nullptr, *d_v = nullptr, *d_T = nullptr;
     double *d_V = nullptr, *d_invV = nullptr;
     double *d_masses = nullptr;

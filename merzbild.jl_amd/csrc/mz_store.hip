@@ -153,7 +153,9 @@ static int alloc_species(MzSpecies &s, int64_t cap, int n_cells) {
     MZ_HIP(hipMalloc(&s.id, cap * sizeof(int32_t)));
     MZ_HIP(hipMalloc(&s.idb, cap * sizeof(int32_t)));
     MZ_HIP(hipMalloc(&s.key, cap * sizeof(int32_t)));
-    MZ_HIP(hipMalloc(&s.keyb, cap * sizeof(int32_t)));
+    const int64_t cap2 = (cap + 1) & ~(int64_t)1;   // int2 alignment of what follows
+    MZ_HIP(hipMalloc(&s.keyb, cap2 * sizeof(int32_t) + (cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK * sizeof(int2)));
+    s.krange = (int2 *)(s.keyb + cap2);
     MZ_HIP(hipMalloc(&s.buffer, s.bufcap * sizeof(int32_t)));
     int32_t **f[7] = {&s.pia.start1, &s.pia.end1, &s.pia.n1, &s.pia.start2, &s.pia.end2, &s.pia.n2, &s.pia.nloc};
     for (auto p : f) MZ_HIP(hipMalloc(p, n_cells * sizeof(int32_t)));
@@ -187,8 +189,10 @@ extern "C" int mz_create(int32_t n_cells, int32_t n_species, const int64_t *capa
     MZ_HIP(hipMemset(h->d_cfcnt, 0, (size_t)nss * n_cells * 5 * sizeof(int32_t)));
     MZ_HIP(hipMalloc(&h->d_err, sizeof(int32_t)));
     MZ_HIP(hipMemset(h->d_err, 0, sizeof(int32_t)));
-    MZ_HIP(hipMalloc(&h->d_ticket, sizeof(uint32_t)));
-    MZ_HIP(hipMemset(h->d_ticket, 0, sizeof(uint32_t)));
+    const size_t ncp = ((size_t)n_cells + 15) & ~(size_t)15;
+    MZ_HIP(hipMalloc(&h->d_ccount, (2 * ncp + 16) * sizeof(int32_t)));
+    MZ_HIP(hipMemset(h->d_ccount, 0, ncp * sizeof(int32_t)));
+    h->d_cstart = h->d_ccount + ncp;
     size_t pn = (size_t)n_species * n_cells;
     MZ_HIP(hipMalloc(&h->d_np, pn * sizeof(double)));
     MZ_HIP(hipMalloc(&h->d_n, pn * sizeof(double)));
@@ -260,7 +264,7 @@ extern "C" int mz_destroy(mz_store *h) {
     if (h->h_report) hipHostFree(h->h_report);
     mz_graph_release(h);
     for (auto &s : h->sp) free_species(s);
-    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ticket);
+    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ccount);
     hipFree(h->d_np); hipFree(h->d_n); hipFree(h->d_T); hipFree(h->d_v); hipFree(h->d_V);
     hipFree(h->d_invV);
     hipFree(h->d_masses);
@@ -572,29 +576,47 @@ MzRngParams mz_rng_params(mz_store *h, int kind, uint64_t tag, int mode) {
 
 // ===========================================================================
 // Sorting: stable counting sort by cell (grid_sorting.jl:58-182).
-//   1. k_sort_hist: per chunk of MZ_SORT_CHUNK positions, cell keys (from x,
-//      or the stored keys) and a per-chunk histogram in LDS; the histogram is
-//      written cell-major [cell][chunk].
-//   2. k_sort_rows: per cell, an exclusive scan over chunks gives each
-//      chunk's offset inside the cell; the cell totals, scanned by the block
-//      that finishes last, give the cell starts and the new PIA.
-//   3. k_sort_scatter: per chunk, its slot of particle i is cell start +
+//   1. k_sort_hist: per chunk of positions, cell keys (from x, or the stored
+//      keys), their range [kmin, kmax] and the counts of the keys in it,
+//      written [chunk][cell]; the cells' totals.
+//   2. k_sort_rows: per cell, an exclusive scan over the chunks whose range
+//      holds it gives each chunk's offset inside the cell; one more block
+//      scans the totals into the cell starts.
+//   3. k_sort_scatter: per chunk, the slot of particle i is cell start +
 //      chunk offset + rank of i among the chunk's equal keys in position
-//      order, so the sort is stable like the reference's reverse scatter.
+//      order, so the sort is stable like the reference's reverse scatter; it
+//      also writes the PIA (group 1 only, group 2 cleared, as
+//      grid_sorting.jl:76-98 writes it).
 // The data moves with the sort (x, v, w, id); the key array stays in the
 // pre-sort order, like the reference's pv.cell.
+//
+// What bounds it: the moved data (112 B + 8 B of ids and 12 B of keys and
+// positions a particle) for large stores, three launches' latency for small
+// ones.  After a step a chunk's particles lie in a few neighbouring cells, so
+// only the counts inside its range are written and read (any order of the
+// particles is sorted; a chunk that spans all cells writes a count for each).
+// Chunks of 1,024 keep the chip busy on small stores, chunks of 4,096 keep the
+// count matrix small on large ones.  Measured against whole-matrix counts and
+// ranks formed by one wavefront a chunk: see the table at SORT_SMALL_SLOTS.
 
-__global__ void k_sort_hist(MzSpView sp, MzGrid g, int32_t compute_cells, int32_t n_cells, int32_t nchunks,
-                            int32_t *__restrict__ hist) {
-    extern __shared__ int32_t sh[];
+#define SORT_KEYS 4096   // keys counted or ranked in LDS at once; a wider range takes several sweeps
+
+template <int IPT>
+__global__ void __launch_bounds__(256) k_sort_hist(MzSpView sp, MzGrid g, int32_t compute_cells, int32_t n_cells,
+                                                   int32_t *__restrict__ hist, int2 *__restrict__ range,
+                                                   int32_t *__restrict__ counts) {
+    __shared__ int32_t sh[SORT_KEYS];
+    __shared__ int32_t wlo[4], whi[4];
     const int32_t n = mz_ntotal(sp);
-    for (int c = threadIdx.x; c < n_cells; c += blockDim.x) sh[c] = 0;
-    __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * MZ_SORT_CHUNK;
-    for (int i = threadIdx.x; i < MZ_SORT_CHUNK; i += blockDim.x) {
-        int64_t p = base + i;
+    const int64_t base = (int64_t)blockIdx.x * (256 * IPT);
+    if (base >= n) return;
+    const int tid = threadIdx.x;
+    int32_t key[IPT], lo = INT32_MAX, hi = 0;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const int64_t p = base + r * 256 + tid;
+        int32_t c = 0;
         if (p < n) {
-            int32_t c;
             if (compute_cells) {
                 c = mz_cell_of(sp.x0[p], g, n_cells, &sp.ctr->err);
                 sp.key[p] = c;
@@ -605,143 +627,241 @@ __global__ void k_sort_hist(MzSpView sp, MzGrid g, int32_t compute_cells, int32_
                     c = c < 1 ? 1 : n_cells;
                 }
             }
-            atomicAdd(&sh[c - 1], 1);
+            lo = min(lo, c);
+            hi = max(hi, c);
         }
+        key[r] = c;   // 0 past the end
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((tid & 63) == 0) {
+        wlo[tid >> 6] = lo;
+        whi[tid >> 6] = hi;
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < n_cells; c += blockDim.x) hist[(int64_t)c * nchunks + blockIdx.x] = sh[c];
+    lo = min(min(wlo[0], wlo[1]), min(wlo[2], wlo[3]));
+    hi = max(max(whi[0], whi[1]), max(whi[2], whi[3]));
+    if (tid == 0) range[blockIdx.x] = make_int2(lo, hi);
+    for (int32_t w0 = lo; w0 <= hi; w0 += SORT_KEYS) {
+        const int32_t width = min(SORT_KEYS, hi - w0 + 1);
+        for (int d = tid; d < width; d += 256) sh[d] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPT; ++r)
+            if (key[r] >= w0 && key[r] - w0 < width) atomicAdd(&sh[key[r] - w0], 1);
+        __syncthreads();
+        for (int d = tid; d < width; d += 256) {
+            const int32_t v = sh[d], c = w0 - 1 + d;
+            hist[(int64_t)blockIdx.x * n_cells + c] = v;
+            if (v > 0) atomicAdd(&counts[c], v);
+        }
+        __syncthreads();
+    }
 }
 
-// One wave per cell scans that cell's row of the count matrix over chunks
-// (exclusive, in place) and leaves the cell total; the block that finishes
-// last turns the totals into cell starts and writes the PIA (group 1 only,
-// group 2 cleared, as grid_sorting.jl:76-98 writes it).
-__global__ void __launch_bounds__(256) k_sort_rows(MzSpView sp, int32_t n_cells, int32_t nchunks,
-                                                   int32_t *__restrict__ hist, int32_t *__restrict__ cstart,
-                                                   uint32_t *__restrict__ ticket) {
-    __shared__ int32_t is_last;
+#define SORT_SCAN 4096   // cell totals scanned at once
+
+// Block 0: exclusive scan of the cell totals into cstart[0 .. n_cells], the
+// totals cleared for the next sort (both arrays are padded to 16 entries).
+// Blocks 1 ..: eight cells per wave; the wave finds the chunks whose ranges
+// hold any of them, and lane s 8 + k scans cell k's counts over them eight at
+// a time (exclusive, in place), chunk s of the eight.
+__global__ void __launch_bounds__(256) k_sort_rows(MzSpView sp, int32_t n_cells, int32_t chunk,
+                                                   int32_t *__restrict__ hist, const int2 *__restrict__ range,
+                                                   int32_t *__restrict__ counts, int32_t *__restrict__ cstart) {
     __shared__ int32_t wsum[4];
-    __shared__ int32_t carry_s;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int c = blockIdx.x * 4 + wv;
-    if (c < n_cells) {
-        int32_t *row = hist + (int64_t)c * nchunks;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    if (blockIdx.x > 0) {
+        const int c0 = ((blockIdx.x - 1) * 4 + wv) * 8;
+        if (c0 >= n_cells) return;
+        const int c = c0 + (lane & 7), sub = lane >> 3;
+        const int c_last = min(n_cells, c0 + 8) - 1;
+        const int32_t used = (int32_t)(((int64_t)mz_ntotal(sp) + chunk - 1) / chunk);
         int32_t carry = 0;
-        for (int b0 = 0; b0 < nchunks; b0 += 64) {
-            int b = b0 + lane;
-            int32_t v = b < nchunks ? row[b] : 0;
-            int32_t x = v;
+        for (int b0 = 0; b0 < used; b0 += 256) {
+            int2 rg[4];   // the ranges of 256 chunks in one round trip
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                int32_t y = __shfl_up(x, o, 64);
-                if (lane >= o) x += y;
+            for (int q = 0; q < 4; ++q) {
+                const int b = b0 + q * 64 + lane;
+                rg[q] = b < used ? range[b] : make_int2(INT32_MAX, 0);
             }
-            if (b < nchunks) row[b] = carry + x - v;
-            carry += __shfl(x, 63, 64);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint64_t m = __ballot(rg[q].x <= c_last + 1 && c0 + 1 <= rg[q].y);
+                while (m) {
+                    uint64_t mm = m;
+                    for (int t = 0; t < sub; ++t) mm &= mm - 1;   // drop the chunks of the lower subs
+                    const int bl = mm ? __ffsll((unsigned long long)mm) - 1 : 0;
+                    const int32_t lo = __shfl(rg[q].x, bl, 64), hi = __shfl(rg[q].y, bl, 64);
+                    const bool in = mm != 0 && c < n_cells && lo <= c + 1 && c + 1 <= hi;
+                    int32_t *e = hist + (int64_t)(b0 + q * 64 + bl) * n_cells + c;
+                    const int32_t v = in ? *e : 0;
+                    int32_t x = v;
+#pragma unroll
+                    for (int o = 8; o < 64; o <<= 1) {
+                        const int32_t y = __shfl_up(x, o, 64);
+                        if (lane >= o) x += y;
+                    }
+                    if (in) *e = carry + x - v;
+                    carry += __shfl(x, 56 + (lane & 7), 64);
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) m &= m - 1;
+                }
+            }
         }
-        if (lane == 0) __hip_atomic_store(&cstart[c], carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
     }
-    mz_wait_stores();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t = atomicAdd(ticket, 1u);
-        is_last = (t == gridDim.x - 1);
-        carry_s = 0;
-    }
-    __syncthreads();
-    if (!is_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    const int32_t total = mz_ntotal(sp);
-    for (int c0 = 0; c0 < n_cells; c0 += 256) {
-        const int cc = c0 + threadIdx.x;
-        int32_t v = cc < n_cells ? __hip_atomic_load(&cstart[cc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-        int32_t x = v;
+    int32_t carry = 0;
+    for (int c0 = 0; c0 < n_cells; c0 += SORT_SCAN) {
+        const int i0 = c0 + tid * 16;   // sixteen consecutive totals per thread
+        int4 v[4] = {};
+        if (i0 < n_cells) {
+            int4 *src = reinterpret_cast<int4 *>(counts + i0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = src[q];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) src[q] = make_int4(0, 0, 0, 0);
+        }
+        int32_t s = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += v[q].x + v[q].y + v[q].z + v[q].w;
+        int32_t x = s;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            int32_t y = __shfl_up(x, o, 64);
+            const int32_t y = __shfl_up(x, o, 64);
             if (lane >= o) x += y;
         }
         if (lane == 63) wsum[wv] = x;
         __syncthreads();
-        int32_t pre = carry_s;
-        for (int k = 0; k < wv; ++k) pre += wsum[k];
-        int32_t excl = pre + x - v;
-        if (cc < n_cells) {
-            cstart[cc] = excl;
-            sp.pia.start2[cc] = 0;
-            sp.pia.end2[cc] = -1;
-            sp.pia.n2[cc] = 0;
-            sp.pia.start1[cc] = v > 0 ? excl + 1 : 0;
-            sp.pia.end1[cc] = v > 0 ? excl + v : -1;
-            sp.pia.n1[cc] = v;
-            sp.pia.nloc[cc] = v;
+        int32_t run = carry + x - s;
+        for (int k = 0; k < wv; ++k) run += wsum[k];
+        if (i0 < n_cells) {
+            int4 *dst = reinterpret_cast<int4 *>(cstart + i0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                int4 o;
+                o.x = run; run += v[q].x;
+                o.y = run; run += v[q].y;
+                o.z = run; run += v[q].z;
+                o.w = run; run += v[q].w;
+                dst[q] = o;
+            }
         }
-        __syncthreads();
-        if (threadIdx.x == 255) carry_s = excl + v;
+        carry += wsum[0] + wsum[1] + wsum[2] + wsum[3];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        *ticket = 0;
-        sp.ctr->contiguous = 1;
-        sp.ctr->n_pos = total;
-    }
+    if (tid == 0) cstart[n_cells] = carry;
 }
 
-// One block per chunk: the chunk's keys go to LDS, wave 0 ranks them in
-// position order (64 at a time; lanes with equal keys are ranked with a
-// ballot, so equal keys keep their order: stable, as the reference's reverse
-// scatter), then all threads move the particles to their slots.
-__global__ void __launch_bounds__(256) k_sort_scatter(MzSpView a, MzSpView b, int32_t n_cells, int32_t nchunks,
-                                                     const int32_t *__restrict__ rows,
-                                                     const int32_t *__restrict__ cstart) {
-    extern __shared__ int32_t run[];   // [n_cells]: next slot of each cell for this chunk
-    __shared__ int32_t keys[MZ_SORT_CHUNK];
-    __shared__ int32_t dst[MZ_SORT_CHUNK];
+// One block per chunk, a quarter of it to each wave, 64 positions at a time:
+// lanes of equal keys find each other with one ballot per bit of the key's
+// place in the chunk's range; their first lane adds their number to the
+// wave's 16-bit field of the key's LDS word, whose former value is the rank
+// of the first.  The earlier waves' fields, the chunk's offset in the cell
+// and the cell start complete the slot.
+template <int IPT>
+__global__ void __launch_bounds__(256) k_sort_scatter(MzSpView a, MzSpView b, int32_t n_cells,
+                                                      const int32_t *__restrict__ rows,
+                                                      const int2 *__restrict__ range,
+                                                      const int32_t *__restrict__ cstart) {
+    __shared__ unsigned long long tab[SORT_KEYS];
     const int32_t n = mz_ntotal(a);
-    const int64_t p0 = (int64_t)blockIdx.x * MZ_SORT_CHUNK;
-    if (p0 >= n) return;
-    const int cnt = (int)min((int64_t)MZ_SORT_CHUNK, (int64_t)n - p0);
-    for (int k = threadIdx.x; k < n_cells; k += 256) run[k] = cstart[k] + rows[(int64_t)k * nchunks + blockIdx.x];
-    for (int i = threadIdx.x; i < cnt; i += 256) {
-        int32_t k = a.key[p0 + i];
-        keys[i] = k < 1 ? 1 : (k > n_cells ? n_cells : k);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    for (int c = blockIdx.x * 256 + tid; c < n_cells; c += gridDim.x * 256) {
+        const int32_t s = cstart[c], v = cstart[c + 1] - s;
+        a.pia.start2[c] = 0;
+        a.pia.end2[c] = -1;
+        a.pia.n2[c] = 0;
+        a.pia.start1[c] = v > 0 ? s + 1 : 0;
+        a.pia.end1[c] = v > 0 ? s + v : -1;
+        a.pia.n1[c] = v;
+        a.pia.nloc[c] = v;
     }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        volatile int32_t *vrun = run;
-        const int lane = threadIdx.x;
-        const uint64_t lt = mz_lanemask_lt();
-        for (int bt = 0; bt < cnt; bt += 64) {
-            const int i = bt + lane;
-            const bool valid = i < cnt;
-            const int32_t key = valid ? keys[i] : 0;
-            uint64_t active = __ballot(valid);
-            while (active) {
-                const int leader = __ffsll((unsigned long long)active) - 1;
-                const int32_t k = __shfl(key, leader, 64);
-                const uint64_t mask = __ballot(valid && key == k);
-                const int32_t bk = vrun[k - 1];
-                if (valid && key == k) dst[i] = bk + __popcll(mask & lt);
-                vrun[k - 1] = bk + __popcll(mask);
-                active &= ~mask;
+    if (blockIdx.x == 0 && tid == 0) {
+        a.ctr->contiguous = 1;
+        a.ctr->n_pos = n;
+    }
+    if ((int64_t)blockIdx.x * (256 * IPT) >= n) return;
+    const int64_t p0 = (int64_t)blockIdx.x * (256 * IPT) + wv * (64 * IPT) + lane;
+    const int32_t lo = range[blockIdx.x].x, hi = range[blockIdx.x].y;
+    const uint64_t lt = mz_lanemask_lt();
+    int32_t key[IPT], dst[IPT];
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const int64_t p = p0 + r * 64;
+        const int32_t k = p < n ? a.key[p] : 0;
+        key[r] = p < n ? (k < 1 ? 1 : (k > n_cells ? n_cells : k)) : 0;
+    }
+    for (int32_t w0 = lo; w0 <= hi; w0 += SORT_KEYS) {
+        const int32_t width = min(SORT_KEYS, hi - w0 + 1);
+        const int nbits = width > 1 ? 32 - __clz(width - 1) : 0;
+        for (int d = tid; d < width; d += 256) tab[d] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {
+            const int32_t d = key[r] - w0;
+            const bool in = key[r] > 0 && d >= 0 && d < width;
+            uint64_t peers = __ballot(in);
+            for (int t = 0; t < nbits; ++t) {
+                const uint64_t m = __ballot((d >> t) & 1);
+                peers &= ((d >> t) & 1) ? m : ~m;
+            }
+            const int first = in ? __ffsll((unsigned long long)peers) - 1 : lane;
+            unsigned long long old = 0;
+            if (in && first == lane) old = atomicAdd(&tab[d], (unsigned long long)__popcll(peers) << (16 * wv));
+            old = (unsigned long long)__shfl((long long)old, first, 64);
+            if (in) dst[r] = (int32_t)((old >> (16 * wv)) & 0xFFFF) + __popcll(peers & lt);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {
+            const int32_t d = key[r] - w0;
+            if (key[r] > 0 && d >= 0 && d < width) {
+                const unsigned long long t = tab[d];
+                int32_t q = dst[r] + cstart[key[r] - 1] + rows[(int64_t)blockIdx.x * n_cells + key[r] - 1];
+                if (wv > 0) q += (int32_t)(t & 0xFFFF);
+                if (wv > 1) q += (int32_t)((t >> 16) & 0xFFFF);
+                if (wv > 2) q += (int32_t)((t >> 32) & 0xFFFF);
+                dst[r] = q;
+            }
+        }
+        __syncthreads();
+    }
+    // four particles' loads in flight a lane (the compiler keeps loads behind
+    // the stores to the other buffers)
+#pragma unroll
+    for (int r0 = 0; r0 < IPT; r0 += 4) {
+        double f[4][7];
+        int32_t id[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t p = p0 + (r0 + q) * 64;
+            if (key[r0 + q] > 0) {
+                f[q][0] = a.x0[p]; f[q][1] = a.x1[p]; f[q][2] = a.x2[p];
+                f[q][3] = a.v0[p]; f[q][4] = a.v1[p]; f[q][5] = a.v2[p];
+                f[q][6] = a.w[p];
+                id[q] = a.id[p];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t d = dst[r0 + q];
+            if (key[r0 + q] > 0) {
+                b.x0[d] = f[q][0]; b.x1[d] = f[q][1]; b.x2[d] = f[q][2];
+                b.v0[d] = f[q][3]; b.v1[d] = f[q][4]; b.v2[d] = f[q][5];
+                b.w[d] = f[q][6];
+                b.id[d] = id[q];
             }
         }
     }
-    __syncthreads();
-#pragma unroll 4
-    for (int i = threadIdx.x; i < cnt; i += 256) {
-        const int64_t p = p0 + i, d = dst[i];
-        b.x0[d] = a.x0[p]; b.x1[d] = a.x1[p]; b.x2[d] = a.x2[p];
-        b.v0[d] = a.v0[p]; b.v1[d] = a.v1[p]; b.v2[d] = a.v2[p];
-        b.w[d] = a.w[p];
-        b.id[d] = a.id[p];
-    }
 }
 
-// Sorting with many cells.  The count matrix of the path above holds
-// n_cells x chunks entries, so its traffic grows with the cell count (12,288
-// cells over 12.8M particles: 1.2 GB per sort).  Past a bound the sort runs
-// as a least-significant-digit radix sort of the (key, position) pairs on
+// Sorting with many cells.  The count matrix of the path above has room for
+// n_cells x chunks entries.  Past a bound the sort runs as a
+// least-significant-digit radix sort of the (key, position) pairs on
 // 8-bit digits of key - 1, whose matrices hold 256 x chunks entries:
 //   k_rs_keys     keys (as k_sort_hist computes them), the clamped copy the
 //                 passes read, and the cell totals (wave-aggregated atomics);
@@ -952,12 +1072,33 @@ __global__ void __launch_bounds__(1024) k_rs_pia(MzSpView sp, int32_t n_cells, c
     }
 }
 
-// the count matrix costs 4 B x cells x chunks; past 32 B per particle slot
-// (or past the LDS histogram's cell bound) the radix path moves less
+// Chunk of the count-matrix sort.  Up to SORT_SMALL_SLOTS slots (and 4,096
+// cells) 1,024, so that a small store still makes hundreds of blocks; past
+// it 4,096, which keeps the matrix at most 16 B per slot up to 16,384 cells.
+// Measured per sort (hist + rows + scatter; before: whole-matrix counts, one
+// wavefront ranking a chunk, the 8-bit radix sort past 8,192 cells):
+//   500 cells, 100k particles        4.5 + 6.1 + 19.0 -> 5.5 + 3.6 + 8.5 us
+//   2,000 cells, 500k, +-15 cells   11.4 + 18.5 + 39.7 -> 5.2 + 4.8 + 14.9 us
+//   4,096 cells, 4.2M in 10.2M slots  474 + 112 + 232 -> 32 + 8 + 123 us
+//   16,000 cells, 4M (radix before)             425 -> 20 + 8 + 131 us
+// The scatter moves 120 B a particle at 3.7 TB/s (a plain copy: 4.7).
+#define SORT_SMALL_SLOTS (1 << 21)
+static int32_t sort_chunk(const mz_store *h, const MzSpecies &s) {
+    return s.cap <= SORT_SMALL_SLOTS && h->n_cells <= 4096 ? MZ_SORT_CHUNK : 4 * MZ_SORT_CHUNK;
+}
+
+// The count matrix may take 16 B per particle slot, the radix path's scratch;
+// with more cells the radix sort runs.
 static bool sort_uses_radix(const mz_store *h, const MzSpecies &s) {
+    return h->sort_path == 2 || (h->sort_path == 0 && h->n_cells > 16384);
+}
+
+// The count-matrix sort of mz_sort_noalloc keeps chunks of 1,024 and the
+// bounds its interface states.
+static bool sort_noalloc_fits(const mz_store *h, const MzSpecies &s) {
     const int64_t nchunks = (s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK;
-    return h->sort_path == 2 ||
-           (h->sort_path == 0 && (h->n_cells > MZ_SORT_MAX_CELLS || (int64_t)h->n_cells * nchunks > 8 * s.cap));
+    return h->sort_path != 2 && (h->sort_path == 1 || (h->n_cells <= MZ_SORT_MAX_CELLS &&
+                                                       (int64_t)h->n_cells * nchunks <= 8 * s.cap));
 }
 
 struct RsScratch {
@@ -986,9 +1127,8 @@ int mz_sort_prealloc(mz_store *h, int species) {
         MZ_CHECK(rs_scratch(h, s, r), "sort: scratch allocation failed");
         return 0;
     }
-    const int64_t nchunks = (s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK;
-    MZ_CHECK(mz_scratch(h, "sort_hist", (size_t)h->n_cells * nchunks * sizeof(int32_t)) != nullptr &&
-                 mz_scratch(h, "sort_cstart", (size_t)h->n_cells * sizeof(int32_t)) != nullptr,
+    const int64_t chunk = sort_chunk(h, s), nchunks = (s.cap + chunk - 1) / chunk;
+    MZ_CHECK(mz_scratch(h, "sort_hist", (size_t)h->n_cells * nchunks * sizeof(int32_t)) != nullptr,
              "sort: scratch allocation failed");
     return 0;
 }
@@ -1047,20 +1187,22 @@ static MzSpView view_b(const MzSpecies &s) {
     return v;
 }
 
-// launches the three sort kernels on the current A buffers; the caller swaps
-// The count-matrix sort's three kernels over the count matrix hist
-// [n_cells][chunks] and the cell starts cstart [n_cells]; every launch
-// overwrites both in full, so neither needs clearing.
-static int launch_count_sort(mz_store *h, MzSpecies &s, int compute_cells, int32_t *hist, int32_t *cstart) {
+// The count-matrix sort's three kernels on the current A buffers (the caller
+// swaps) over the count matrix hist [chunks][n_cells].  What a launch reads
+// of hist, the chunks' ranges and the cell starts it has written itself, and
+// it leaves the cell totals cleared, so none of them needs clearing.
+template <int IPT>
+static int launch_count_sort(mz_store *h, MzSpecies &s, int compute_cells, int32_t *hist) {
     const int nc = h->n_cells;
-    const int32_t nchunks = (int32_t)((s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK);
+    const int32_t chunk = 256 * IPT;
+    const int32_t nchunks = (int32_t)((s.cap + chunk - 1) / chunk);
     MzSpView a = mz_view(s), b = view_b(s);
-    size_t lds = (size_t)nc * sizeof(int32_t);
-    hipLaunchKernelGGL(k_sort_hist, dim3(nchunks), dim3(256), lds, h->stream, a, h->grid, compute_cells, nc,
-                       nchunks, hist);
-    hipLaunchKernelGGL(k_sort_rows, dim3((nc + 3) / 4), dim3(256), 0, h->stream, a, nc, nchunks, hist, cstart,
-                       h->d_ticket);
-    hipLaunchKernelGGL(k_sort_scatter, dim3(nchunks), dim3(256), lds, h->stream, a, b, nc, nchunks, hist, cstart);
+    hipLaunchKernelGGL(k_sort_hist<IPT>, dim3(nchunks), dim3(256), 0, h->stream, a, h->grid, compute_cells, nc, hist,
+                       s.krange, h->d_ccount);
+    hipLaunchKernelGGL(k_sort_rows, dim3((nc + 31) / 32 + 1), dim3(256), 0, h->stream, a, nc, chunk, hist, s.krange,
+                       h->d_ccount, h->d_cstart);
+    hipLaunchKernelGGL(k_sort_scatter<IPT>, dim3(nchunks), dim3(256), 0, h->stream, a, b, nc, hist, s.krange,
+                       h->d_cstart);
     MZ_HIP(hipGetLastError());
     return 0;
 }
@@ -1069,14 +1211,14 @@ int mz_launch_sort(mz_store *h, int species, int compute_cells) {
     MzSpecies &s = h->sp[species - 1];
     int nc = h->n_cells;
     MZ_CHECK(!compute_cells || h->has_grid, "sort: no grid set");
-    int32_t nchunks = (int32_t)((s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK);
     const bool radix = sort_uses_radix(h, s);
-    MZ_CHECK(radix || nc <= MZ_SORT_MAX_CELLS, "sort: too many cells for the LDS histogram");
+    MZ_CHECK(radix || h->sort_path != 1 || nc <= MZ_SORT_MAX_CELLS, "sort: too many cells for the count matrix");
     if (radix) return launch_radix_sort(h, s, mz_view(s), view_b(s), compute_cells);
+    const int64_t chunk = sort_chunk(h, s), nchunks = (s.cap + chunk - 1) / chunk;
     int32_t *hist = (int32_t *)mz_scratch(h, "sort_hist", (size_t)nc * nchunks * sizeof(int32_t));
-    int32_t *cstart = (int32_t *)mz_scratch(h, "sort_cstart", (size_t)nc * sizeof(int32_t));
-    MZ_CHECK(hist != nullptr && cstart != nullptr, "sort: scratch allocation failed");
-    return launch_count_sort(h, s, compute_cells, hist, cstart);
+    MZ_CHECK(hist != nullptr, "sort: scratch allocation failed");
+    return chunk == MZ_SORT_CHUNK ? launch_count_sort<4>(h, s, compute_cells, hist)
+                                  : launch_count_sort<16>(h, s, compute_cells, hist);
 }
 
 extern "C" int mz_set_sort_path(mz_store *h, int32_t path) {
@@ -1146,7 +1288,7 @@ extern "C" int mz_sort_noalloc(mz_store *h, int32_t species, int32_t compute_cel
     MZ_CHECK(species >= 1 && species <= h->n_species, "sort_noalloc: bad species");
     MzSpecies &s = h->sp[species - 1];
     MZ_CHECK(!compute_cells || h->has_grid, "sort_noalloc: no grid set");
-    MZ_CHECK(!sort_uses_radix(h, s),
+    MZ_CHECK(sort_noalloc_fits(h, s),
              "sort_noalloc: only the count-matrix sort runs without allocating (at most 14336 cells, n_cells x "
              "chunks <= 8 x capacity, sort path not radix)");
     const int64_t nc = h->n_cells;
@@ -1169,7 +1311,7 @@ extern "C" int mz_sort_noalloc(mz_store *h, int32_t species, int32_t compute_cel
         s.contig_known = true;
     }
     // no timing bracket: its events would be allocations
-    r = launch_count_sort(h, s, compute_cells, scr, scr + nc * nchunks);
+    r = launch_count_sort<4>(h, s, compute_cells, scr);
     if (r) return r;
     mz_swap_buffers(s);
     return 0;
