@@ -328,25 +328,24 @@ struct NtcWaveDraw {
 // evaluates that lattice: lane a M + j takes the candidate after a
 // collisions and j rejections (T tracks of M candidates, T M <= 64) -- pair,
 // relative speed, collision rate, acceptance test, post-collision
-// velocities.  The wave then walks it in the reference's order, jumping from
-// event to event with ballots: rejections in between need no work, a
-// collision moves to the next track, a new (sigma g w)_max renews every
-// lane's acceptance test.  The window ends, and the next one starts at that
-// draw, at a candidate that shares a particle with a collision of the window
-// or picks one created in it, where the particle count is not the predicted
-// one, and where a track or the tracks run out; T follows the acceptance
-// rate (doubled when the tracks run out, halved when a track does).  A
-// candidate whose k must be drawn again runs on its own.  Same draws, same
-// operands, same order of updates as the loop over ntc_candidate: the results
-// are equal.
+// velocities.  The wave then follows the sequential loop's path through it
+// (mz_window_walk): a new (sigma g w)_max renews every lane's acceptance
+// test, and the window ends, and the next one starts at that draw, at a
+// candidate that shares a particle with a collision of the window or picks
+// one created in it, where the particle count is not the predicted one, and
+// where a track or the tracks run out; then all its collisions are carried
+// out at once.  T follows the acceptance rate (doubled when the tracks run
+// out, halved when a track does).  A candidate whose k must be drawn again
+// runs on its own.  Same draws, same operands, same order of updates as the
+// loop over ntc_candidate: the results are equal.
 //
 // What bounds it: the latency of one window (draw exchange, the two gathers,
 // the power chain; about 4 us) times the windows of the cell with the most.
 // Few acceptances make windows of 40 candidates, many make eight tracks of
 // eight.  Measured against one lane per cell, and against windows that ended
 // at every split: 8,192 boxes of 90 particles with 130 candidates, 8% accepted,
-// 4,030 -> 330 us a call; 2,048 boxes with 580 candidates (up to 3,500), 4%
-// accepted, SWPM, 5,560 -> 285 us; 4,096 boxes with 150 candidates, 39%
+// 4,030 -> 300 us a call; 2,048 boxes with 580 candidates (up to 3,500), 4%
+// accepted, SWPM, 5,560 -> 200 us; 4,096 boxes with 150 candidates, 39%
 // accepted, SWPM, 1,220 -> 190 us; 1,024 cells of up to 30,000 particles, 290
 // candidates (up to 2,900), 40% accepted, 3,250 -> 1,320 us; 500 cells of 35
 // candidates, 5% accepted, 46 -> 22 us.
@@ -431,130 +430,100 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
                 mz_vhs_along(A.mu1, A.mu2, g, vc0, vc1, vc2, e0, e1, e2, ui0, ui1, ui2, uk0, uk1, uk2);
             }
         }
-        // lanes at which the window ends before their candidate
-        uint64_t stop = __ballot(live && fresh);
-        const uint64_t end = __ballot(!live), samem = __ballot(live && same && !fresh), slowm = __ballot(slow);
-        const uint64_t eqm = __ballot(A.equal_weight || fabs(wi - wk) < A.dw_tol), heavym = __ballot(wi > wk);
+        const uint64_t samem = __ballot(live && same && !fresh), slowm = __ballot(slow);
+        const uint64_t stop = __ballot(!live || fresh) | samem | slowm, ends = mz_window_ends(T, M);
+        const bool eq = KIND == NTC_PLAIN || (KIND == NTC_SPLIT && fabs(wi - wk) < A.dw_tol);
+        // collisions after which the particle count is not the predicted one
+        const uint64_t eqm = __ballot(eq), last = KIND != NTC_SPLIT ? 0 : __ballot(eq == (inc > 0));
         uint64_t accm = __ballot(acc), maxm = __ballot(sg > sgwm);
-        int a = 0, j = 0;
-        bool direct = false, at_o = false, ran_out = false;
+        uint64_t taken = 0, seen = 0, dirty = 0, checked = 0;
+        int pos = 0, why;
         for (;;) {
-            if (j >= M) {   // the track ran out
-                ran_out = true;
+            why = mz_window_walk(accm, stop | maxm, last, ends, T * M, M, pos, taken, seen);
+            // candidates that share a particle with an earlier collision
+            for (uint64_t m = taken & ~checked; m; m &= m - 1) {
+                const int L = __builtin_ctzll(m);
+                const int32_t i = __builtin_amdgcn_readlane(si, L), k = __builtin_amdgcn_readlane(sk, L);
+                dirty |= __ballot(single ? si == i || sk == i || si == k || sk == k : si == i || sk == k) &
+                         (~1ull << L);
+            }
+            checked = taken;
+            if (dirty & seen) {
+                pos = __builtin_ctzll(dirty & seen);
+                taken &= (1ull << pos) - 1;
+                why = -1;
                 break;
             }
-            const int at0 = a * M + j;
-            uint64_t track = ~0ull << at0;
-            if (a * M + M < 64) track &= (1ull << (a * M + M)) - 1;
-            const uint64_t hit = (stop | end | samem | slowm | accm | maxm) & track;
-            if (!hit) {
-                cc += M - j;
-                j = M;
-                continue;
-            }
-            const int L = __ffsll((unsigned long long)hit) - 1;
-            const uint64_t bit = 1ull << L;
-            cc += L - at0;
-            j += L - at0;
-            if ((stop | end) & bit) break;
-            if (samem & bit) {
-                direct = true;
-                break;
-            }
-            ++cc;
-            if (slowm & bit) {
-                o = D + (uint64_t)(5 * a + 3 * j + 2);
-                at_o = true;
-                break;
-            }
-            if (maxm & bit) {
-                sgwm = mz_readlane_d(sg, L);   // above the running maximum
-                accm = __ballot(acc && d2 < t / sgwm);
-                maxm = __ballot(sg > sgwm);
-            }
-            if (!(accm & bit)) {
-                ++j;
-                continue;
-            }
+            if (why != MZ_WALK_STOP || (stop >> pos) & 1) break;
+            sgwm = mz_readlane_d(sg, pos);   // above the running maximum
+            accm = __ballot(acc && d2 < t / sgwm);
+            maxm = __ballot(sg > sgwm);
+        }
+        const int a = __popcll(taken), j = pos - a * M;
+        // The window's collisions, all at once: no particle is in two of them.
+        // Each makes at most one split (SWPM: two particles), so the scratch,
+        // one entry (two) per candidate, has room.
+        const bool heavy_i = wi > wk;
+        const bool on_a = KIND != NTC_SPLIT || single || heavy_i;
+        if ((taken >> lane) & 1) {
             if (SWPM) {
-                ++S.performed;
                 const double dw = (wi < wk ? wi : wk) * wtf;
-                if (lane == L) {
-                    (in_i ? A.a.w : A.sc[6])[pi] = wi - dw;
-                    (in_k ? A.b.w : A.sc[6])[pk] = wk - dw;
-                }
-                if (S.ca + 1 >= 2 * C.n_coll) {
-                    if (lane == 0) atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
-                    o = D + (uint64_t)(5 * a + 3 * j + 3);
-                    at_o = true;
-                    break;
-                }
-                if (lane == L) {
-                    const int64_t e = C.s_base + S.ca;
-                    A.sc[0][e] = xi0; A.sc[1][e] = xi1; A.sc[2][e] = xi2;
-                    A.sc[3][e] = ui0; A.sc[4][e] = ui1; A.sc[5][e] = ui2; A.sc[6][e] = dw;
-                    A.sc[0][e + 1] = xk0; A.sc[1][e + 1] = xk1; A.sc[2][e + 1] = xk2;
-                    A.sc[3][e + 1] = uk0; A.sc[4][e + 1] = uk1; A.sc[5][e + 1] = uk2; A.sc[6][e + 1] = dw;
-                }
-                S.ca += 2;
-                S.na += 2;
+                (in_i ? A.a.w : A.sc[6])[pi] = wi - dw;
+                (in_k ? A.b.w : A.sc[6])[pk] = wk - dw;
+                const int64_t e = C.s_base + S.ca + 2 * __popcll(taken & mz_lanemask_lt());
+                A.sc[0][e] = xi0; A.sc[1][e] = xi1; A.sc[2][e] = xi2;
+                A.sc[3][e] = ui0; A.sc[4][e] = ui1; A.sc[5][e] = ui2; A.sc[6][e] = dw;
+                A.sc[0][e + 1] = xk0; A.sc[1][e + 1] = xk1; A.sc[2][e + 1] = xk2;
+                A.sc[3][e + 1] = uk0; A.sc[4][e + 1] = uk1; A.sc[5][e + 1] = uk2; A.sc[6][e + 1] = dw;
             } else {
-                const bool eq = (eqm & bit) != 0, heavy_i = (heavym & bit) != 0;
-                const bool split = CREATES && !eq;
-                const bool on_a = heavy_i || single;
-                const int32_t q = on_a ? (single ? S.ca + S.cb : S.ca) : S.cb;
-                ++S.performed;
-                if (split && q >= C.n_coll) {   // no room for the split: ends before its scattering draws
-                    if (lane == 0) atomicOr(&(on_a ? A.a : A.b).ctr->err, MZ_ERR_SCRATCH);
-                    ++j;
-                    continue;
+                if (KIND == NTC_SPLIT && !eq) {
+                    // the split of the heavier particle
+                    const int32_t q = (on_a ? (single ? S.ca + S.cb : S.ca) : S.cb) +
+                                      __popcll(taken & ~eqm & mz_lanemask_lt());
+                    const int64_t e = (on_a ? 0 : sc_b) + C.s_base + q;
+                    A.sc[0][e] = heavy_i ? xi0 : xk0; A.sc[1][e] = heavy_i ? xi1 : xk1;
+                    A.sc[2][e] = heavy_i ? xi2 : xk2;
+                    A.sc[3][e] = heavy_i ? vi0 : vk0; A.sc[4][e] = heavy_i ? vi1 : vk1;
+                    A.sc[5][e] = heavy_i ? vi2 : vk2;
+                    A.sc[6][e] = heavy_i ? wi - wk : wk - wi;
+                    if (heavy_i) (in_i ? A.a.w : A.sc[6])[pi] = wk;
+                    else (in_k ? A.b.w : A.sc[6])[pk] = wi;
                 }
-                if (eq) {
-                    ++S.eqw;
-                } else if (!CREATES) {
-                    if (lane == 0) atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
-                }
-                if (lane == L) {
-                    if (split) {
-                        const int64_t e = (on_a ? 0 : sc_b) + C.s_base + q;
-                        A.sc[0][e] = heavy_i ? xi0 : xk0; A.sc[1][e] = heavy_i ? xi1 : xk1;
-                        A.sc[2][e] = heavy_i ? xi2 : xk2;
-                        A.sc[3][e] = heavy_i ? vi0 : vk0; A.sc[4][e] = heavy_i ? vi1 : vk1;
-                        A.sc[5][e] = heavy_i ? vi2 : vk2;
-                        A.sc[6][e] = heavy_i ? wi - wk : wk - wi;
-                        if (heavy_i) (in_i ? A.a.w : A.sc[6])[pi] = wk;
-                        else (in_k ? A.b.w : A.sc[6])[pk] = wi;
-                    }
-                    (in_i ? A.a.v0 : A.sc[3])[pi] = ui0; (in_i ? A.a.v1 : A.sc[4])[pi] = ui1;
-                    (in_i ? A.a.v2 : A.sc[5])[pi] = ui2;
-                    (in_k ? A.b.v0 : A.sc[3])[pk] = uk0; (in_k ? A.b.v1 : A.sc[4])[pk] = uk1;
-                    (in_k ? A.b.v2 : A.sc[5])[pk] = uk2;
-                }
-                if (split) {
-                    if (on_a) {
-                        ++S.ca;
-                        ++S.na;
-                    } else {
-                        ++S.cb;
-                        ++S.nb;
-                    }
-                }
-            }
-            const int32_t i = __builtin_amdgcn_readlane(si, L), k = __builtin_amdgcn_readlane(sk, L);
-            stop |= single ? __ballot(si == i || sk == i || si == k || sk == k) : __ballot(si == i || sk == k);
-            ++a;
-            if (single ? S.na != na0 + inc * a : (S.na != na0 || S.nb != nb0)) {
-                if (single && KIND == NTC_SPLIT) inc = S.na - na0 == inc * (a - 1) ? 0 : 1;
-                break;
-            }
-            if (a == T) {
-                T = min(8, 2 * T);
-                break;
+                (in_i ? A.a.v0 : A.sc[3])[pi] = ui0; (in_i ? A.a.v1 : A.sc[4])[pi] = ui1;
+                (in_i ? A.a.v2 : A.sc[5])[pi] = ui2;
+                (in_k ? A.b.v0 : A.sc[3])[pk] = uk0; (in_k ? A.b.v1 : A.sc[4])[pk] = uk1;
+                (in_k ? A.b.v2 : A.sc[5])[pk] = uk2;
             }
         }
-        if (!at_o) o = D + (uint64_t)(5 * a + 3 * j);
-        if (ran_out && 2 * a < T) T = max(1, T / 2);
-        if (a + j == 0 && !at_o) direct = true;   // a first pick out of range by rounding: taken as the loop takes it
+        S.performed += a;
+        if (SWPM) {
+            S.ca += 2 * a;
+            S.na += 2 * a;
+        } else if (KIND == NTC_PLAIN) {
+            S.eqw += a;
+        } else {
+            const uint64_t am = __ballot(on_a);
+            const int ne = __popcll(taken & eqm), na = __popcll(taken & ~eqm & am), nb = a - ne - na;
+            S.eqw += ne;
+            S.ca += na;
+            S.na += na;
+            S.cb += nb;
+            S.nb += nb;
+            if (why == MZ_WALK_LAST && single) inc ^= 1;   // the prediction for the next window
+        }
+        cc += a + j;
+        o = D + (uint64_t)(5 * a + 3 * j);
+        if (why == MZ_WALK_TRACKS) T = min(8, 2 * T);
+        else if (why == MZ_WALK_TRACK && 2 * a < T) T = max(1, T / 2);
+        bool direct = false;
+        if (why == MZ_WALK_STOP) {
+            direct = ((samem >> pos) & 1) || pos == 0;   // pos 0: a pick out of range by rounding
+            if ((slowm >> pos) & 1) {                     // g <= eps: two draws, no acceptance test
+                direct = false;
+                ++cc;
+                o += 2;
+            }
+        }
         S.sgwm = sgwm;
         // the window's stores before the loads that follow: one wave's vector
         // memory operations stay in order, so this only holds the compiler

@@ -99,6 +99,49 @@ __device__ inline void mz_vhs_scatter(const MzRngParams &rp, MzStream &st, doubl
     mz_vhs_post(mu1, mu2, g, vc0, vc1, vc2, R_phi, R_ct, vi0, vi1, vi2, vk0, vk1, vk2);
 }
 
+// The walk over a window of candidates evaluated ahead by one wavefront.
+// Lane a M + j holds the candidate reached after `a` collisions and `j`
+// rejections of the window (T tracks of M lanes, T M <= 64), so the path of
+// the sequential loop is: a rejected candidate leads to the next lane, one
+// that collides to the lane M further.  All masks hold one bit per lane and
+// are the same on every lane; the path only moves up, so it is followed in
+// scalar registers, from event to event:
+//   acc    the candidate collides,
+//   stop   the window ends before the candidate,
+//   last   the candidate is accepted and the window ends after it,
+//   ends   the last lane of each track.
+// Follows the path from lane pos; on return pos is where it ended (past the
+// tracks' lanes when they ran out, one past a track's last lane when that track did),
+// `taken` gains the lanes that collide and `seen` the lanes it came by.
+enum { MZ_WALK_STOP = 0, MZ_WALK_LAST = 1, MZ_WALK_TRACKS = 2, MZ_WALK_TRACK = 3 };
+
+__device__ __forceinline__ int mz_window_walk(uint64_t acc, uint64_t stop, uint64_t last, uint64_t ends,
+                                              int lanes, int M, int &pos, uint64_t &taken, uint64_t &seen) {
+    const uint64_t ev = acc | stop | ends;
+    for (;;) {
+        const int p0 = pos;
+        pos += __builtin_ctzll(ev >> pos);   // never empty: every track has an end
+        const uint64_t bit = 1ull << pos;
+        seen |= (bit | (bit - 1)) & (~0ull << p0);
+        if (stop & bit) return MZ_WALK_STOP;
+        if (!(acc & bit)) {
+            ++pos;
+            return MZ_WALK_TRACK;
+        }
+        taken |= bit;
+        pos += M;
+        if (last & bit) return MZ_WALK_LAST;
+        if (pos >= lanes) return MZ_WALK_TRACKS;
+    }
+}
+
+// The last lane of each track.
+__device__ __forceinline__ uint64_t mz_window_ends(int T, int M) {
+    uint64_t e = 0;
+    for (int a = 1; a <= T; ++a) e |= 1ull << (a * M - 1);
+    return e;
+}
+
 // Diffuse re-emission from a wall: three draws (normal, tangential speed
 // factors clamped at 1e-50, then the tangential angle).
 __device__ inline void mz_diffuse_reflect(const MzRngParams &rp, MzStream &st, double &v0, double &v1, double &v2,

@@ -38,7 +38,6 @@
 #include <cstring>
 #include <vector>
 
-#define SLAB_THREADS 256
 #define SLAB_MAXC 32                  // cells per slab
 #define SLAB_KMAX (SLAB_MAXC + 2)     // keys: local cells, left, right
 #define SLAB_MB_CAP 256               // particles per mailbox (slab side, step parity)
@@ -151,10 +150,38 @@ __device__ inline void slab_raise_abort(const SlabArgs &A) {
 }
 
 // Draw k of the cell's stream: from the block of draws the workgroup
-// computed ahead, then from the stream itself.
+// computed ahead (if any), then from the stream itself.
 __device__ inline double slab_draw(const MzRngParams &rp, MzStream &st, const double *pre) {
-    if (st.k < SLAB_DRAWS) return pre[st.k++];
+    if (pre && st.k < SLAB_DRAWS) return pre[st.k++];
     return mz_rand(rp, st);
+}
+
+// One candidate of ntc_equal_weight! over the cell's LDS segment; 1 when it
+// collides.
+__device__ inline int32_t slab_candidate(const SlabArgs &A, const MzRngParams &rp, MzStream &st, const double *pre,
+                                         int32_t base, int32_t nla, double *sv0, double *sv1, double *sv2,
+                                         const double *sw, double &sgwm) {
+    int32_t i = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
+    int32_t k = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
+    while (i == k) k = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
+    const int pi = base + i, pk = base + k;
+    double vi0 = sv0[pi], vi1 = sv1[pi], vi2 = sv2[pi];
+    double vk0 = sv0[pk], vk1 = sv1[pk], vk2 = sv2[pk];
+    double g0, g1, g2;
+    double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
+    if (!(g > MZ_G_EPS)) return 0;
+    double sgw = mz_vhs_sgw(A.factor, A.expo, g, sw[pi], sw[pk]);
+    sgwm = sgw > sgwm ? sgw : sgwm;
+    if (!(slab_draw(rp, st, pre) < sgw / sgwm)) return 0;
+    double vc0, vc1, vc2;
+    mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
+    double ui0, ui1, ui2, uk0, uk1, uk2;
+    const double R_phi = slab_draw(rp, st, pre);
+    const double R_ct = slab_draw(rp, st, pre);
+    mz_vhs_post(A.mu1, A.mu2, g, vc0, vc1, vc2, R_phi, R_ct, ui0, ui1, ui2, uk0, uk1, uk2);
+    sv0[pi] = ui0; sv1[pi] = ui1; sv2[pi] = ui2;
+    sv0[pk] = uk0; sv1[pk] = uk1; sv2[pk] = uk2;
+    return 1;
 }
 
 // ntc_equal_weight! of one cell over its LDS segment [base, base + nla);
@@ -171,42 +198,143 @@ __device__ inline void slab_ntc_cell(const SlabArgs &A, const MzRngParams &rp, i
         n_coll = 0;
     }
     performed = 0;
-    eqw = 0;
-    for (int64_t cc = 0; cc < n_coll; ++cc) {
-        int32_t i = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
-        int32_t k = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
-        while (i == k) k = (int32_t)floor(slab_draw(rp, st, pre) * (double)nla);
-        const int pi = base + i, pk = base + k;
-        double vi0 = sv0[pi], vi1 = sv1[pi], vi2 = sv2[pi];
-        double vk0 = sv0[pk], vk1 = sv1[pk], vk2 = sv2[pk];
-        double g0, g1, g2;
-        double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
-        if (!(g > MZ_G_EPS)) continue;
-        double sgw = mz_vhs_sgw(A.factor, A.expo, g, sw[pi], sw[pk]);
-        sgwm = sgw > sgwm ? sgw : sgwm;
-        if (!(slab_draw(rp, st, pre) < sgw / sgwm)) continue;
-        ++performed;
-        ++eqw;
-        double vc0, vc1, vc2;
-        mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
-        double ui0, ui1, ui2, uk0, uk1, uk2;
-        const double R_phi = slab_draw(rp, st, pre);
-        const double R_ct = slab_draw(rp, st, pre);
-        mz_vhs_post(A.mu1, A.mu2, g, vc0, vc1, vc2, R_phi, R_ct, ui0, ui1, ui2, uk0, uk1, uk2);
-        sv0[pi] = ui0; sv1[pi] = ui1; sv2[pi] = ui2;
-        sv0[pk] = uk0; sv1[pk] = uk1; sv2[pk] = uk2;
-    }
+    for (int64_t cc = 0; cc < n_coll; ++cc) performed += slab_candidate(A, rp, st, pre, base, nla, sv0, sv1, sv2, sw, sgwm);
+    eqw = performed;
     n_coll_out = (int32_t)n_coll;
 }
 
-template <int R, bool AVG>
-__global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(SlabArgs A) {
-    constexpr int P = R * SLAB_THREADS;   // LDS particle capacity
+// The same on a whole wavefront, candidates evaluated ahead (the windows of
+// mz_ntc.hip, without created particles): the candidate reached after a
+// collisions and r rejections starts at draw D + 5 a + 3 r, point a M + j is the
+// one after a collisions and j rejections, a lane each, and the wave
+// walks them in order with ballots; the number T of tracks is kept from step
+// to step.  nd draws are ready in pre; a window past them computes its own.
+// All lanes return the same values.
+__device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &rp, int c, double Vc, int32_t base,
+                                          int32_t nla, double *sv0, double *sv1, double *sv2, const double *sw,
+                                          const double *pre, int nd, int &T, double &sgwm, int32_t &n_coll_out,
+                                          int32_t &performed, int32_t &eqw) {
+    const int lane = threadIdx.x & 63;
+    int64_t est = (int64_t)floor(mz_ncoll_est(true, A.dt, nla, nla, sgwm, Vc, pre[0]));
+    if (!(est <= MZ_NTC_MAX_CANDIDATES)) {
+        if (lane == 0) atomicOr(&A.a.ctr->err, MZ_ERR_SCRATCH);
+        est = 0;
+    }
+    // uniform values kept in scalar registers: the walk then runs there
+    const int32_t n_coll = __builtin_amdgcn_readfirstlane((int32_t)est);
+    performed = 0;
+    int32_t cc = 0;
+    uint32_t o = 1;   // the next draw: at most 2^32 / 5 candidates' draws
+    while (cc < n_coll) {
+        const uint32_t D = o;
+        const int M = 64 / T;   // T = 1, 2, 4 or 8
+        const int a_l = lane / M, j_l = lane - a_l * M;
+        const bool live = cc + a_l + j_l < n_coll;
+        const uint32_t sL = D + (uint32_t)(5 * a_l + 3 * j_l);
+        double d0, d1, d2, d3, d4;
+        if (D + (uint32_t)(5 * (T - 1) + 3 * (M - 1) + 5) <= (uint32_t)nd) {
+            d0 = pre[sL]; d1 = pre[sL + 1]; d2 = pre[sL + 2]; d3 = pre[sL + 3]; d4 = pre[sL + 4];
+        } else {
+            double h0, h1, h2, h3, h4, h5;
+            mz_philox_pair(rp, (uint64_t)c, sL >> 1, h0, h1);
+            mz_philox_pair(rp, (uint64_t)c, (sL >> 1) + 1, h2, h3);
+            mz_philox_pair(rp, (uint64_t)c, (sL >> 1) + 2, h4, h5);
+            const bool odd = sL & 1;
+            d0 = odd ? h1 : h0; d1 = odd ? h2 : h1; d2 = odd ? h3 : h2; d3 = odd ? h4 : h3; d4 = odd ? h5 : h4;
+        }
+        const int32_t si = (int32_t)floor(d0 * (double)nla), sk = (int32_t)floor(d1 * (double)nla);
+        const bool same = si == sk;
+        const int pi = base + si, pk = base + sk;
+        double g0, g1, g2, e0, e1, e2;
+        const double vi0 = sv0[pi], vi1 = sv1[pi], vi2 = sv2[pi];
+        const double vk0 = sv0[pk], vk1 = sv1[pk], vk2 = sv2[pk];
+        const double g = mz_rel_speed(vi0, vi1, vi2, vk0, vk1, vk2, g0, g1, g2);
+        const bool slow = live && !same && !(g > MZ_G_EPS);
+        const double sg = live && !same && !slow ? mz_vhs_sgw(A.factor, A.expo, g, sw[pi], sw[pk]) : 0.0;
+        mz_vhs_dir(d3, d4, e0, e1, e2);
+        const uint64_t samem = __ballot(live && same), slowm = __ballot(slow);
+        const uint64_t stop = __ballot(!live) | samem | slowm, ends = mz_window_ends(T, M);
+        uint64_t accm = __ballot(d2 < sg / sgwm), maxm = __ballot(sg > sgwm);
+        uint64_t taken = 0, seen = 0, dirty = 0, checked = 0;
+        int pos = 0, why;
+        for (;;) {
+            why = mz_window_walk(accm, stop | maxm, 0, ends, 64, M, pos, taken, seen);
+            // candidates that share a particle with an earlier collision
+            for (uint64_t m = taken & ~checked; m; m &= m - 1) {
+                const int L = __builtin_ctzll(m);
+                const int32_t i = __builtin_amdgcn_readlane(si, L), k = __builtin_amdgcn_readlane(sk, L);
+                dirty |= __ballot(si == i || sk == i || si == k || sk == k) & (~1ull << L);
+            }
+            checked = taken;
+            if (dirty & seen) {
+                pos = __builtin_ctzll(dirty & seen);
+                taken &= (1ull << pos) - 1;
+                why = -1;
+                break;
+            }
+            if (why != MZ_WALK_STOP || (stop >> pos) & 1) break;
+            sgwm = mz_readlane_d(sg, pos);   // above the running maximum
+            accm = __ballot(d2 < sg / sgwm);
+            maxm = __ballot(sg > sgwm);
+        }
+        if ((taken >> lane) & 1) {
+            double vc0, vc1, vc2, ui0, ui1, ui2, uk0, uk1, uk2;
+            mz_com(A.mu1, A.mu2, vi0, vi1, vi2, vk0, vk1, vk2, vc0, vc1, vc2);
+            mz_vhs_along(A.mu1, A.mu2, g, vc0, vc1, vc2, e0, e1, e2, ui0, ui1, ui2, uk0, uk1, uk2);
+            sv0[pi] = ui0; sv1[pi] = ui1; sv2[pi] = ui2;
+            sv0[pk] = uk0; sv1[pk] = uk1; sv2[pk] = uk2;
+        }
+        const int a = __popcll(taken), j = pos - a * M;
+        performed += a;
+        cc += a + j;
+        o = D + (uint32_t)(5 * a + 3 * j);
+        if (why == MZ_WALK_TRACKS) T = min(8, 2 * T);
+        else if (why == MZ_WALK_TRACK && 2 * a < T) T = max(1, T / 2);
+        bool direct = false;
+        if (why == MZ_WALK_STOP) {
+            direct = (samem >> pos) & 1;
+            if ((slowm >> pos) & 1) {   // g <= eps: two draws, no acceptance test
+                ++cc;
+                o += 2;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if (direct) {
+            // k drawn again: this candidate on its own, on one lane
+            double sgl = sgwm;
+            uint32_t ol = 0;
+            int32_t done = 0;
+            if (lane == 0) {
+                MzStream st = mz_stream((uint64_t)c, o);
+                done = slab_candidate(A, rp, st, nullptr, base, nla, sv0, sv1, sv2, sw, sgl);
+                ol = (uint32_t)st.k;
+            }
+            sgwm = mz_readlane_d(sgl, 0);
+            o = (uint32_t)__builtin_amdgcn_readlane((int)ol, 0);
+            performed += __builtin_amdgcn_readlane(done, 0);
+            ++cc;
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+    }
+    eqw = performed;
+    n_coll_out = n_coll;
+}
+
+// R particles per thread, NT threads: slabs of up to 512 particles run 256
+// threads, two workgroups per CU; larger ones 512 (256 in the averaging
+// phase), one workgroup per CU (50 cells of 1,000 particles, us per step of a
+// slab: convection and ranking 5.6 -> 1.7, mailbox 2.7 -> 1.8, scatter 1.4 ->
+// 0.9; the whole step 65 -> 22 with the windows and the list of wall hits).
+template <int R, bool AVG, int NT>
+__global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(SlabArgs A) {
+    constexpr int P = R * NT;             // LDS particle capacity
+    constexpr int NW = NT / 64;           // waves
+    constexpr bool LARGE = P >= 1024;
     constexpr int NCH = P / 64;           // 64-particle chunks
-    // With R <= 4 the velocities the sort left are also kept in a snapshot,
+    // Up to 1,024 particles the velocities the sort left are also kept in a snapshot,
     // so a step's props run next to the following NTC; the largest slabs have
     // no LDS room for it and compute props right after the scatter.
-    constexpr bool SNAP = R <= 4;
+    constexpr bool SNAP = P <= 1024;
     constexpr int PS = SNAP ? P : 1;
     static_assert(NCH <= 64, "chunk scan uses one wave");
     __shared__ double sx0[P], sx1[P], sx2[P], sv0[P], sv1[P], sv2[P], sw[P];
@@ -215,7 +343,9 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     __shared__ int32_t tot[SLAB_KMAX];
     __shared__ int32_t cst[SLAB_MAXC], ccn[SLAB_MAXC], runL[SLAB_MAXC], runR[SLAB_MAXC];
     __shared__ int32_t arank[2][SLAB_MB_CAP], akey[2][SLAB_MB_CAP];
-    __shared__ double sdraw[SLAB_MAXC][SLAB_DRAWS];
+    // the cells' first draws of a step: SLAB_DRAWS each, or in the large slabs
+    // an even share of the whole array
+    __shared__ double sdraw[SLAB_MAXC * SLAB_DRAWS];
     __shared__ double ss0[PS], ss1[PS], ss2[PS];   // velocities as the last sort left them (props input)
     constexpr int WC = SNAP ? SLAB_WALL_CAP : 1;
     __shared__ double swl[3][WC];                  // reflected velocities drawn ahead (wall slab)
@@ -224,11 +354,11 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     // assumed and the end position (NaN where the flight bounces again)
     constexpr int WX = (SNAP && !AVG) ? SLAB_WALL_CAP : 1;
     __shared__ double swv[WX], swx[WX];
-    __shared__ int32_t s_abort, s_n, s_na[2];
-    __shared__ int64_t s_red[4][4];
+    __shared__ int32_t s_abort, s_n, s_na[2], s_hits;
+    __shared__ int64_t s_red[NW][4];
     constexpr int SC = AVG ? SLAB_SURF_CAP : 1;
-    __shared__ double srec[AVG ? 4 : 1][SC][8];   // wall contacts of the last convection, per wave
-    __shared__ int32_t scnt[4];
+    __shared__ double srec[AVG ? NW : 1][SC][8];   // wall contacts of the last convection, per wave
+    __shared__ int32_t scnt[NW];
     __shared__ double pav[AVG ? SLAB_MAXC : 1][6];  // the slab's cells' time-averaged props
 
     const int b = blockIdx.x;
@@ -237,7 +367,8 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     // the check before the launch found a state this kernel cannot take, or
     // another slab has already aborted: touch nothing
     if (__hip_atomic_load(A.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform, so its branches and cells are scalar
     const int clo = g * A.spc;
     const int chi = min(A.n_cells, clo + A.spc) - 1;
     const int ncl = chi - clo + 1;
@@ -272,7 +403,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         if (tid == 0) slab_raise_abort(A);
         return;
     }
-    for (int i = tid; i < n_loc; i += SLAB_THREADS) {
+    for (int i = tid; i < n_loc; i += NT) {
         const int64_t p = (int64_t)first + i;
         sx0[i] = A.a.x0[p]; sx1[i] = A.a.x1[p]; sx2[i] = A.a.x2[p];
         sv0[i] = A.a.v0[p]; sv1[i] = A.a.v1[p]; sv2[i] = A.a.v2[p];
@@ -280,12 +411,13 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         sid[i] = A.a.id[p];
         if (SNAP) { ss0[i] = sv0[i]; ss1[i] = sv1[i]; ss2[i] = sv2[i]; }
     }
-    // NTC lanes: cell k runs on lane k / 4 of wave k % 4
-    const int my_k = lane * 4 + wave;
-    const bool ntc_lane = lane < SLAB_MAXC / 4 && my_k < ncl;
+    // NTC lanes: cell k runs on lane k / NW of wave k % NW
+    const int my_k = lane * NW + wave;
+    const bool ntc_lane = lane < SLAB_MAXC / NW && my_k < ncl;
     double my_sgwm = ntc_lane ? A.sgwm[clo + my_k] : 0.0;
     const double my_V = ntc_lane ? A.V[clo + my_k] : 1.0;
     int32_t my_nla = 0, my_ncoll = 0, my_perf = 0, my_eqw = 0;
+    int ntc_tracks = 8;   // of slab_ntc_cell_wave
 
     double px0[R], px1[R], px2[R], pv0[R], pv1[R], pv2[R], pw[R];
     int32_t pid[R], pkey[R], prank[R], pcell[R];
@@ -294,20 +426,27 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
 
     // The first SLAB_DRAWS draws of every cell's NTC stream for step stp,
     // computed by threads t0, t0 + stride, ...
+    constexpr bool WAVE_NTC = LARGE;
+    // The large slabs' particles that reach a wall (a few per cent of the wall
+    // cell, so some in every 64) are listed, in the arrival-rank rows, and
+    // flown one per lane, so a wave spends one reflection's latency (about 3
+    // us) and not one for each particle slot of its threads.
+    constexpr bool HIT_LIST = LARGE && !AVG;
+    const int nd = WAVE_NTC ? (ncl <= 8 ? 256 : SLAB_DRAWS) : SLAB_DRAWS;
     auto fill_draws = [&](uint64_t stp, int t0, int stride) {
         MzRngParams rpf = A.rp;
         rpf.tag = (stp << 4) | 1u;
-        for (int j = t0; j < ncl * (SLAB_DRAWS / 2); j += stride) {
-            const int k = j / (SLAB_DRAWS / 2), blk = j % (SLAB_DRAWS / 2);
-            mz_philox_pair(rpf, (uint64_t)(clo + k), (uint64_t)blk, sdraw[k][2 * blk], sdraw[k][2 * blk + 1]);
+        for (int j = t0; j < ncl * (nd / 2); j += stride) {
+            const int k = j / (nd / 2), blk = j % (nd / 2);
+            mz_philox_pair(rpf, (uint64_t)(clo + k), (uint64_t)blk, sdraw[k * nd + 2 * blk], sdraw[k * nd + 2 * blk + 1]);
         }
     };
     // compute_props_sorted! of the slab's cells from the snapshot the last
-    // scatter wrote: cell k on wave (k + 1) % 4, the sums of k_props.  It runs
-    // while the next step's NTC, on wave k % 4, changes the live velocities.
+    // scatter wrote: cell k on wave (k + 1) % NW, the sums of k_props.  It runs
+    // while the next step's NTC, on wave k % NW, changes the live velocities.
     auto props_cells = [&]() {
         for (int k = 0; k < ncl; ++k) {
-            if (((k + 1) & 3) != wave) continue;
+            if ((k + 1) % NW != wave) continue;
             const int32_t st1 = cst[k], tn = ccn[k];
             auto get = [&](int32_t i, double &w, double &v0, double &v1, double &v2) {
                 const int p = st1 + i;
@@ -345,7 +484,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     // waves that carry no NTC or props cell do it: waves 2-3 of a one-cell
     // slab, wave 3 of a two-cell slab.
     int wall_side = -1;
-    if (SNAP && has_left != has_right && ncl <= 2) {
+    if (SNAP && !HIT_LIST && has_left != has_right && ncl <= 2) {
         const int s = has_left ? 1 : 0;
         if (A.wl.acc[s] == 1.0) wall_side = s;
     }
@@ -359,7 +498,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         MzRngParams rpw = A.rp;
         rpw.tag = (stp << 4) | 2u;
         const int32_t lo = cst[wall_k], n = min(ccn[wall_k], SLAB_WALL_CAP);
-        const int nthr = SLAB_THREADS - wall_w0 * 64;
+        const int nthr = NT - wall_w0 * 64;
         int32_t *list = arank[wave & 1];
         int nh = 0;
         for (int j0 = (wave - wall_w0) * 64; j0 < n; j0 += nthr) {
@@ -395,10 +534,10 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
             }
         }
     };
-    if (A.n_steps > 0) fill_draws(A.step0, tid, SLAB_THREADS);
+    if (A.n_steps > 0) fill_draws(A.step0, tid, NT);
     const int32_t pn = A.n_cells;
     if (AVG) {
-        if (tid < 4) scnt[tid] = 0;
+        if (tid < NW) scnt[tid] = 0;
         if (tid < ncl * 6) {
             const int k = tid / 6, f = tid % 6, c = clo + k;
             pav[k][f] = f == 0 ? A.pavg[c] : f == 1 ? A.pavg[pn + c]
@@ -413,7 +552,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         if (lane < 2 * MZ_SURF_Q) {
             const int e = lane / MZ_SURF_Q, k = lane % MZ_SURF_Q;
             double sum = 0.0;
-            for (int w = 0; w < 4; ++w) {
+            for (int w = 0; w < NW; ++w) {
                 const int n = min((int)scnt[w], SLAB_SURF_CAP);
                 for (int j = 0; j < n; ++j) {
                     const double *r = srec[w][j];
@@ -426,7 +565,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
             surf_acc = fma(inst, A.avg_inv, surf_acc);
             surf_last = inst;
         }
-        if (lane < 4) scnt[lane] = 0;
+        if (lane < NW) scnt[lane] = 0;
     };
     __syncthreads();
 
@@ -437,14 +576,29 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         // ---- 1. ntc_equal_weight! per cell (its draws were computed during
         // the previous step), next to the previous step's props; clear the
         // ranking tables.
-        for (int j = tid; j < NCH * SLAB_KMAX; j += SLAB_THREADS) (&tab[0][0])[j] = 0;
+        for (int j = tid; j < NCH * SLAB_KMAX; j += NT) (&tab[0][0])[j] = 0;
         if (tid < SLAB_MAXC) { runL[tid] = 0; runR[tid] = 0; }
+        if (HIT_LIST && tid == 0) s_hits = 0;
         if (SNAP && t > 0 && props_due(t - 1)) props_cells();
-        if (ntc_lane) {
+        if (WAVE_NTC) {
+            MzRngParams rp = A.rp;
+            rp.tag = (step << 4) | 1u;
+            for (int k = wave, l = 0; k < ncl; k += NW, ++l) {   // its values on lane l
+                const int32_t nla = ccn[k];
+                double sg = mz_readlane_d(my_sgwm, l);
+                int32_t nc_, pf_, eq_;
+                slab_ntc_cell_wave(A, rp, clo + k, mz_readlane_d(my_V, l), cst[k], nla, sv0, sv1, sv2, sw,
+                                   sdraw + k * nd, nd, ntc_tracks, sg, nc_, pf_, eq_);
+                if (lane == l) {
+                    my_sgwm = sg;
+                    my_nla = nla; my_ncoll = nc_; my_perf = pf_; my_eqw = eq_;
+                }
+            }
+        } else if (ntc_lane) {
             MzRngParams rp = A.rp;
             rp.tag = (step << 4) | 1u;
             my_nla = ccn[my_k];
-            slab_ntc_cell(A, rp, clo + my_k, my_V, cst[my_k], my_nla, sv0, sv1, sv2, sw, sdraw[my_k], my_sgwm,
+            slab_ntc_cell(A, rp, clo + my_k, my_V, cst[my_k], my_nla, sv0, sv1, sv2, sw, sdraw + my_k * nd, my_sgwm,
                           my_ncoll, my_perf, my_eqw);
         }
         if (wall_side >= 0 && wave >= wall_w0) wall_draws(step);
@@ -454,9 +608,40 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         {
             MzRngParams rp = A.rp;
             rp.tag = (step << 4) | 2u;
+            uint32_t flown = 0;   // bit r: the flight of this thread's r-th particle is done
+            if (HIT_LIST && !(has_left && has_right)) {
+                for (;;) {   // as many as the list takes at a time
+                    for (int r = 0; r < R; ++r) {
+                        const int i = r * NT + tid;
+                        if (i < n_loc && !((flown >> r) & 1)) {
+                            const double x_new = fma(sv0[i], A.dt, sx0[i]);
+                            if (!(x_new < A.g.L && x_new > 0.0)) {
+                                const int h = atomicAdd(&s_hits, 1);
+                                if (h < 2 * SLAB_MB_CAP) {
+                                    (&arank[0][0])[h] = i;
+                                    flown |= 1u << r;
+                                }
+                            }
+                        }
+                    }
+                    __syncthreads();
+                    const int hits = s_hits;
+                    for (int h = tid; h < min(hits, 2 * SLAB_MB_CAP); h += NT) {
+                        const int i = (&arank[0][0])[h];
+                        double x0 = sx0[i], v0 = sv0[i], v1 = sv1[i], v2 = sv2[i];
+                        mz_convect_one(rp, A.g, A.wl, 0, A.dt, sid[i], x0, v0, v1, v2, &A.a.ctr->err);
+                        sx0[i] = x0;
+                        sv0[i] = v0; sv1[i] = v1; sv2[i] = v2;
+                    }
+                    __syncthreads();
+                    if (hits <= 2 * SLAB_MB_CAP) break;
+                    if (tid == 0) s_hits = 0;
+                    __syncthreads();
+                }
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const int i = r * SLAB_THREADS + tid;
+                const int i = r * NT + tid;
                 const bool valid = i < n_loc;
                 pkey[r] = -1;
                 prank[r] = 0;
@@ -466,9 +651,9 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
                     pw[r] = sw[i];
                     pid[r] = sid[i];
                     double x_new = fma(pv0[r], A.dt, px0[r]);
-                    if (x_new < A.g.L && x_new > 0.0) {
+                    if (HIT_LIST ? !((flown >> r) & 1) : (x_new < A.g.L && x_new > 0.0)) {
                         px0[r] = x_new < A.g.min_x ? A.g.min_x : (x_new > A.g.max_x ? A.g.max_x : x_new);
-                    } else {
+                    } else if (!HIT_LIST) {
                         double p0 = 0.0, p1 = 0.0, p2 = 0.0;
                         int pre_bc = -1;
                         bool done = false;
@@ -511,7 +696,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
                     }
                     pkey[r] = key;
                 }
-                const int ch = r * 4 + wave;
+                const int ch = r * NW + wave;
                 uint64_t active = __ballot(valid);
                 while (active) {
                     const int leader = __ffsll((unsigned long long)active) - 1;
@@ -530,7 +715,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         // its own.
         constexpr bool SMALL_SCAN = NCH <= 8;
         if (!SMALL_SCAN) {
-            for (int kk = wave; kk < K; kk += 4) {
+            for (int kk = wave; kk < K; kk += NW) {
                 int32_t v = lane < NCH ? tab[lane][kk] : 0;
                 int32_t x = v;
 #pragma unroll
@@ -556,12 +741,12 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
             for (int r = 0; r < R; ++r) {
                 if (pkey[r] < 0) continue;
                 if (SMALL_SCAN) {
-                    const int ch = r * 4 + wave;
+                    const int ch = r * NW + wave;
                     int32_t base = 0;
                     for (int c2 = 0; c2 < ch; ++c2) base += tab[c2][pkey[r]];
                     prank[r] += base;
                 } else {
-                    prank[r] += tab[r * 4 + wave][pkey[r]];
+                    prank[r] += tab[r * NW + wave][pkey[r]];
                 }
                 if (pkey[r] >= KL && prank[r] < SLAB_MB_CAP) {
                     const int side = pkey[r] == KL ? 0 : 1;
@@ -664,7 +849,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
                 }
             }
         }
-        if (wave >= 2 && t + 1 < A.n_steps) fill_draws(step + 1, tid - 128, SLAB_THREADS - 128);
+        if (wave >= 2 && t + 1 < A.n_steps) fill_draws(step + 1, tid - 128, NT - 128);
         __syncthreads();
         if (s_abort) {
             if (tid == 0) slab_raise_abort(A);
@@ -741,7 +926,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         {
             // arrivals beyond the first 64 of a side are read again
             const int xl = max(s_na[0] - 64, 0), xr = max(s_na[1] - 64, 0);
-            for (int j = tid; j < xl + xr; j += SLAB_THREADS) {
+            for (int j = tid; j < xl + xr; j += NT) {
                 const int s = j < xl ? 0 : 1;
                 const int jj = 64 + (s == 0 ? j : j - xl);
                 const int key = akey[s][jj];
@@ -777,7 +962,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     }
     int64_t pre_prev = 0, pre_new = 0, all_new = 0;
     bool ok = true;
-    for (int s = tid; s < A.n_slabs; s += SLAB_THREADS) {
+    for (int s = tid; s < A.n_slabs; s += NT) {
         uint64_t v = 0;
         if (!slab_wait(A.fin + (size_t)s * SLAB_LINE, 1, 0, A.abort_flag, v)) {
             ok = false;
@@ -801,15 +986,18 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
         if (tid == 0) slab_raise_abort(A);
         return;
     }
-    const int64_t off_prev = s_red[0][0] + s_red[1][0] + s_red[2][0] + s_red[3][0];
-    const int64_t off_new = s_red[0][1] + s_red[1][1] + s_red[2][1] + s_red[3][1];
-    const int64_t total = s_red[0][2] + s_red[1][2] + s_red[2][2] + s_red[3][2];
+    int64_t off_prev = 0, off_new = 0, total = 0;
+    for (int w = 0; w < NW; ++w) {
+        off_prev += s_red[w][0];
+        off_new += s_red[w][1];
+        total += s_red[w][2];
+    }
     if (off_new + n_loc > A.a.cap || off_prev + n_prev > A.a.cap) {
         // counts that do not add up to the store: flag it, write nothing
         if (tid == 0) atomicOr(&A.a.ctr->err, MZ_ERR_CAPACITY);
         return;
     }
-    for (int i = tid; i < n_loc; i += SLAB_THREADS) {
+    for (int i = tid; i < n_loc; i += NT) {
         const int64_t p = off_new + i;
         A.bx0[p] = sx0[i]; A.bx1[p] = sx1[i]; A.bx2[p] = sx2[i];
         A.bv0[p] = sv0[i]; A.bv1[p] = sv1[i]; A.bv2[p] = sv2[i];
@@ -819,7 +1007,7 @@ __global__ void __launch_bounds__(SLAB_THREADS, R <= 2 ? 2 : 1) k_slab_couette(S
     // pv.cell keeps the cells of the last sort's input order
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int i = r * SLAB_THREADS + tid;
+        const int i = r * NT + tid;
         if (i < n_prev) A.a.key[off_prev + i] = pcell[r];
     }
     if (tid < ncl) {
@@ -1004,15 +1192,17 @@ struct SlabShape {
     SlabKernel fn = nullptr;
 };
 
-SlabKernel slab_kernel(int R, bool avg = false) {
-    switch (R) {
-    case 1: return avg ? k_slab_couette<1, true> : k_slab_couette<1, false>;
-    case 2: return avg ? k_slab_couette<2, true> : k_slab_couette<2, false>;
-    case 4: return avg ? k_slab_couette<4, true> : k_slab_couette<4, false>;
-    case 8: return avg ? k_slab_couette<8, true> : k_slab_couette<8, false>;
+// the kernel of slabs of 256 ppt particles, and its threads
+SlabKernel slab_kernel(int ppt, bool avg = false) {
+    switch (ppt) {
+    case 1: return avg ? k_slab_couette<1, true, 256> : k_slab_couette<1, false, 256>;
+    case 2: return avg ? k_slab_couette<2, true, 256> : k_slab_couette<2, false, 256>;
+    case 4: return avg ? k_slab_couette<4, true, 256> : k_slab_couette<2, false, 512>;
+    case 8: return avg ? k_slab_couette<8, true, 256> : k_slab_couette<4, false, 512>;
     default: return nullptr;
     }
 }
+int slab_threads(int ppt, bool avg = false) { return ppt >= 4 && !avg ? 512 : 256; }
 
 // Largest per-slab occupancy for a given number of cells per slab.
 int32_t max_slab_particles(const std::vector<int32_t> &n1, int spc) {
@@ -1040,7 +1230,7 @@ extern "C" int mz_slab_occupancy(int32_t particles_per_thread, int32_t *blocks_p
     SlabKernel fn = slab_kernel(particles_per_thread);
     MZ_CHECK(fn != nullptr, "slab occupancy: particles per thread must be 1, 2, 4 or 8");
     int per_cu = 0;
-    MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)fn, SLAB_THREADS, 0));
+    MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)fn, slab_threads(particles_per_thread), 0));
     hipFuncAttributes fa;
     MZ_HIP(hipFuncGetAttributes(&fa, (const void *)fn));
     if (blocks_per_cu) *blocks_per_cu = per_cu;
@@ -1074,7 +1264,7 @@ static int slab_pick_shape(mz_store *h, bool avg, MzSlabShapeCache &out) {
         if (R < h->slab_min_ppt) continue;
         SlabKernel fn = slab_kernel(R, avg);
         int per_cu = 0;
-        MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)fn, SLAB_THREADS, 0));
+        MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)fn, slab_threads(R, avg), 0));
         const int max_wg = per_cu * n_cu;
         if (max_wg <= 0) continue;
         int spc = h->slab_spc ? h->slab_spc : (nc + max_wg - 1) / max_wg;
@@ -1082,7 +1272,7 @@ static int slab_pick_shape(mz_store *h, bool avg, MzSlabShapeCache &out) {
         const int n_slabs = (nc + spc - 1) / spc;
         const int spx = (n_slabs + 7) / 8;
         if (8 * spx > max_wg) continue;
-        const int64_t P = (int64_t)R * SLAB_THREADS;
+        const int64_t P = (int64_t)R * 256;
         // room for the slab's occupancy to fluctuate (25% plus four standard
         // deviations of a Poisson count); a slab that still overflows aborts
         // the launch and the steps run on the step graph
@@ -1197,7 +1387,7 @@ int mz_couette_slab(mz_store *h, int32_t n_steps, uint64_t step0, double dt, con
     if (mz_other_stores_busy(h)) MZ_HIP(hipDeviceSynchronize());
     {
         MzTimed tm(h, "slab", n_steps);
-        MZ_HIP(hipLaunchKernel(sh.fn, dim3(sh.grid), dim3(SLAB_THREADS), args, 0, h->stream));
+        MZ_HIP(hipLaunchKernel(sh.fn, dim3(sh.grid), dim3(slab_threads(sh.R, avg)), args, 0, h->stream));
     }
     hipLaunchKernelGGL(k_slab_report, dim3(1), dim3(64), 0, h->stream, abort_flag, h->h_report);
     MZ_HIP(hipGetLastError());
