@@ -250,6 +250,8 @@ __device__ inline double mz_readlane_d(double v, int l) {
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
+// value of v in lane l (l may differ between lanes)
+__device__ inline double mz_shfl_d(double v, int l) { return __shfl(v, l, 64); }
 __device__ inline uint64_t mz_lanemask_lt() {
     uint32_t lane = __lane_id();
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));

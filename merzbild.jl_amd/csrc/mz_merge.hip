@@ -32,7 +32,7 @@
 #define OCT_MAX_N 2048
 #define OCT_MAX_BINS 512
 #define OCT_LANE_NP 16        // bins of at most this many particles get a lane each for their moments
-#define OCT_BIG_BLOCKS 4096   // most 64-bin blocks whose maxima the device-memory path keeps in LDS
+#define OCT_LIST_LDS 143360   // bytes of LDS the device-memory path's list of bins may take
 
 struct OctArgs {
     MzSpView sp;
@@ -55,11 +55,16 @@ struct OctArgs {
     int32_t *big_pis, *big_psort, *big_bslot;
     double *big_stage;        // per workgroup: w, v0, v1, v2 of two tree-order buffers
     uint8_t *big_poct;
-    double *big_bkey;
+    double *big_list_mem;     // the lists of bins that may be refined, where LDS cannot hold them
     void *big_bins;
-    int32_t big_ncap, big_bcap;
-    int32_t big_blocks;       // 1: the 64-bin blocks' maxima are kept in dynamic LDS
+    int32_t big_ncap, big_bcap, big_hcap;
 };
+
+// the bytes of a list of hc bins that may be refined (hc a multiple of 64):
+// weight, bin, state
+__host__ __device__ inline size_t oct_list_bytes(int64_t hc) {
+    return (size_t)(hc * (sizeof(double) + sizeof(int32_t) + 1));
+}
 
 // A bin of the octree; IdxT holds particle counts and positions (int16_t in
 // LDS, where a cell holds at most OCT_MAX_N = 2048 particles, int32_t in
@@ -69,25 +74,26 @@ struct OctBinT {
     double w;
     double vmin[3], vmax[3];
     IdxT np, start, end;
-    int8_t depth, refine;
+    int8_t depth;
 };
 using OctBin = OctBinT<int16_t>;
 
-// The working arrays of one cell's merge: the particle order, its scatter
-// target (after the splits: per-bin output slots and draw offsets), each
-// particle's octant, the bins and the refine pick's keys.
+// The working arrays of one cell's merge: the particle order in two buffers
+// (a bin's particles lie in the buffer of its depth's parity), each particle's
+// octant, the bins, the refine pick's keys, and after the splits the bins'
+// output slots and draw offsets.
 template <class IdxT>
 struct OctWork {
-    IdxT *pis, *psort;
+    IdxT *pis, *psort;        // LDS path: the order of parity 0 and 1
     uint8_t *poct;
     OctBinT<IdxT> *bins;
-    double *bkey;
-    int32_t *bslot, *bdraw;
+    IdxT *bslot, *bdraw;
     int32_t bins_cap;
-    // per block of 64 bins: the largest key and its lowest bin (nullptr:
-    // the pick scans the keys themselves)
-    double *bmv;
-    int32_t *bmi;
+    // the bins that may be refined, in no order: weight, bin and state (0, or
+    // 1 + k when split ahead into pre[k])
+    double *hkey;
+    IdxT *hid;
+    uint8_t *hst;
     // device-memory path: the particles' ids and values in tree order, in the
     // buffer of the parity of their bin's depth (a split moves its bin's
     // particles to the other buffer, so a pass reads a contiguous segment)
@@ -98,17 +104,34 @@ struct OctWork {
 };
 
 
+// A split worked out ahead: its octants' weights and particle counts.
+struct OctSplit {
+    double w[8];
+    double vmin[3], vmax[3];  // the bin's bounds
+    int32_t cnt[8];
+    int32_t start, depth;
+    int32_t ent;              // the bin's entry in the list of bins that may be refined
+};
+// Splits held before the refine order takes them (at most 62): enough for the
+// waves of a workgroup to share, as LDS allows.
+#define OCT_PRE_LDS 24
+#define OCT_PRE_BIG 62
+
 // The small per-cell state of the split loop and the output scan, in LDS.
+template <int PRE>
 struct OctShared {
-    double red[4];
+    double red[8];
+    int32_t rid[8], rent[8];
     double vel_mid[3];
-    int32_t cnt8[9], start8[9];
-    double ndens8[9];
     int32_t Nbins_s, total_post_s, stop_s, defer_s;
-    int64_t wsc[4];
+    int64_t wsc[8];
     int32_t n_new_s, ticket_s;
-    double ckey[8];           // a split's children: key and bin id, by child
-    int32_t cbi[8];
+    int32_t n_ent;            // bins that may be refined
+    OctSplit pre[PRE];
+    uint64_t pre_free;        // free entries of pre
+    int32_t list[PRE], n_list;              // entries of the bins to split next
+    unsigned long long dropped;             // largest weight that found no place in the list, as bits
+    int32_t order[PRE], obin[PRE], onb[PRE], orp[PRE], oent[PRE];   // the splits taken, in order
 };
 
 // orders LDS accesses among the lanes of one wave (a barrier for code that a
@@ -142,7 +165,7 @@ __device__ __forceinline__ void oct_ld(const OctArgs &A, const OctWork<IdxT> &W,
     if constexpr (BIG) {
         w = oct_stg(W, par, 0)[i]; a0 = oct_stg(W, par, 1)[i]; a1 = oct_stg(W, par, 2)[i]; a2 = oct_stg(W, par, 3)[i];
     } else {
-        const int64_t p = oct_slot(pis[i], s1, n1, s2);
+        const int64_t p = oct_slot((par ? W.psort : W.pis)[i], s1, n1, s2);
         w = A.sp.w[p]; a0 = A.sp.v0[p]; a1 = A.sp.v1[p]; a2 = A.sp.v2[p];
     }
 }
@@ -151,7 +174,7 @@ __device__ __forceinline__ void oct_ld(const OctArgs &A, const OctWork<IdxT> &W,
 template <class IdxT, bool BIG>
 __device__ __forceinline__ int oct_id(const OctWork<IdxT> &W, const IdxT *pis, int par, int i) {
     if constexpr (BIG) return oct_sid(W, par)[i];
-    else return pis[i];
+    else return (par ? W.psort : W.pis)[i];
 }
 
 __device__ inline double blk_min(double v, double *red) {
@@ -159,7 +182,8 @@ __device__ inline double blk_min(double v, double *red) {
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    double r = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
+    double r = red[0];
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmin(r, red[k]);
     __syncthreads();
     return r;
 }
@@ -168,7 +192,8 @@ __device__ inline double blk_max(double v, double *red) {
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    double r = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    double r = red[0];
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, red[k]);
     __syncthreads();
     return r;
 }
@@ -262,8 +287,13 @@ __device__ inline void oct_emit(const OctArgs &A, int c, int32_t draw, int slot,
     MzStream st = mz_stream((uint64_t)c);
     st.k = 6 * (uint64_t)draw;
     double dv[3], dx[3];
-    for (int d = 0; d < 3; ++d) dv[d] = mz_rand(A.rp, st) < 0.5 ? -1.0 : 1.0;
-    for (int d = 0; d < 3; ++d) dx[d] = mz_rand(A.rp, st) < 0.5 ? -1.0 : 1.0;
+    uint32_t neg = 0;   // bit d: draw d below 1/2 (one copy of the draw's code)
+#pragma unroll 1
+    for (int d = 0; d < 6; ++d) neg |= (mz_rand(A.rp, st) < 0.5 ? 1u : 0u) << d;
+    for (int d = 0; d < 3; ++d) {
+        dv[d] = (neg >> d) & 1 ? -1.0 : 1.0;
+        dx[d] = (neg >> (3 + d)) & 1 ? -1.0 : 1.0;
+    }
     const double w1 = 0.5 * Wb;
     for (int k = 0; k < 2; ++k) {
         const double sg = k == 0 ? 1.0 : -1.0;
@@ -293,21 +323,15 @@ __device__ inline void oct_defer(const OctArgs &A, int c, int32_t N) {
     }
 }
 
-template <class IdxT, int NW, bool BIG>
+template <class IdxT, int NW, bool BIG, int PRE>
 __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, const int32_t N,
-                                               const int32_t target_np, const OctWork<IdxT> &W, OctShared &S) {
+                                               const int32_t target_np, const OctWork<IdxT> &W, OctShared<PRE> &S) {
     IdxT *const pis = W.pis;
     IdxT *const psort = W.psort;
     uint8_t *const poct = W.poct;
     OctBinT<IdxT> *const bins = W.bins;
-    // the refine pick's keys: bins[b].w when bin b may be refined, else -1
-    // (contiguous, so the pick's scan reads without bank conflicts)
-    double *const bkey = W.bkey;
     double *const red = S.red;
     double *const vel_mid = S.vel_mid;
-    int32_t *const cnt8 = S.cnt8;
-    int32_t *const start8 = S.start8;
-    double *const ndens8 = S.ndens8;
     int32_t &Nbins_s = S.Nbins_s;
     int32_t &total_post_s = S.total_post_s;
     int32_t &stop_s = S.stop_s;
@@ -345,349 +369,468 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         b.w = 1e50;
         for (int d = 0; d < 3; ++d) { b.vmin[d] = mn[d]; b.vmax[d] = mx[d]; }
         b.np = N; b.start = 0; b.end = N - 1; b.depth = 0;
-        b.refine = (N > 2) && (A.max_depth > 0);
-        bkey[0] = b.refine ? b.w : -1.0;
-        if (W.bmv) {
-            W.bmv[0] = bkey[0];
-            W.bmi[0] = 0;
-        }
+        S.n_ent = N > 2 && A.max_depth > 0 ? 1 : 0;
+        W.hkey[0] = b.w;
+        W.hid[0] = 0;
+        W.hst[0] = 0;
         Nbins_s = 1;
         total_post_s = N >= 2 ? 2 : N;
         for (int d = 0; d < 3; ++d) vel_mid[d] = 0.0;
         stop_s = 0;
         S.defer_s = 0;
+        S.pre_free = (1ull << PRE) - 1;
     }
     __syncthreads();
 
-    // compute_octree! (merging_octree_N2.jl:998-1039).  Each split depends on
-    // the one before, so the loop runs on wave 0 alone, where a barrier is a
-    // wave-level fence; the other waves wait at the block barrier after it.
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        for (;;) {
-            // refine pick: first maximum of w over refinable bins (lowest id on ties)
-            double bw = -1.0;
-            int bid = -1;
-            if (W.bmv) {
-                // the blocks' maxima (each the lowest bin of its block's maximum)
-                for (int k = lane; k < (Nbins_s + 63) >> 6; k += 64) {
-                    const double kb = W.bmv[k];
-                    if (kb > bw) { bw = kb; bid = W.bmi[k]; }
+    // compute_octree! (merging_octree_N2.jl:998-1039): the heaviest bin that
+    // may be refined (the lowest id on ties) is split until the target is met.
+    // What a split makes of a bin does not depend on the splits of other bins,
+    // and no child is heavier than its parent, so the order's weights only
+    // fall.  The bins are therefore split ahead of the order, in rounds:
+    //   - all waves find the heaviest bin, and list it and the other bins of
+    //     at least a share f of its weight that are not split yet;
+    //   - all waves split the listed bins, one bin a wave at a time, into
+    //     entries of S.pre;
+    //   - wave 0 takes from S.pre, in the order, every split whose bin is
+    //     heavier than all bins not split and than the children that the
+    //     splits before it bring, as far as the target goes, all at once (bin
+    //     ids, list entries and totals from prefix sums over them).
+    // A split that the order never reaches is left unused (a bin's particles
+    // stay in the buffer of its depth's parity).  The mean split carries the
+    // middle velocity from one split to the next, so there each is worked out
+    // as its turn comes.
+    //
+    // What bounds it: the latency of one small bin's split (about 3.3 us of
+    // dependent loads, ballots and ordered sums) over the waves.  Measured
+    // against one wave splitting each bin as it is picked: 1,024 cells of 20 to
+    // 30,000 particles, about 120 merged (the largest in 2,194 splits, 66 rounds,
+    // 3.6 ms), 14.9 -> 3.5 ms a call with eight waves a cell for one; 1,850
+    // boxes of 1,300 particles to 1,000 (89 splits, 16 rounds) 1.02 -> 0.72 ms.
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    // split_bin! (merging_octree_N2.jl:503-633) of entry e's bin up to its
+    // children: the octants' weights and counts into pre[slot], the particles
+    // in octant order into the other buffer; one wave
+    auto split = [&](const int e, const int slot) {
+        const int b = W.hid[e];
+        const int bs = bins[b].start, be = bins[b].end;
+        const int par = bins[b].depth & 1;
+        if (A.bounds_mode == 2) {
+            double bmn[3], bmx[3];
+            for (int d = 0; d < 3; ++d) {
+                double lo = 9299792458.0, hi = -9299792458.0;
+                for (int i = bs + lane; i <= be; i += 64) {
+                    double w, x[3];
+                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, x[0], x[1], x[2]);
+                    lo = fmin(lo, x[d]);
+                    hi = fmax(hi, x[d]);
                 }
-            } else {
-                for (int b = lane; b < Nbins_s; b += 64) {
-                    const double kb = bkey[b];
-                    if (kb > bw) { bw = kb; bid = b; }
-                }
+                bmn[d] = mz_wave_min(lo);
+                bmx[d] = mz_wave_max(hi);
             }
-            // the largest key, then the lowest bin holding it (two wave reductions)
-            {
-                const double mw = mz_wave_max(bw);
-                bid = mw > -1.0 ? mz_wave_min_i32(bw == mw ? bid : 0x7FFFFFFF) : -1;
-            }
-            if (bid < 0 || total_post_s + 14 > target_np) break;
-            // split_bin! (merging_octree_N2.jl:503-633)
-            const int b = bid;
-            // the keys of b's block, loaded with bin b: the block's maximum is
-            // rebuilt from them after the split
-            double k0key = -2.0;
-            if (W.bmv && (b & ~63) + lane < Nbins_s) k0key = bkey[(b & ~63) + lane];
-            const int bs = bins[b].start, be = bins[b].end;
-            const int depth = bins[b].depth;
-            const int par = depth & 1;
-            if (A.bounds_mode == 2) {
-                double bmn[3], bmx[3];
-                for (int d = 0; d < 3; ++d) {
-                    const double *vv;
-                    if constexpr (BIG) vv = d == 0 ? oct_stg(W, par, 1) : (d == 1 ? oct_stg(W, par, 2) : oct_stg(W, par, 3));
-                    else vv = d == 0 ? A.sp.v0 : (d == 1 ? A.sp.v1 : A.sp.v2);
-                    double lo = 9299792458.0, hi = -9299792458.0;
-                    for (int i = bs + lane; i <= be; i += 64) {
-                        double x;
-                        if constexpr (BIG) x = vv[i];
-                        else x = vv[oct_slot(pis[i], s1, n1, s2)];
-                        lo = fmin(lo, x);
-                        hi = fmax(hi, x);
-                    }
-                    bmn[d] = mz_wave_min(lo);
-                    bmx[d] = mz_wave_max(hi);
-                }
-                if (lane == 0 && be >= bs)
-                    for (int d = 0; d < 3; ++d) { bins[b].vmin[d] = bmn[d]; bins[b].vmax[d] = bmx[d]; }
-                oct_wave_sync();
-            }
-            // the parent's bounds, read once by every lane
-            double pmin[3], pmax[3];
-            for (int d = 0; d < 3; ++d) { pmin[d] = bins[b].vmin[d]; pmax[d] = bins[b].vmax[d]; }
+            if (lane == 0 && be >= bs)
+                for (int d = 0; d < 3; ++d) { bins[b].vmin[d] = bmn[d]; bins[b].vmax[d] = bmx[d]; }
+            oct_wave_sync();
+        }
+        if (lane < 3) {
+            S.pre[slot].vmin[lane] = bins[b].vmin[lane];
+            S.pre[slot].vmax[lane] = bins[b].vmax[lane];
+        }
+        if (lane == 0) {
+            S.pre[slot].start = bs;
+            S.pre[slot].depth = bins[b].depth;
+            S.pre[slot].ent = e;
+        }
+        double mid0, mid1, mid2;
+        if (A.split == 1) {
+            mid0 = 0.5 * (bins[b].vmin[0] + bins[b].vmax[0]);
+            mid1 = 0.5 * (bins[b].vmin[1] + bins[b].vmax[1]);
+            mid2 = 0.5 * (bins[b].vmin[2] + bins[b].vmax[2]);
+        } else {
             if (lane == 0) {
-                if (A.split == 1) {
-                    for (int d = 0; d < 3; ++d) vel_mid[d] = 0.5 * (pmin[d] + pmax[d]);
-                } else {
-                    // compute_v_mean! keeps the previous middle velocity in the sum
-                    double nt = 0.0;
-                    for (int i = bs; i <= be; ++i) {
-                        double w, a0, a1, a2;
-                        oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, a0, a1, a2);
-                        nt += w;
-                        vel_mid[0] = vel_mid[0] + w * a0;
-                        vel_mid[1] = vel_mid[1] + w * a1;
-                        vel_mid[2] = vel_mid[2] + w * a2;
-                    }
-                    for (int d = 0; d < 3; ++d) vel_mid[d] = vel_mid[d] / nt;
+                // compute_v_mean! keeps the previous middle velocity in the sum
+                double nt = 0.0;
+                for (int i = bs; i <= be; ++i) {
+                    double w, a0, a1, a2;
+                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, a0, a1, a2);
+                    nt += w;
+                    vel_mid[0] = vel_mid[0] + w * a0;
+                    vel_mid[1] = vel_mid[1] + w * a1;
+                    vel_mid[2] = vel_mid[2] + w * a2;
                 }
-                for (int o = 0; o < 9; ++o) { cnt8[o] = 0; ndens8[o] = 0.0; }
+                for (int d = 0; d < 3; ++d) vel_mid[d] = vel_mid[d] / nt;
             }
             oct_wave_sync();
-            // each particle's octant (compute_octant, :304-316: strict >), the
-            // octants' counts from one ballot per octant and chunk of 64, and the
-            // octants' weights in the reference's accumulation order (the bin's
-            // particles in order, each weight added to its octant's sum: the
-            // chunk's lanes are walked in order, lane o keeping octant o's sum)
-            int cq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-            double sw = 0.0;
-            const double mid0 = vel_mid[0], mid1 = vel_mid[1], mid2 = vel_mid[2];
-            // the next chunk's particle loads are issued before this chunk's
-            // ballots and sums, so their latency overlaps that work
-            // A bin of at most 64 particles is one chunk: its ids and octants
-            // stay in registers and the scatter writes pis directly.
-            const bool one = be - bs < 64;
-            double nw = 0.0, nv0 = 0.0, nv1 = 0.0, nv2 = 0.0;
-            IdxT pi1 = 0;
-            if (bs + lane <= be) {
-                pi1 = oct_id<IdxT, BIG>(W, pis, par, bs + lane);
-                oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, nw, nv0, nv1, nv2);
+            mid0 = vel_mid[0]; mid1 = vel_mid[1]; mid2 = vel_mid[2];
+        }
+        // each particle's octant (compute_octant, :304-316: strict >), the
+        // octants' counts from one ballot per octant and chunk of 64, and the
+        // octants' weights in the reference's accumulation order (the bin's
+        // particles in order, each weight added to its octant's sum: the
+        // chunk's lanes are walked in order, lane o keeping octant o's sum)
+        int cq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        double sw = 0.0;
+        // the next chunk's particle loads are issued before this chunk's
+        // ballots and sums, so their latency overlaps that work
+        // A bin of at most 64 particles is one chunk: its ids and octants
+        // stay in registers.
+        const bool one = be - bs < 64;
+        double nw = 0.0, nv0 = 0.0, nv1 = 0.0, nv2 = 0.0;
+        IdxT pi1 = 0;
+        if (bs + lane <= be) {
+            pi1 = oct_id<IdxT, BIG>(W, pis, par, bs + lane);
+            oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, nw, nv0, nv1, nv2);
+        }
+        // the next chunk's ids, loaded a chunk ahead of its values (the
+        // staged values need no ids)
+        IdxT pin = 0;
+        if (!BIG && bs + 64 + lane <= be) pin = oct_id<IdxT, BIG>(W, pis, par, bs + 64 + lane);
+        int o1 = 0;
+        for (int i0 = bs; i0 <= be; i0 += 64) {
+            const int i = i0 + lane;
+            const double wi = nw, c0 = nv0, c1 = nv1, c2 = nv2;
+            if (i + 64 <= be) {
+                if constexpr (BIG) {
+                    nw = oct_stg(W, par, 0)[i + 64]; nv0 = oct_stg(W, par, 1)[i + 64];
+                    nv1 = oct_stg(W, par, 2)[i + 64]; nv2 = oct_stg(W, par, 3)[i + 64];
+                } else {
+                    const int64_t p = oct_slot(pin, s1, n1, s2);
+                    nw = A.sp.w[p]; nv0 = A.sp.v0[p]; nv1 = A.sp.v1[p]; nv2 = A.sp.v2[p];
+                }
             }
-            // the next chunk's ids, loaded a chunk ahead of its values (the
-            // staged values need no ids)
-            IdxT pin = 0;
-            if (!BIG && bs + 64 + lane <= be) pin = pis[bs + 64 + lane];
-            int o1 = 0;
+            if (!BIG && i + 128 <= be) pin = oct_id<IdxT, BIG>(W, pis, par, i + 128);
+            int o = 0;
+            if (i <= be) {
+                o = 1;
+                if (c0 > mid0) o += 1;
+                if (c1 > mid1) o += 2;
+                if (c2 > mid2) o += 4;
+                if (!one) poct[i] = (uint8_t)o;
+            }
+            o1 = o;
+            uint64_t mq = 0;   // lane q: the chunk's lanes in octant q
+#pragma unroll
+            for (int q = 1; q <= 8; ++q) {
+                const uint64_t m = __ballot(o == q);
+                cq[q] += __popcll(m);
+                if (lane == q) mq = m;
+            }
+            // lane q adds its octant's weights in lane order, four at a
+            // time, each fetched from its lane with ds_bpermute
+            const int wlo = __double2loint(wi), whi = __double2hiint(wi);
+            while (__ballot(mq != 0)) {
+                int src[4];
+                bool has[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    has[u] = mq != 0;
+                    src[u] = has[u] ? (int)__builtin_ctzll(mq) : 0;
+                    mq &= mq - 1;
+                }
+                double wv4[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    wv4[u] = __hiloint2double(__builtin_amdgcn_ds_bpermute(src[u] << 2, whi),
+                                              __builtin_amdgcn_ds_bpermute(src[u] << 2, wlo));
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (has[u]) sw += wv4[u];
+            }
+        }
+        int sq[9];
+        sq[0] = bs;
+#pragma unroll
+        for (int q = 1; q <= 8; ++q) sq[q] = q == 1 ? bs : sq[q - 1] + cq[q - 1];
+        if (lane >= 1 && lane <= 8) S.pre[slot].w[lane - 1] = sw;
+#pragma unroll
+        for (int q = 1; q <= 8; ++q)
+            if (lane == q) S.pre[slot].cnt[q - 1] = cq[q];
+        // Scatter by octant.  The reference walks the bin forward and fills
+        // each octant from its end (merging_octree_N2.jl:621-626), so every
+        // child holds its particles in reverse parent order: a particle's
+        // place is its octant's end less the octant's particles before it
+        // (earlier chunks, then earlier lanes of its chunk).
+        const uint64_t lt = mz_lanemask_lt();
+        const int oq = par ^ 1;
+        IdxT *const dsto = oq ? psort : pis;   // LDS path
+        if (one) {
+            int dst = 0;
+#pragma unroll
+            for (int q = 1; q <= 8; ++q) {
+                const uint64_t m = __ballot(o1 == q);
+                if (o1 == q) dst = sq[q] + cq[q] - 1 - __popcll(m & lt);
+            }
+            if (bs + lane <= be) {
+                if constexpr (BIG) {
+                    // the values are still those of the bin's one chunk
+                    oct_sid(W, oq)[dst] = pi1;
+                    oct_stg(W, oq, 0)[dst] = nw; oct_stg(W, oq, 1)[dst] = nv0; oct_stg(W, oq, 2)[dst] = nv1; oct_stg(W, oq, 3)[dst] = nv2;
+                } else {
+                    dsto[dst] = pi1;
+                }
+            }
+        } else {
+            int rq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+            // each chunk's octants and ids are loaded a chunk ahead
+            int on = bs + lane <= be ? poct[bs + lane] : 0;
+            IdxT pn = bs + lane <= be ? oct_id<IdxT, BIG>(W, pis, par, bs + lane) : (IdxT)0;
+            double qw = 0.0, qa = 0.0, qb = 0.0, qc = 0.0;
+            if (BIG && bs + lane <= be) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, qw, qa, qb, qc);
             for (int i0 = bs; i0 <= be; i0 += 64) {
                 const int i = i0 + lane;
-                const double wi = nw, c0 = nv0, c1 = nv1, c2 = nv2;
-                if (i + 64 <= be) {
-                    if constexpr (BIG) {
-                        nw = oct_stg(W, par, 0)[i + 64]; nv0 = oct_stg(W, par, 1)[i + 64];
-                        nv1 = oct_stg(W, par, 2)[i + 64]; nv2 = oct_stg(W, par, 3)[i + 64];
-                    } else {
-                        const int64_t p = oct_slot(pin, s1, n1, s2);
-                        nw = A.sp.w[p]; nv0 = A.sp.v0[p]; nv1 = A.sp.v1[p]; nv2 = A.sp.v2[p];
-                    }
-                }
-                if (!BIG && i + 128 <= be) pin = pis[i + 128];
-                int o = 0;
-                if (i <= be) {
-                    o = 1;
-                    if (c0 > mid0) o += 1;
-                    if (c1 > mid1) o += 2;
-                    if (c2 > mid2) o += 4;
-                    if (!one) poct[i - bs] = (uint8_t)o;
-                }
-                o1 = o;
-                uint64_t mq = 0;   // lane q: the chunk's lanes in octant q
-#pragma unroll
-                for (int q = 1; q <= 8; ++q) {
-                    const uint64_t m = __ballot(o == q);
-                    cq[q] += __popcll(m);
-                    if (lane == q) mq = m;
-                }
-                // lane q adds its octant's weights in lane order, four at a
-                // time, each fetched from its lane with ds_bpermute
-                const int wlo = __double2loint(wi), whi = __double2hiint(wi);
-                while (__ballot(mq != 0)) {
-                    int src[4];
-                    bool has[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        has[u] = mq != 0;
-                        src[u] = has[u] ? (int)__builtin_ctzll(mq) : 0;
-                        mq &= mq - 1;
-                    }
-                    double wv[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        wv[u] = __hiloint2double(__builtin_amdgcn_ds_bpermute(src[u] << 2, whi),
-                                                 __builtin_amdgcn_ds_bpermute(src[u] << 2, wlo));
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (has[u]) sw += wv[u];
-                }
-            }
-            if (lane >= 1 && lane <= 8) ndens8[lane] = sw;
-            int sq[9];
-            sq[0] = bs;
-#pragma unroll
-            for (int q = 1; q <= 8; ++q) sq[q] = q == 1 ? bs : sq[q - 1] + cq[q - 1];
-#pragma unroll
-            for (int q = 1; q <= 8; ++q)
-                if (lane == q) { cnt8[q] = cq[q]; start8[q] = sq[q]; }
-            // Scatter by octant.  The reference walks the bin forward and fills
-            // each octant from its end (merging_octree_N2.jl:621-626), so every
-            // child holds its particles in reverse parent order: a particle's
-            // place is its octant's end less the octant's particles before it
-            // (earlier chunks, then earlier lanes of its chunk).
-            if (one) {
-                const uint64_t lt = mz_lanemask_lt();
+                const bool valid = i <= be;
+                const int o = on;
+                const IdxT pv = pn;
+                const double vw = qw, va = qa, vb = qb, vc = qc;
+                const bool vn = i + 64 <= be;
+                on = vn ? poct[i + 64] : 0;
+                pn = vn ? oct_id<IdxT, BIG>(W, pis, par, i + 64) : (IdxT)0;
+                if (BIG && vn) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i + 64, qw, qa, qb, qc);
                 int dst = 0;
 #pragma unroll
                 for (int q = 1; q <= 8; ++q) {
-                    const uint64_t m = __ballot(o1 == q);
-                    if (o1 == q) dst = sq[q] + cq[q] - 1 - __popcll(m & lt);
+                    const uint64_t m = __ballot(o == q);
+                    if (o == q) dst = sq[q] + cq[q] - 1 - (rq[q] + __popcll(m & lt));
+                    rq[q] += __popcll(m);
                 }
-                if (bs + lane <= be) {
+                if (valid) {
                     if constexpr (BIG) {
-                        // the values are still those of the bin's one chunk
-                        const int q = par ^ 1;
-                        oct_sid(W, q)[dst] = pi1;
-                        oct_stg(W, q, 0)[dst] = nw; oct_stg(W, q, 1)[dst] = nv0; oct_stg(W, q, 2)[dst] = nv1; oct_stg(W, q, 3)[dst] = nv2;
+                        oct_sid(W, oq)[dst] = pv;
+                        oct_stg(W, oq, 0)[dst] = vw; oct_stg(W, oq, 1)[dst] = va; oct_stg(W, oq, 2)[dst] = vb; oct_stg(W, oq, 3)[dst] = vc;
                     } else {
-                        pis[dst] = pi1;
-                    }
-                }
-                oct_wave_sync();
-            } else {
-                const uint64_t lt = mz_lanemask_lt();
-                int rq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-                // each chunk's octants and ids are loaded a chunk ahead
-                int on = bs + lane <= be ? poct[lane] : 0;
-                IdxT pn = bs + lane <= be ? oct_id<IdxT, BIG>(W, pis, par, bs + lane) : (IdxT)0;
-                double qw = 0.0, qa = 0.0, qb = 0.0, qc = 0.0;
-                if (BIG && bs + lane <= be) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, qw, qa, qb, qc);
-                for (int i0 = bs; i0 <= be; i0 += 64) {
-                    const int i = i0 + lane;
-                    const bool valid = i <= be;
-                    const int o = on;
-                    const IdxT pv = pn;
-                    const double vw = qw, va = qa, vb = qb, vc = qc;
-                    const bool vn = i + 64 <= be;
-                    on = vn ? poct[i + 64 - bs] : 0;
-                    pn = vn ? oct_id<IdxT, BIG>(W, pis, par, i + 64) : (IdxT)0;
-                    if (BIG && vn) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i + 64, qw, qa, qb, qc);
-                    int dst = 0;
-#pragma unroll
-                    for (int q = 1; q <= 8; ++q) {
-                        const uint64_t m = __ballot(o == q);
-                        if (o == q) dst = sq[q] + cq[q] - 1 - (rq[q] + __popcll(m & lt));
-                        rq[q] += __popcll(m);
-                    }
-                    if (valid) {
-                        if constexpr (BIG) {
-                            const int q = par ^ 1;
-                            oct_sid(W, q)[dst] = pv;
-                            oct_stg(W, q, 0)[dst] = vw; oct_stg(W, q, 1)[dst] = va; oct_stg(W, q, 2)[dst] = vb; oct_stg(W, q, 3)[dst] = vc;
-                        } else {
-                            psort[dst] = pv;
-                        }
-                    }
-                }
-                oct_wave_sync();
-                if constexpr (!BIG) {
-                    for (int i = bs + lane; i <= be; i += 256) {
-                        IdxT t[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) t[u] = i + 64 * u <= be ? psort[i + 64 * u] : (IdxT)0;
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            if (i + 64 * u <= be) pis[i + 64 * u] = t[u];
-                    }
-                    oct_wave_sync();
-                }
-            }
-            // the children (split_bin!, :588-633), lane o for octant o: the
-            // k-th non-empty octant becomes bin b (k = 1) or Nb + k - 2
-            // (get_new_bin_id), its particles the octant's segment
-            const int Nb = Nbins_s;
-            // a new bin's key and id on its octant's lane (for the blocks' maxima)
-            double nkey = -2.0;
-            int nbi = 0x7FFFFFFF;
-            int n_ne = 0;
-            {
-                const int o = lane;
-                const bool ne = o >= 1 && o <= 8 && cnt8[o] > 0;
-                const uint64_t m = __ballot(ne);
-                n_ne = __popcll(m);
-                int contrib = 0;
-                oct_wave_sync();   // every lane has read bin b before child 1 overwrites it
-                if (ne) {
-                    const int k = __popcll(m & mz_lanemask_lt()) + 1;
-                    const int bi = k == 1 ? b : Nb + k - 2;
-                    if (bi < W.bins_cap) {
-                        OctBinT<IdxT> &nb = bins[bi];
-                        nb.start = start8[o];
-                        nb.end = start8[o] + cnt8[o] - 1;
-                        if (A.bounds_mode == 1) {   // bin_bounds_inherit! (:341-367)
-                            const int sx = (o - 1) & 1, sy = ((o - 1) >> 1) & 1, sz = ((o - 1) >> 2) & 1;
-                            nb.vmin[0] = sx ? vel_mid[0] : pmin[0]; nb.vmax[0] = sx ? pmax[0] : vel_mid[0];
-                            nb.vmin[1] = sy ? vel_mid[1] : pmin[1]; nb.vmax[1] = sy ? pmax[1] : vel_mid[1];
-                            nb.vmin[2] = sz ? vel_mid[2] : pmin[2]; nb.vmax[2] = sz ? pmax[2] : vel_mid[2];
-                        }
-                        nb.np = cnt8[o];
-                        nb.w = ndens8[o];
-                        nb.depth = depth + 1;
-                        nb.refine = (cnt8[o] > 2) && (depth + 1 < A.max_depth);
-                        const double key = nb.refine ? nb.w : -1.0;
-                        bkey[bi] = key;
-                        S.ckey[k - 1] = key;
-                        S.cbi[k - 1] = bi;
-                        if (k > 1) { nkey = key; nbi = bi; }
-                    }
-                    contrib = cnt8[o] >= 2 ? 2 : cnt8[o];
-                }
-                const int added = mz_wave_sum_i(contrib);
-                if (lane == 0) {
-                    total_post_s += added - 2;
-                    Nbins_s = Nb + n_ne - 1;
-                    if (Nbins_s + 7 > A.max_Nbins) {
-                        stop_s = 1;
-                    } else if (Nbins_s + 7 > max_bins) {
-                        // the arrays' bin budget is below the caller's max_Nbins:
-                        // the cell goes to the device-memory path (or fails)
-                        stop_s = 1;
-                        S.defer_s = 1;
+                        dsto[dst] = pv;
                     }
                 }
             }
-            oct_wave_sync();
-            if (W.bmv) {
-                // the keys of bin b and of the new bins Nb .. Nbins - 1 changed:
-                // their blocks' maxima again (at most three blocks)
-                const int nb_now = Nbins_s;
-                const int k0 = b >> 6;
-                // b's block from its keys as loaded, the children's keys put
-                // in (b's key fell; new bins may lie in the block)
-                {
-                    const int i = (k0 << 6) + lane;
-                    double v = i < nb_now ? k0key : -2.0;
-                    for (int j = 0; j < n_ne; ++j)
-                        if (S.cbi[j] == i) v = S.ckey[j];
-                    const double mv = mz_wave_max(v);
-                    const int vi = mz_wave_min_i32(i < nb_now && v == mv ? i : 0x7FFFFFFF);
-                    v = mv;
-                    if (lane == 0) {
-                        W.bmv[k0] = v;
-                        W.bmi[k0] = vi;
-                    }
-                }
-                // the other blocks that gained new bins Nb .. nb_now - 1: their
-                // old maximum against the new keys (an old bin wins a tie, its id
-                // being lower)
-                if (nb_now > Nb) {
-                    for (int k = Nb >> 6; k <= (nb_now - 1) >> 6; ++k) {
-                        if (k == k0) continue;
-                        const bool in = (nbi >> 6) == k && nbi != 0x7FFFFFFF;
-                        const double mv = mz_wave_max(in ? nkey : -2.0);
-                        const int mi = mz_wave_min_i32(in && nkey == mv ? nbi : 0x7FFFFFFF);
-                        const bool had = (k << 6) < Nb;
-                        if (lane == 0 && (!had || mv > W.bmv[k])) {
-                            W.bmv[k] = mv;
-                            W.bmi[k] = mi;
-                        }
-                    }
-                }
-                oct_wave_sync();
-            }
-            if (stop_s) break;
         }
+        if (lane == 0) W.hst[e] = (uint8_t)(1 + slot);
+        oct_wave_sync();
+    };
+
+    // Takes splits from S.pre in the refine order (split_bin!, :588-633): the
+    // bin of entry e_pick first, then the others heavier than `bound` (or as
+    // heavy, with `with_bound`), as far as each is heavier than the children
+    // before it and the target and the bins allow; wave 0.  The k-th non-empty
+    // octant of a split becomes its bin (k = 1) or the next new bin
+    // (get_new_bin_id), its particles the octant's segment.
+    auto take = [&](const int e_pick, const double bound, const bool with_bound) {
+        const bool used = lane < PRE && !((S.pre_free >> lane) & 1);
+        double w = 0.0, cmax = -1.0;   // the bin's weight, its heaviest child that may be refined
+        int id = 0, ent = 0, n_ne = 0, n_ref = 0, added = 0;
+        if (used) {
+            const OctSplit &P = S.pre[lane];
+            ent = P.ent;
+            w = W.hkey[ent];
+            id = W.hid[ent];
+            const bool deeper = P.depth + 1 < A.max_depth;
+#pragma unroll
+            for (int o = 0; o < 8; ++o) {
+                const int cnt = P.cnt[o];
+                n_ne += cnt > 0;
+                added += cnt >= 2 ? 2 : cnt;
+                if (cnt > 2 && deeper) {
+                    ++n_ref;
+                    cmax = fmax(cmax, P.w[o]);
+                }
+            }
+        }
+        const bool first = used && ent == e_pick;
+        const bool elig = used && (first || w > bound || (with_bound && w == bound));
+        const uint64_t em = __ballot(elig);
+        int rank = 0;
+        for (uint64_t m = em; m; m &= m - 1) {
+            const int j = __builtin_ctzll(m);
+            const double wj = mz_readlane_d(w, j);
+            const int idj = __builtin_amdgcn_readlane(id, j);
+            rank += wj > w || (wj == w && idj < id);
+        }
+        if (elig) S.order[rank] = lane;
+        oct_wave_sync();
+        // lane r: the r-th of the order
+        const int K0 = __popcll(em);
+        const int src = lane < K0 ? S.order[lane] : 0;
+        const double wr = mz_shfl_d(w, src), cr = mz_shfl_d(cmax, src);
+        // every lane takes part in the exchanges: a lane that does not would
+        // hand over nothing
+        int ne_r = __shfl(n_ne, src, 64) - 1, ref_r = __shfl(n_ref, src, 64), add_r = __shfl(added, src, 64) - 2;
+        const int id_r = __shfl(id, src, 64), ent_r = __shfl(ent, src, 64);
+        if (lane >= K0) ne_r = ref_r = add_r = 0;
+        int sn = ne_r, sa = add_r, sr = ref_r;
+        double sc = lane < K0 ? cr : -1.0;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y0 = __shfl_up(sn, o, 64), y1 = __shfl_up(sa, o, 64), y2 = __shfl_up(sr, o, 64);
+            const double y3 = __shfl_up(sc, o, 64);
+            if (lane >= o) { sn += y0; sa += y1; sr += y2; sc = fmax(sc, y3); }
+        }
+        const double c_before = __shfl_up(sc, 1, 64);
+        const int Nb = Nbins_s, tot = total_post_s, n0 = S.n_ent;
+        const bool ok = lane < K0 && (lane == 0 || (wr > c_before && tot + sa - add_r + 14 <= target_np &&
+                                                    Nb + sn - ne_r + 7 <= max_bins));
+        const uint64_t okm = __ballot(ok);
+        const int K = okm == ~0ull ? 64 : __builtin_ctzll(~okm);   // the leading run; lane 0 always
+        if (lane < K) {
+            S.obin[lane] = id_r;
+            S.onb[lane] = Nb + sn - ne_r;
+            S.orp[lane] = sr - ref_r;
+            S.oent[lane] = ent_r;
+        }
+        const int new_bins = __shfl(sn, K - 1, 64), new_tot = __shfl(sa, K - 1, 64), C = __shfl(sr, K - 1, 64);
+        const uint64_t done = __ballot(elig && rank < K);
+        oct_wave_sync();
+        // the children, eight lanes a split
+        for (int i0 = 0; i0 < K * 8; i0 += 64) {
+            const int r = (i0 + lane) >> 3, o = lane & 7;
+            const bool in = r < K;
+            const OctSplit &P = S.pre[in ? S.order[r] : 0];
+            const int cnt = in ? P.cnt[o] : 0;
+            int start = cnt;   // exclusive scan over the octants
+#pragma unroll
+            for (int q = 1; q < 8; q <<= 1) {
+                const int y = __shfl_up(start, q, 8);
+                if (o >= q) start += y;
+            }
+            const bool ne = cnt > 0, ref = cnt > 2 && P.depth + 1 < A.max_depth;
+            const int sh = lane & 56;
+            const uint32_t low = (1u << o) - 1;
+            const uint32_t mn8 = (uint32_t)(__ballot(ne) >> sh) & 0xFF, mr8 = (uint32_t)(__ballot(ref) >> sh) & 0xFF;
+            if (ne) {
+                const int k = __popc(mn8 & low) + 1;
+                const int bi = k == 1 ? S.obin[r] : S.onb[r] + k - 2;
+                const double cw = P.w[o];
+                OctBinT<IdxT> &nb = bins[bi];
+                nb.start = P.start + start - cnt;
+                nb.end = P.start + start - 1;
+                if (A.bounds_mode == 1) {   // bin_bounds_inherit! (:341-367)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const double lo = P.vmin[d], hi = P.vmax[d];
+                        const double mid = A.split == 1 ? 0.5 * (lo + hi) : vel_mid[d];
+                        const bool up = (o >> d) & 1;
+                        nb.vmin[d] = up ? mid : lo;
+                        nb.vmax[d] = up ? hi : mid;
+                    }
+                }
+                nb.np = cnt;
+                nb.w = cw;
+                nb.depth = P.depth + 1;
+                if (ref) {
+                    // into the taken bins' entries, then at the end
+                    const int g = S.orp[r] + __popc(mr8 & low);
+                    const int e = g < K ? S.oent[g] : n0 + g - K;
+                    W.hkey[e] = cw;
+                    W.hid[e] = bi;
+                    W.hst[e] = 0;
+                }
+            }
+        }
+        oct_wave_sync();
+        // fewer children than bins taken: the last entries fill the gaps
+        const int H = K - C, n_new = n0 + C - K;
+        if (H > 0) {
+            const int gap = lane < H ? S.oent[C + lane] : 0x7FFFFFFF;
+            if (lane < H) W.hst[gap] = 255;
+            oct_wave_sync();
+            const bool keep = lane < H && W.hst[n_new + lane] != 255;
+            const uint64_t km = __ballot(keep), gm = __ballot(gap < n_new);
+            if (keep) S.obin[__popcll(km & mz_lanemask_lt())] = n_new + lane;
+            oct_wave_sync();
+            if (gap < n_new) {
+                const int from = S.obin[__popcll(gm & mz_lanemask_lt())];
+                W.hkey[gap] = W.hkey[from];
+                W.hid[gap] = W.hid[from];
+                const int st = W.hst[from];
+                W.hst[gap] = (uint8_t)st;
+                if (st) S.pre[st - 1].ent = gap;
+            }
+        }
+        if (lane == 0) {
+            S.n_ent = n_new;
+            S.pre_free |= done;
+            total_post_s = tot + new_tot;
+            const int nb_now = Nb + new_bins;
+            Nbins_s = nb_now;
+            if (nb_now + 7 > A.max_Nbins) {
+                stop_s = 1;
+            } else if (nb_now + 7 > max_bins) {
+                // the arrays' bin budget is below the caller's max_Nbins:
+                // the cell goes to the device-memory path (or fails)
+                stop_s = 1;
+                S.defer_s = 1;
+            }
+        }
+        oct_wave_sync();
+    };
+
+    double share = 0.5;   // the listed bins' least share of the heaviest's weight
+    for (;;) {
+        const int n_ent = S.n_ent;
+        if (n_ent == 0 || total_post_s + 14 > target_np) break;
+        // the heaviest bin, the lowest id on ties
+        double bw = -1.0;
+        int bid = 0x7FFFFFFF, ent = 0;
+        for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
+            const double kw = W.hkey[i];
+            const int ki = W.hid[i];
+            if (kw > bw || (kw == bw && ki < bid)) { bw = kw; bid = ki; ent = i; }
+        }
+        {
+            const double mw = mz_wave_max(bw);
+            const int mi = mz_wave_min_i32(bw == mw ? bid : 0x7FFFFFFF);
+            const uint64_t m = __ballot(bw == mw && bid == mi);
+            const int me = __builtin_amdgcn_readlane(ent, m ? __builtin_ctzll(m) : 0);
+            if (lane == 0) { red[wv] = mw; S.rid[wv] = mi; S.rent[wv] = me; }
+        }
+        __syncthreads();
+        double mw = red[0];
+        int mi = S.rid[0], e_pick = S.rent[0];
+#pragma unroll
+        for (int k = 1; k < NW; ++k)
+            if (red[k] > mw || (red[k] == mw && S.rid[k] < mi)) { mw = red[k]; mi = S.rid[k]; e_pick = S.rent[k]; }
+        if (!(mw > -1.0)) break;   // weights that do not compare
+        const bool fresh = W.hst[e_pick] == 0;   // not split yet
+        if (threadIdx.x == 0) {
+            S.list[0] = e_pick;
+            S.n_list = fresh ? 1 : 0;
+            S.dropped = 0;
+        }
+        __syncthreads();
+        // the list; one entry of pre is kept free for the next heaviest bin
+        const uint64_t free = S.pre_free;
+        const int room = A.split != 1 ? (fresh ? 1 : 0)
+                                      : min(__popcll(free) - 1, (target_np - total_post_s) / 6 + 1);
+        const double thr = share * mw;
+        for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
+            const double kw = W.hkey[i];
+            if (kw >= thr && i != e_pick && W.hst[i] == 0) {
+                const int at = atomicAdd(&S.n_list, 1);
+                if (at < room) S.list[at] = i;
+                else atomicMax(&S.dropped, (unsigned long long)__double_as_longlong(kw));
+            }
+        }
+        __syncthreads();
+        const int n_all = S.n_list, n_list = max(fresh ? 1 : 0, min(n_all, room));
+        const double dropped = __longlong_as_double((long long)S.dropped);
+        for (int k = wv; k < n_list; k += NW) {
+            uint64_t f = free;   // the k-th free entry
+            for (int j = 0; j < k; ++j) f &= f - 1;
+            split(__builtin_amdgcn_readfirstlane(S.list[k]), __builtin_ctzll(f));
+        }
+        __syncthreads();
+        if (wv == 0) {
+            uint64_t f = free;
+            for (int j = 0; j < n_list; ++j) f &= f - 1;
+            if (lane == 0) S.pre_free = f;
+            oct_wave_sync();
+            // bins not split: lighter than thr, or at most as heavy as `dropped`
+            take(e_pick, n_all > n_list ? dropped : thr, n_all <= n_list);
+        }
+        // a list that overflows leaves bins out that come before listed ones: a
+        // narrower share then, a wider one while half the places stay empty
+        share = n_all > n_list ? 1.0 - 0.7 * (1.0 - share) : (2 * n_all < PRE ? fmax(0.25, 1.0 - 1.2 * (1.0 - share)) : share);
+        __syncthreads();
+        if (stop_s) break;
     }
     __syncthreads();
     if (S.defer_s) {
@@ -718,9 +861,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
     // particles is summed by its whole wave as a 256-wide block reduction
     // (lane l holds the block threads l, l + 64, l + 128, l + 192), so the
     // values do not depend on which wave runs the bin.
-    int32_t *const bslot = W.bslot;
-    int32_t *const bdraw = W.bdraw;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    IdxT *const bslot = W.bslot;
+    IdxT *const bdraw = W.bdraw;
+    constexpr int LANE_BINS = BIG ? 32 : 128;
     // each bin's output slots (2, or its particles when it has at most 2)
     // and draw offset (6 sign draws per bin of more than 2 particles): an
     // exclusive scan over the bins, two bins per thread and pass, slots in
@@ -752,11 +895,11 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             const int64_t ex = pre + x - v;
             const int b = b0 + 2 * threadIdx.x;
             if (b < Nbins) {
-                bslot[b] = (int32_t)(ex & 0xFFFFFFFF);
-                bdraw[b] = (int32_t)(ex >> 32);
+                bslot[b] = (IdxT)(ex & 0xFFFFFFFF);
+                bdraw[b] = (IdxT)(ex >> 32);
                 if (b + 1 < Nbins) {
-                    bslot[b + 1] = (int32_t)(ex & 0xFFFFFFFF) + (int32_t)oc[0];
-                    bdraw[b + 1] = (int32_t)(ex >> 32) + (int32_t)dr[0];
+                    bslot[b + 1] = (IdxT)((int32_t)(ex & 0xFFFFFFFF) + (int32_t)oc[0]);
+                    bdraw[b + 1] = (IdxT)((int32_t)(ex >> 32) + (int32_t)dr[0]);
                 }
             }
             carry = tot;
@@ -849,11 +992,11 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         }
         if (lane == 0) oct_emit(A, c, bdraw[b], bslot[b], Wb, vm, xm, sdv, sdx, s1, n1, s2);
     };
-    // compute_bin_props! and compute_new_particles! per bin.  With at least 32
-    // bins per wave a bin of at most OCT_LANE_NP particles takes one lane, its
+    // compute_bin_props! and compute_new_particles! per bin.  With at least
+    // LANE_BINS bins (whatever the number of waves, so the sums are the same) a bin of at most OCT_LANE_NP particles takes one lane, its
     // sums in particle order (the reference's order), and a larger bin the whole
     // wavefront; with fewer bins the waves take the bins in turn.
-    if (Nbins < 32 * NW) {
+    if (Nbins < LANE_BINS) {
         for (int b = wv; b < Nbins; b += NW) {
             const int32_t bnp = bins[b].w == 0.0 ? 0 : (int32_t)bins[b].np;
             if (bnp <= 0) continue;
@@ -867,7 +1010,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             wave_bin(b);
         }
     }
-    for (int b0 = wv * 64; Nbins >= 32 * NW && b0 < Nbins; b0 += NW * 64) {
+    for (int b0 = wv * 64; Nbins >= LANE_BINS && b0 < Nbins; b0 += NW * 64) {
         const int bl = b0 + lane;
         int32_t bnp = 0;
         int bs = 0, par = 0;
@@ -942,11 +1085,13 @@ __device__ inline bool oct_pick(const OctArgs &A, int c, int32_t &N, int32_t &ta
 // One workgroup per cell, the working arrays in LDS.
 __global__ void __launch_bounds__(256) k_octree_merge(OctArgs A) {
     __shared__ int16_t pis[OCT_MAX_N];
-    __shared__ __align__(16) int16_t psort[OCT_MAX_N];   // after the splits: per-bin slots and draws
-    __shared__ uint8_t poct[OCT_MAX_N];
+    __shared__ int16_t psort[OCT_MAX_N];
+    __shared__ __align__(16) uint8_t poct[OCT_MAX_N];   // after the splits: per-bin slots and draws
     __shared__ OctBin bins[OCT_MAX_BINS];
-    __shared__ double bkey[OCT_MAX_BINS];
-    __shared__ OctShared S;
+    __shared__ double hkey[OCT_MAX_BINS];
+    __shared__ int16_t hid[OCT_MAX_BINS];
+    __shared__ uint8_t hst[OCT_MAX_BINS];
+    __shared__ OctShared<OCT_PRE_LDS> S;
     const int c = blockIdx.x;
     A.rp = mz_rng_resolve(A.rp);
     int32_t N, target;
@@ -959,27 +1104,37 @@ __global__ void __launch_bounds__(256) k_octree_merge(OctArgs A) {
         return;
     }
     OctWork<int16_t> W;
-    W.pis = pis; W.psort = psort; W.poct = poct; W.bins = bins; W.bkey = bkey;
-    W.bslot = reinterpret_cast<int32_t *>(psort);
+    W.pis = pis; W.psort = psort; W.poct = poct; W.bins = bins;
+    W.hkey = hkey; W.hid = hid; W.hst = hst;
+    static_assert(2 * OCT_MAX_BINS * sizeof(int16_t) <= OCT_MAX_N, "the slots and draws fit the octants");
+    W.bslot = reinterpret_cast<int16_t *>(poct);
     W.bdraw = W.bslot + OCT_MAX_BINS;
     W.bins_cap = OCT_MAX_BINS;
-    W.bmv = nullptr;
-    W.bmi = nullptr;
-    oct_merge_cell<int16_t, 4, false>(A, c, N, target, W, S);
+    oct_merge_cell<int16_t, 4, false, OCT_PRE_LDS>(A, c, N, target, W, S);
 }
 
-// The listed cells, one wavefront per workgroup, the working arrays in the
-// workgroup's slice of device memory.  The workgroups take cells from a queue,
-// the largest size class first, so the longest merges start first.
-__global__ void __launch_bounds__(64) k_octree_merge_big(OctArgs A) {
-    __shared__ OctShared S;
-    // per 64-bin block: its largest key (nblk doubles), then its lowest bin
-    // holding that key (nblk int32s)
-    extern __shared__ double s_blk[];
+// The listed cells, one workgroup per cell, the working arrays in the
+// workgroup's slice of device memory; the list of bins that may be refined
+// (13 B each) in dynamic LDS, or in the slice too.  The workgroups take cells
+// from a queue, the largest size class first, so the longest merges start
+// first.
+// Up to one listed cell per CU, the longest merge is the launch: eight waves a
+// cell and the list in LDS where it fits (30 to 180 cells of up to 30,000
+// particles: 4 % less for the whole step than four waves with the list in
+// memory).  More cells than CUs: four waves and the list in memory, so that
+// three cells share a CU (25,935 cells of up to 30,333 particles, mean of 14
+// calls: 10.3 ms; eight waves with the list in LDS, one cell a CU: 13.3 ms;
+// eight, in memory: 13.8; two: 10.5; one: 11.4; the picks one at a time by one
+// wave each: 10.9).
+#define OCT_BIG_WAVES 8
+#define OCT_BIG_WAVES_MANY 4
+template <bool LDS_LIST, int WAVES>
+__global__ void __launch_bounds__(WAVES * 64) k_octree_merge_big(OctArgs A) {
+    __shared__ OctShared<OCT_PRE_BIG> S;
+    extern __shared__ double s_list[];
     A.rp = mz_rng_resolve(A.rp);
     const int32_t n_list = A.big_info[0];
     const size_t g = blockIdx.x;
-    const int nblk = (A.big_bcap + 63) >> 6;
     OctWork<int32_t> W;
     W.pis = A.big_pis + g * (size_t)A.big_ncap;
     W.psort = A.big_psort + g * (size_t)A.big_ncap;
@@ -989,12 +1144,16 @@ __global__ void __launch_bounds__(64) k_octree_merge_big(OctArgs A) {
     W.n_stg = A.big_ncap;
     W.poct = A.big_poct + g * (size_t)A.big_ncap;
     W.bins = reinterpret_cast<OctBinT<int32_t> *>(A.big_bins) + g * (size_t)A.big_bcap;
-    W.bkey = A.big_bkey + g * (size_t)A.big_bcap;
     W.bslot = A.big_bslot + g * (size_t)A.big_bcap * 2;
     W.bdraw = W.bslot + A.big_bcap;
     W.bins_cap = A.big_bcap;
-    W.bmv = A.big_blocks ? s_blk : nullptr;
-    W.bmi = A.big_blocks ? reinterpret_cast<int32_t *>(s_blk + nblk) : nullptr;
+    {
+        const int hc = A.big_hcap;   // a multiple of 64
+        double *base = LDS_LIST ? s_list : A.big_list_mem + g * (oct_list_bytes(hc) / sizeof(double));
+        W.hkey = base;
+        W.hid = reinterpret_cast<int32_t *>(W.hkey + hc);
+        W.hst = reinterpret_cast<uint8_t *>(W.hid + hc);
+    }
     for (;;) {
         if (threadIdx.x == 0) S.ticket_s = atomicAdd(&A.big_info[6], 1);
         __syncthreads();
@@ -1006,7 +1165,7 @@ __global__ void __launch_bounds__(64) k_octree_merge_big(OctArgs A) {
         const int c = A.big_list[(size_t)cls * A.n_cells + t];
         int32_t N, target;
         oct_pick(A, c, N, target);
-        if (N <= A.big_ncap) oct_merge_cell<int32_t, 1, true>(A, c, N, target, W, S);
+        if (N <= A.big_ncap) oct_merge_cell<int32_t, WAVES, true, OCT_PRE_BIG>(A, c, N, target, W, S);
         else if (threadIdx.x == 0) atomicOr(&A.sp.ctr->err, MZ_ERR_MERGE_SIZE);
         __syncthreads();
     }
@@ -1215,12 +1374,18 @@ static int octree_merge_launch(mz_store *h, int32_t species, int32_t threshold, 
             // largest per-cell target when there are several)
             const int64_t ncap = ((int64_t)info[1] + 255) / 256 * 256;
             const int64_t bcap = std::min<int64_t>({(int64_t)max_Nbins, ncap, (int64_t)std::max(target_np, 2)}) + 8;
+            // a bin that may be refined holds three particles or more, of
+            // which two count towards the target: at most target / 2 at a time
+            const int64_t hcap = (std::max<int64_t>(target_np, 2) / 2 + 8 + 63) / 64 * 64;
+            const size_t lb = oct_list_bytes(hcap);
+            int dev = 0, n_cu = 0, per_cu = 0;
+            MZ_HIP(hipGetDevice(&dev));
+            MZ_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+            const bool many = info[0] > n_cu;   // the measurements stand at k_octree_merge_big
+            const bool lds = !many && lb <= OCT_LIST_LDS;
+            const size_t dyn = lds ? lb : 0;
             const int64_t per = ncap * (2 * sizeof(int32_t) + 8 * sizeof(double) + 1) +
-                                bcap * (sizeof(OctBinT<int32_t>) + 3 * sizeof(double));
-            // the blocks' maxima in LDS: 12 bytes per 64-bin block
-            const int64_t nblk = (bcap + 63) / 64;
-            const bool blocks = nblk <= OCT_BIG_BLOCKS;
-            const size_t dyn = blocks ? (size_t)((nblk * 12 + 15) / 16 * 16) : 0;
+                                bcap * (sizeof(OctBinT<int32_t>) + 2 * sizeof(int32_t)) + (lds ? 0 : (int64_t)lb);
             // workgroups: as many as can be resident (the loop is latency-bound,
             // so every resident wave helps), within a quarter of the free memory
             // (at least 2 GiB, at most 16 GiB)
@@ -1228,10 +1393,12 @@ static int octree_merge_launch(mz_store *h, int32_t species, int32_t threshold, 
             MZ_HIP(hipMemGetInfo(&mfree, &mtot));
             const int64_t budget = std::min<int64_t>((int64_t)16 << 30, std::max<int64_t>((int64_t)2 << 30,
                                                                                           (int64_t)(mfree / 4)));
-            int dev = 0, n_cu = 0, per_cu = 0;
-            MZ_HIP(hipGetDevice(&dev));
-            MZ_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-            MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_octree_merge_big, 64, dyn));
+            const int nt = (many ? OCT_BIG_WAVES_MANY : OCT_BIG_WAVES) * 64;
+            const void *fn = many  ? (const void *)k_octree_merge_big<false, OCT_BIG_WAVES_MANY>
+                             : lds ? (const void *)k_octree_merge_big<true, OCT_BIG_WAVES>
+                                   : (const void *)k_octree_merge_big<false, OCT_BIG_WAVES>;
+            if (lds) MZ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn));
+            MZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, nt, dyn));
             const int64_t G = std::max<int64_t>(1, std::min<int64_t>({(int64_t)info[0],
                                                                       (int64_t)std::max(per_cu, 1) * n_cu,
                                                                       budget / per}));
@@ -1239,20 +1406,21 @@ static int octree_merge_launch(mz_store *h, int32_t species, int32_t threshold, 
             uint8_t *ob = (uint8_t *)mz_scratch(h, "oct_big_oct", (size_t)(G * ncap));
             double *stg = (double *)mz_scratch(h, "oct_big_stage", (size_t)(G * ncap * 8 * sizeof(double)));
             void *bb = mz_scratch(h, "oct_big_bins", (size_t)(G * bcap * sizeof(OctBinT<int32_t>)));
-            double *kb = (double *)mz_scratch(h, "oct_big_key", (size_t)(G * bcap * sizeof(double)));
+            double *kb = lds ? nullptr : (double *)mz_scratch(h, "oct_big_list_mem", (size_t)G * lb);
             int32_t *sb = (int32_t *)mz_scratch(h, "oct_big_slot", (size_t)(G * bcap * 2 * sizeof(int32_t)));
-            MZ_CHECK(ib && ob && stg && bb && kb && sb, "merge_octree: scratch allocation for large cells failed");
+            MZ_CHECK(ib && ob && stg && bb && (lds || kb) && sb, "merge_octree: scratch allocation for large cells failed");
             A.big_pis = ib;
             A.big_psort = ib + G * ncap;
             A.big_poct = ob;
             A.big_stage = stg;
             A.big_bins = bb;
-            A.big_bkey = kb;
+            A.big_list_mem = kb;
             A.big_bslot = sb;
             A.big_ncap = (int32_t)ncap;
             A.big_bcap = (int32_t)bcap;
-            A.big_blocks = blocks ? 1 : 0;
-            hipLaunchKernelGGL(k_octree_merge_big, dim3((unsigned)G), dim3(64), dyn, h->stream, A);
+            A.big_hcap = (int32_t)hcap;
+            void *args[] = {&A};
+            MZ_HIP(hipLaunchKernel(fn, dim3((unsigned)G), dim3((unsigned)nt), args, dyn, h->stream));
         }
         hipLaunchKernelGGL(k_merge_ndel, dim3((nc + 255) / 256), dim3(256), 0, h->stream, old_pia, nc, ndel);
         hipLaunchKernelGGL(k_scan_i32m, dim3(1), dim3(1024), 0, h->stream, ndel, (int64_t)nc, off, off + nc);
