@@ -321,14 +321,20 @@ __device__ inline int32_t mz_cell_of(double x0, const MzGrid &g, int32_t n_cells
 // compute_props! of one cell on one wave (physical_props.jl:104-154 and
 // 317-454): n = sum w, vbar = sum w v / n, and T from the centred energy,
 // in one pass with shifted sums (shift = the cell's first particle), lanes
-// striding over the cell's logical positions.  get(i, w, v0, v1, v2) loads
-// logical particle i.  Every kernel that computes props goes through here,
+// striding over the cell's logical positions, AHEAD loads of a lane in flight
+// (the sums' order is the same with any).  get(i, w, v0, v1, v2) loads logical
+// particle i.  Every kernel that computes props goes through here,
 // so all paths sum in the same order.
 struct MzPropsOut {
     double n, v0, v1, v2, T;
 };
 
-template <class Get>
+// One load a pass left a wave waiting on memory: a cell of 20,000 particles took
+// 100 us a step, about 35 us with eight loads of a lane in flight (k_batch0d, one
+// wave on the cell; 2,048 uneven cells, 50 steps: 29.3 -> 25.7 ms).  Kernels
+// that are short of registers, with cells of a few hundred particles, keep 1.
+#define MZ_PROPS_AHEAD 8
+template <int AHEAD = 1, class Get>
 __device__ inline MzPropsOut mz_props_wave(const Get &get, int32_t tot, double mass) {
     const int lane = threadIdx.x & 63;
     double sx = 0.0, sy = 0.0, sz = 0.0;
@@ -337,15 +343,28 @@ __device__ inline MzPropsOut mz_props_wave(const Get &get, int32_t tot, double m
         get(0, w0, sx, sy, sz);
     }
     double n = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0, e = 0.0;
-    for (int32_t i = lane; i < tot; i += 64) {
-        double w, v0, v1, v2;
-        get(i, w, v0, v1, v2);
+    auto add = [&](double w, double v0, double v1, double v2) {
         const double d0 = v0 - sx, d1 = v1 - sy, d2 = v2 - sz;
         n += w;
         a0 = fma(w, d0, a0);
         a1 = fma(w, d1, a1);
         a2 = fma(w, d2, a2);
         e = fma(w, d0 * d0 + d1 * d1 + d2 * d2, e);
+    };
+    int32_t i = lane;
+    if (AHEAD > 1) {
+        for (; i + 64 * (AHEAD - 1) < tot; i += 64 * AHEAD) {
+            double w[AHEAD], v0[AHEAD], v1[AHEAD], v2[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) get(i + 64 * k, w[k], v0[k], v1[k], v2[k]);
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) add(w[k], v0[k], v1[k], v2[k]);
+        }
+    }
+    for (; i < tot; i += 64) {
+        double w, v0, v1, v2;
+        get(i, w, v0, v1, v2);
+        add(w, v0, v1, v2);
     }
     n = mz_wave_sum(n);
     a0 = mz_wave_sum(a0);

@@ -1859,7 +1859,7 @@ __global__ void __launch_bounds__(256) k_props(MzViews views, int32_t n_cells, i
         const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
         w = sp.w[p]; v0 = sp.v0[p]; v1 = sp.v1[p]; v2 = sp.v2[p];
     };
-    const MzPropsOut o = mz_props_wave(get, tot, masses[sidx]);
+    const MzPropsOut o = mz_props_wave<MZ_PROPS_AHEAD>(get, tot, masses[sidx]);
     if (lane == 0) {
         const int64_t ix = (int64_t)sidx * n_cells + c;
         out_np[ix] = (double)tot;
@@ -2004,8 +2004,16 @@ extern "C" int mz_get_flux(mz_store *h, int32_t which, double *kinetic_energy_fl
 
 // compute_props_with_total_moments! (physical_props.jl:168-245): n, v and T
 // over groups 1 and 2 as compute_props!, plus the total moments
-// sum w |v - vbar|^p / (scaling_p n) for the requested powers p.  One wave per
-// (cell, species); the mean is reduced first, then the centred sums.
+// sum w |v - vbar|^p / (scaling_p n) for the requested powers p.  One wave or
+// workgroup per (cell, species); the mean is reduced first, then the centred sums.
+//
+// What bounds it: the powers (a pow of each particle's speed per moment) on
+// the one wave of the largest cell.  With cells few enough that their
+// workgroups are resident together, a workgroup takes a cell (1,024 uneven
+// cells of up to 30,000 particles, three moments: 13.9 -> 12.7 ms for a pass
+// of two calls among splitting steps; 4,096 cells of about 1,150: no change).
+#define MOMENTS_JOINT_CELLS 4096
+template <int WAVES>
 __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_cells, int32_t n_mom,
                                                        const int32_t *__restrict__ powers,
                                                        const double *__restrict__ scale,   // [species][n_mom]
@@ -2014,14 +2022,26 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
                                                        double *__restrict__ out_T, double *__restrict__ out_m) {
     const int sidx = blockIdx.y;
     const MzSpView &sp = views.v[sidx];
-    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    const int c = WAVES > 1 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int lane = WAVES > 1 ? (int)threadIdx.x : (int)(threadIdx.x & 63);   // among the cell's threads
+    __shared__ double part[WAVES];
+    // the sum over the cell's threads, on every one of them
+    auto total = [&](double x) {
+        x = mz_wave_sum(x);
+        if (WAVES == 1) return x;
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+        __syncthreads();
+        x = part[0];
+        for (int k = 1; k < WAVES; ++k) x += part[k];
+        return x;
+    };
     if (c >= n_cells) return;
     const int32_t st1 = sp.pia.start1[c] - 1, n1 = sp.pia.n1[c];
     const int32_t st2 = sp.pia.start2[c] - 1, n2 = sp.pia.n2[c] > 0 ? sp.pia.n2[c] : 0;
     const int32_t tot = n1 + n2;
     double n = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int32_t i = lane; i < tot; i += 64) {
+    for (int32_t i = lane; i < tot; i += 64 * WAVES) {
         const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
         const double w = sp.w[p];
         n += w;
@@ -2029,17 +2049,17 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
         a1 = a1 + sp.v1[p] * w;
         a2 = a2 + sp.v2[p] * w;
     }
-    n = mz_wave_sum(n);
-    a0 = mz_wave_sum(a0);
-    a1 = mz_wave_sum(a1);
-    a2 = mz_wave_sum(a2);
+    n = total(n);
+    a0 = total(a0);
+    a1 = total(a1);
+    a2 = total(a2);
     double m0 = 0.0, m1 = 0.0, m2 = 0.0, E = 0.0;
     double mom[MZ_MAX_MOMENTS];
 #pragma unroll
     for (int j = 0; j < MZ_MAX_MOMENTS; ++j) mom[j] = 0.0;
     if (n > 0.0) {
         m0 = a0 / n; m1 = a1 / n; m2 = a2 / n;
-        for (int32_t i = lane; i < tot; i += 64) {
+        for (int32_t i = lane; i < tot; i += 64 * WAVES) {
             const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
             const double w = sp.w[p];
             const double d0 = sp.v0[p] - m0, d1 = sp.v1[p] - m1, d2 = sp.v2[p] - m2;
@@ -2049,10 +2069,10 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
             for (int j = 0; j < MZ_MAX_MOMENTS; ++j)
                 if (j < n_mom) mom[j] += w * pow(normv, (double)powers[j]);
         }
-        E = mz_wave_sum(E);
+        E = total(E);
 #pragma unroll
         for (int j = 0; j < MZ_MAX_MOMENTS; ++j)
-            if (j < n_mom) mom[j] = mz_wave_sum(mom[j]);
+            if (j < n_mom) mom[j] = total(mom[j]);
     }
     if (lane == 0) {
         double T = 0.0;
@@ -2093,9 +2113,14 @@ extern "C" int mz_compute_props_moments(mz_store *h, const int32_t *powers, int3
     h->masses_valid = false;   // the couette drivers upload their mass again
     {
         MzTimed tm(h, "props");
-        dim3 grid((h->n_cells + 3) / 4, ns);
-        hipLaunchKernelGGL(k_props_moments, grid, dim3(256), 0, h->stream, mz_views(h), h->n_cells, n_moments,
-                           d_pow, d_sc, h->d_masses, h->d_np, h->d_n, h->d_v, h->d_T, d_m);
+        if ((int64_t)h->n_cells * ns <= MOMENTS_JOINT_CELLS)
+            hipLaunchKernelGGL(k_props_moments<4>, dim3(h->n_cells, ns), dim3(256), 0, h->stream, mz_views(h),
+                               h->n_cells, n_moments, d_pow, d_sc, h->d_masses, h->d_np, h->d_n, h->d_v, h->d_T,
+                               d_m);
+        else
+            hipLaunchKernelGGL(k_props_moments<1>, dim3((h->n_cells + 3) / 4, ns), dim3(256), 0, h->stream,
+                               mz_views(h), h->n_cells, n_moments, d_pow, d_sc, h->d_masses, h->d_np, h->d_n,
+                               h->d_v, h->d_T, d_m);
         MZ_HIP(hipGetLastError());
     }
     MZ_HIP(hipStreamSynchronize(h->stream));
