@@ -606,36 +606,7 @@ __global__ void k_ntc_count(NtcArgs A, int32_t *__restrict__ ncoll) {
 // total goes to *total.
 __global__ void __launch_bounds__(1024) k_scan_i32(const int32_t *__restrict__ in, int64_t n,
                                                    int64_t *__restrict__ out, int64_t *__restrict__ total) {
-    __shared__ int64_t wsum[16];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int64_t per = (n + 1023) / 1024;
-    const int64_t lo = t * per, hi = min(n, lo + per);
-    int64_t s = 0;
-    for (int64_t i = lo; i < hi; ++i) s += in[i];
-    int64_t x = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int64_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wv] = x;
-    __syncthreads();
-    if (t < 16) {
-        int64_t a = wsum[t], b = a;
-        for (int o = 1; o < 16; o <<= 1) {
-            int64_t y = __shfl_up(b, o, 16);
-            if ((t & 15) >= o) b += y;
-        }
-        wsum[t] = b - a;
-    }
-    __syncthreads();
-    int64_t run = x - s + wsum[wv];
-    for (int64_t i = lo; i < hi; ++i) {
-        int64_t v = in[i];
-        out[i] = run;
-        run += v;
-    }
-    if (t == 1023) *total = run;
+    mz_scan_counts(in, n, out, total);
 }
 
 // Append pass: created particles of cell c go to positions
