@@ -112,9 +112,9 @@ int mz_set_replay(mz_store *h, int32_t kind, const double *table, int64_t rows, 
 int mz_sort(mz_store *h, int32_t species, int32_t compute_cells);
 /* mz_sort without allocating: no counterpart in the reference; for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc).  The count matrix, the
- * cell starts and (when the species is not contiguous) the squash's group
- * starts use a fixed device array of 2^21 int32 words (8 MiB) that each GPU
+ * serving loops, harnesses that forbid hipMalloc).  The count matrix and
+ * (when the species is not contiguous) the squash's group starts use a
+ * fixed device array of 2^21 int32 words (8 MiB) that each GPU
  * holds until the process ends; no hipMalloc, hipFree or allocating library
  * call is made.  It rejects with an error the radix path (more than 14336
  * cells, or a count matrix over 8 x capacity words) and shapes whose

@@ -245,8 +245,8 @@ __device__ inline int mz_wave_sum_i(int v) {
 }
 // Exclusive scan of n counts by one workgroup of 1,024 threads: tiles of 4,096
 // counts, four a thread, the next tile's loads in flight, one barrier a tile.
-// Latency bounds it.  (A contiguous piece of the counts per thread instead, read
-// twice and written 128 B apart between lanes, took 26 us for 16,000.)
+// Latency bounds it: 10.6 us for 16,000.  (A contiguous piece of the counts per thread instead, read
+// twice and written 128 B apart between lanes, took 26 us.)
 __device__ inline void mz_scan_counts(const int32_t *__restrict__ in, int64_t n, int64_t *__restrict__ out,
                                       int64_t *__restrict__ total) {
     __shared__ int64_t wsum[2][16];
