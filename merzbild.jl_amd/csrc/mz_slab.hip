@@ -430,7 +430,8 @@ __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(Slab
     // The large slabs' particles that reach a wall (a few per cent of the wall
     // cell, so some in every 64) are listed, in the arrival-rank rows, and
     // flown one per lane, so a wave spends one reflection's latency (about 3
-    // us) and not one for each particle slot of its threads.
+    // us) and not one for each particle slot of its threads.  Every slab makes
+    // the list: a fast particle can cross a whole slab and reach the wall.
     constexpr bool HIT_LIST = LARGE && !AVG;
     const int nd = WAVE_NTC ? (ncl <= 8 ? 256 : SLAB_DRAWS) : SLAB_DRAWS;
     auto fill_draws = [&](uint64_t stp, int t0, int stride) {
@@ -609,7 +610,7 @@ __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(Slab
             MzRngParams rp = A.rp;
             rp.tag = (step << 4) | 2u;
             uint32_t flown = 0;   // bit r: the flight of this thread's r-th particle is done
-            if (HIT_LIST && !(has_left && has_right)) {
+            if (HIT_LIST) {
                 for (;;) {   // as many as the list takes at a time
                     for (int r = 0; r < R; ++r) {
                         const int i = r * NT + tid;
@@ -626,6 +627,7 @@ __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(Slab
                     }
                     __syncthreads();
                     const int hits = s_hits;
+                    if (hits == 0) break;   // most steps of most slabs
                     for (int h = tid; h < min(hits, 2 * SLAB_MB_CAP); h += NT) {
                         const int i = (&arank[0][0])[h];
                         double x0 = sx0[i], v0 = sv0[i], v1 = sv1[i], v2 = sv2[i];
