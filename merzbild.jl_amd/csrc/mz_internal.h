@@ -101,7 +101,7 @@ struct mz_store {
     double masses_up[MZ_MAX_SPECIES] = {0.0, 0.0, 0.0, 0.0};
     bool masses_valid = false;
     std::vector<double> V_up;
-    std::vector<double> ntc_V_up;    // of the NTC calls, at ntc_V_dev
+    std::vector<double> ntc_V_up;    // of the NTC and SWPM calls, at ntc_V_dev
     const void *ntc_V_dev = nullptr;
     int32_t last_path = -1;   // of mz_couette_steps: 0 eager, 1 graph, 2 slab
     int32_t n_moments = 0;    // moments of the last mz_compute_props_moments

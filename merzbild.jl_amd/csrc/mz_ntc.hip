@@ -780,7 +780,7 @@ static int launch_ntc_split(mz_store *h, int s1, int s2, double dt, const double
     return 0;
 }
 
-// The cell volumes V[n_cells] of an NTC call on the device.  They upload
+// The cell volumes V[n_cells] of an NTC or SWPM call on the device.  They upload
 // only when they differ from the last upload; an upload first waits for the
 // store's stream, whose queued kernels may still read the previous values.
 static int upload_ntc_volumes(mz_store *h, const double *V, const double **out) {
@@ -949,10 +949,8 @@ extern "C" int mz_swpm(mz_store *h, int32_t species, double G, double dt, const 
     MZ_CHECK(rng_mode == 0 || (rng_mode == 1 && h->d_replay[0]), "swpm: replay table not set");
     const double *dV = h->d_V;
     if (V) {
-        double *v = (double *)mz_scratch(h, "ntc_V", h->n_cells * sizeof(double));
-        MZ_CHECK(v != nullptr, "swpm: scratch allocation failed");
-        MZ_HIP(hipMemcpy(v, V, h->n_cells * sizeof(double), hipMemcpyHostToDevice));
-        dV = v;
+        int r = upload_ntc_volumes(h, V, &dV);
+        if (r) return r;
     } else {
         MZ_CHECK(h->has_grid, "swpm: V is NULL and no grid is set");
     }

@@ -192,3 +192,33 @@ def test_bkw_swpm_octree_on_device(hip, mzo):
         a = ac.bkw_analytic(t, magic, p)
         assert np.max(np.abs(a - mom[:, j]) / a) < tol, (p, np.max(np.abs(a - mom[:, j]) / a))
     st.close()
+
+
+def test_ntc_volumes_after_a_swpm_call(hip, mzo):
+    """ntc, swpm and ntc on one store, each with the volumes it is given: the
+    SWPM call (dt = 0, so it collides nothing) has others than the NTC calls
+    around it."""
+    nc, npc = 12, 60
+    pv, pia = _zero_d_case(mzo, nc, npc, seed=3)
+    it = mzo.interactions(["Ar"])[0][0]
+    vs = np.sqrt(helpers.KB * 300.0 / helpers.MASS_AR)
+    sg = it.vhs_factor * (2 * vs) ** (1.0 - 2 * it.vhs_o) * 2 * vs * 1e12
+    st, it, _ = _ntc_setup(hip, mzo, pv, pia, nc, sg, cap=nc * npc * 2)
+    V = np.linspace(1.0, 2.0, nc)
+    dt = 80.0 / (npc * npc * sg)
+    cfs = (mzo.CF * nc)()
+    for c in range(nc):
+        cfs[c].sigma_g_w_max = sg
+    for step in (1, 2):
+        tag = (step << 4) | 1
+        hip.ntc(st, 1, 1, dt, V=V, equal_weight=True, tag=tag)
+        r = mzo.RNG(seed=77, tag=tag)
+        for c in range(1, nc + 1):
+            mzo.lib().mzo_ntc_single(r.ref, C.byref(cfs[c - 1]), C.byref(it), pv.p, pia.p, c, 1, dt, V[c - 1], 1e-16, 1)
+        cf = st.collision_factors(1, 1)
+        assert np.array_equal(cf["n_coll"], [cfs[c].n_coll for c in range(nc)]), step
+        helpers.assert_state_matches(mzo, st.download_species(1), pv, pia, rtol=1e-11)
+        hip.swpm(st, 1, 1.0, 0.0, V=5.0 * V, tag=tag)
+        st.set_sigma_g_w_max(1, 1, np.array([cfs[c].sigma_g_w_max for c in range(nc)]))
+    assert cf["n_coll"].sum() > 100
+    st.close()
