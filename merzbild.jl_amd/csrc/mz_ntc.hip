@@ -392,13 +392,14 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
         const int64_t pk = in_k ? (int64_t)(sk < C.n1b ? st1b + sk : st2b + (sk - C.n1b))
                                 : sc_b + C.s_base + (sk - C.nlb);
         double sgwm = S.sgwm;
-        bool acc = false;
+        bool acc = false, eq = KIND == NTC_PLAIN;     // eq: the collision makes no split
         if (live && !fresh && !same) {
             vi0 = (in_i ? A.a.v0 : A.sc[3])[pi]; vk0 = (in_k ? A.b.v0 : A.sc[3])[pk];
             vi1 = (in_i ? A.a.v1 : A.sc[4])[pi]; vk1 = (in_k ? A.b.v1 : A.sc[4])[pk];
             vi2 = (in_i ? A.a.v2 : A.sc[5])[pi]; vk2 = (in_k ? A.b.v2 : A.sc[5])[pk];
             wi = (in_i ? A.a.w : A.sc[6])[pi];
             wk = (in_k ? A.b.w : A.sc[6])[pk];
+            if (KIND == NTC_SPLIT) eq = fabs(wi - wk) < A.dw_tol;
             // the direction needs the draws only: it is worked out while the
             // loads are in flight, for every candidate
             double e0, e1, e2;
@@ -417,11 +418,13 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
             // lowers t / (sigma g w)_max
             acc = d2 < t / sgwm;
             if (acc) {
-                if (SWPM || (CREATES && wi > wk)) {
+                // the particle that a split copies: the heavier, or the
+                // second of two equal ones that dw_tol does not call equal
+                if (SWPM || (CREATES && !eq && wi > wk)) {
                     xi0 = (in_i ? A.a.x0 : A.sc[0])[pi]; xi1 = (in_i ? A.a.x1 : A.sc[1])[pi];
                     xi2 = (in_i ? A.a.x2 : A.sc[2])[pi];
                 }
-                if (SWPM || (CREATES && wk > wi)) {
+                if (SWPM || (CREATES && !eq && !(wi > wk))) {
                     xk0 = (in_k ? A.b.x0 : A.sc[0])[pk]; xk1 = (in_k ? A.b.x1 : A.sc[1])[pk];
                     xk2 = (in_k ? A.b.x2 : A.sc[2])[pk];
                 }
@@ -432,7 +435,6 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
         }
         const uint64_t samem = __ballot(live && same && !fresh), slowm = __ballot(slow);
         const uint64_t stop = __ballot(!live || fresh) | samem | slowm, ends = mz_window_ends(T, M);
-        const bool eq = KIND == NTC_PLAIN || (KIND == NTC_SPLIT && fabs(wi - wk) < A.dw_tol);
         // collisions after which the particle count is not the predicted one
         const uint64_t eqm = __ballot(eq), last = KIND != NTC_SPLIT ? 0 : __ballot(eq == (inc > 0));
         uint64_t accm = __ballot(acc), maxm = __ballot(sg > sgwm);

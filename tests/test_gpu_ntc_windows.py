@@ -105,3 +105,54 @@ def test_two_species_windows_vs_oracle(hip, mzo, nc):
         assert got["err"] == 0 and got["n_total"] > nc * (na, nb)[s - 1]
         helpers.assert_state_matches(mzo, got, pvs[s - 1], pia, species=s, rtol=RTOL)
     st.close()
+
+
+@pytest.mark.parametrize("two", [False, True])
+def test_equal_weights_without_tolerance_vs_oracle(hip, mzo, two):
+    """dw_tol = 0 with equal weights: no pair counts as equal, so a collision
+    of two of them leaves a copy of weight 0 of the second, at its position."""
+    nc, n = 6, 40
+    rng = np.random.default_rng(8)
+    names, m = (["Ar", "He"], [66.3e-27, 6.65e-27]) if two else (["Ar"], [66.3e-27])
+    ns = len(names)
+    pvs, pia = [mzo.ParticleVector(nc * n) for _ in names], mzo.PIA(nc, ns)
+    for s, pv in enumerate(pvs, start=1):
+        for i in range(1, nc * n + 1):
+            pv.pop_to(i)
+            pv.set(i, 1e12, rng.normal(0, np.sqrt(helpers.KB * 300.0 / m[s - 1]), 3),
+                   [(i - 1) // n + rng.uniform(0.1, 0.9), *rng.uniform(size=2)])
+        for c in range(1, nc + 1):
+            pia.set(c, s, n, (c - 1) * n + 1, c * n, n)
+        pia.set_n_total(s, nc * n)
+    its = mzo.interactions(names)
+    st = hip.DeviceStore(nc, ns, [8 * nc * n] * ns)
+    for s in range(1, ns + 1):
+        helpers.upload_from_oracle(st, mzo, pvs[s - 1], pia, species=s)
+    st.set_interactions([[type("I", (), dict(mu1=its[i][k].mu1, mu2=its[i][k].mu2, vhs_factor=its[i][k].vhs_factor,
+                                             vhs_o=its[i][k].vhs_o))() for k in range(ns)] for i in range(ns)])
+    it, b = its[0][ns - 1], ns
+    sg = mzo.lib().mzo_estimate_sigma_g_w_max(C.byref(it), m[0], m[-1], 300.0, 300.0, 1e12, 1.0)
+    st.set_sigma_g_w_max(1, b, np.full(nc, sg))
+    st.set_seed(12)
+    cfs = (mzo.CF * nc)()
+    for c in range(nc):
+        cfs[c].sigma_g_w_max = sg
+    dt = 30.0 / (n * n * sg)
+    tag = (2 << 4) | 1
+    hip.ntc(st, 1, b, dt, V=1.0, dw_tol=0.0, tag=tag)
+    r = mzo.RNG(seed=12, tag=tag)
+    for c in range(1, nc + 1):
+        if two:
+            mzo.lib().mzo_ntc_two(r.ref, C.byref(cfs[c - 1]), C.byref(it), pvs[0].p, pvs[1].p, pia.p, c, 1, 2, dt, 1.0,
+                                  0.0, 0)
+        else:
+            mzo.lib().mzo_ntc_single(r.ref, C.byref(cfs[c - 1]), C.byref(it), pvs[0].p, pia.p, c, 1, dt, 1.0, 0.0, 0)
+    cf = st.collision_factors(1, b)
+    assert np.array_equal(cf["n_coll_performed"], [cfs[c].n_coll_performed for c in range(nc)])
+    assert not np.any(cf["n_eq_w_coll_performed"]) and cf["n_coll_performed"].sum() > 20
+    got = [st.download_species(s) for s in range(1, ns + 1)]
+    assert sum(g["n_total"] for g in got) == ns * nc * n + cf["n_coll_performed"].sum()
+    for s, g in enumerate(got, start=1):
+        assert g["err"] == 0
+        helpers.assert_state_matches(mzo, g, pvs[s - 1], pia, species=s, rtol=RTOL)
+    st.close()
