@@ -88,7 +88,8 @@ struct mz_store {
     // captured step graphs
     hipGraphExec_t graph_exec = nullptr;
     hipGraph_t graph = nullptr;
-    std::string graph_key;
+    std::string graph_key;               // the arguments it was captured with
+    const double *graph_x0 = nullptr;    // the buffer current at its start and end
     uint64_t *d_step = nullptr;
     // slab-resident Couette kernel: requested shape (0 = automatic) and the
     // last launch's {particles per thread, cells per slab, slabs, outcome}

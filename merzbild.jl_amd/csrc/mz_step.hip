@@ -3,14 +3,15 @@
 // launched kernel by kernel or replayed as a captured hipGraph.
 //
 // A captured graph holds two steps: the sort writes into the second particle
-// buffer, so two steps bring the buffers back to where the capture started.
+// buffer, so two steps bring the buffers back to where the capture started.  It
+// is captured again when anything its launches hold has changed.
 // The random tags of captured kernels come from a device step counter that the
 // graph's last node advances, so every replay draws fresh numbers in the same
 // (step << 4) | phase layout as eager launches.
 #include "mz_internal.h"
 
-#include <cstdio>
 #include <cstring>
+#include <string>
 #include <vector>
 
 __global__ void k_set_step(uint64_t *step, uint64_t v) {
@@ -154,11 +155,26 @@ static int couette_run(mz_store *h, int32_t n_steps, uint64_t step0, double dt, 
         h->sp[0].contig_known = true;
         return 0;
     }
-    // graph replay
-    char keybuf[256];
-    std::snprintf(keybuf, sizeof(keybuf), "couette:%a:%d:%p:%a:%a:%a:%a:%d", dt, props_every, (const void *)dV,
-                  avg_inv, mass, h->surf_inv_area[0], h->surf_inv_area[1], h->sort_path);
-    if (h->graph_key != keybuf) {
+    // Graph replay.  The captured launches hold their arguments by value, so
+    // the key names all of them that a call can change; the current buffers are
+    // the one exception, below.
+    const MzSpecies &s = h->sp[0];
+    std::string key("couette");
+    auto add = [&key](const void *p, size_t n) { key.append((const char *)p, n); };
+    add(&dt, sizeof(dt));
+    add(&props_every, sizeof(props_every));
+    add(&dV, sizeof(dV));
+    add(&avg_inv, sizeof(avg_inv));
+    add(&mass, sizeof(mass));
+    add(h->surf_inv_area, sizeof(h->surf_inv_area));
+    add(&h->sort_path, sizeof(h->sort_path));
+    add(&h->seed, sizeof(h->seed));
+    add(&h->grid, sizeof(h->grid));
+    add(&h->walls, sizeof(h->walls));
+    add(&h->inter[0], sizeof(h->inter[0]));
+    add(&s.key, sizeof(s.key));         // a squash exchanges the key arrays
+    add(&s.buffer, sizeof(s.buffer));   // an upload may enlarge the free ids
+    if (h->graph_key != key) {
         mz_graph_release(h);
         MZ_HIP(hipMalloc(&h->d_step, sizeof(uint64_t)));
         // scratch is allocated before capture
@@ -178,14 +194,24 @@ static int couette_run(mz_store *h, int32_t n_steps, uint64_t step0, double dt, 
         }
         MZ_HIP(hipStreamEndCapture(h->stream, &h->graph));
         MZ_HIP(hipGraphInstantiate(&h->graph_exec, h->graph, nullptr, nullptr, 0));
-        h->graph_key = keybuf;
+        h->graph_key = key;
+        h->graph_x0 = s.x[0];
     }
-    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, h->stream, h->d_step, step0);
     MzTimed tm(h, "step", n_steps);
-    for (int32_t t = 0; t + 1 < n_steps; t += 2) MZ_HIP(hipGraphLaunch(h->graph_exec, h->stream));
-    if (n_steps & 1) {
-        uint64_t step = step0 + (uint64_t)(n_steps - 1);
-        r = enqueue_step(h, dV, dt, props_every == 1, step, nullptr, avg_inv, mass);
+    int32_t t = 0;
+    auto eager_step = [&]() { return enqueue_step(h, dV, dt, props_every == 1, step0 + (uint64_t)t++, nullptr, avg_inv, mass); };
+    // The graph holds two steps from one of the two buffers back to it.  Where
+    // the other one is current (after an odd number of steps or sorts), one
+    // step launched on its own comes first; an odd step left over comes last.
+    if (n_steps > 0 && s.x[0] != h->graph_x0) {
+        r = eager_step();
+        if (r) return r;
+    }
+    if (t + 1 < n_steps)
+        hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, h->stream, h->d_step, step0 + (uint64_t)t);
+    for (; t + 1 < n_steps; t += 2) MZ_HIP(hipGraphLaunch(h->graph_exec, h->stream));
+    if (t < n_steps) {
+        r = eager_step();
         if (r) return r;
     }
     h->sp[0].contig_known = true;
