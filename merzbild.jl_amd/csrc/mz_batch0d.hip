@@ -483,6 +483,7 @@ extern "C" int mz_batch0d_steps(mz_store *h, int32_t species, int32_t n_steps, u
     MZ_CHECK(n_steps >= 0, "batch0d: negative step count");
     MZ_CHECK(mode >= 0 && mode <= 2,
              "batch0d: mode must be 0 (per-step kernels), 1 (persistent) or 2 (one NTC launch per cell)");
+    MZ_HIP(hipStreamSynchronize(h->stream));   // queued kernels may still read what is uploaded
     MZ_HIP(hipMemcpy(h->d_masses, masses, h->n_species * sizeof(double), hipMemcpyHostToDevice));
     h->masses_valid = false;   // the couette drivers upload their mass again
     const double *dV = h->d_V;

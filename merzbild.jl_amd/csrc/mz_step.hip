@@ -84,8 +84,9 @@ static int couette_run(mz_store *h, int32_t n_steps, uint64_t step0, double dt, 
     MZ_CHECK(masses != nullptr, "couette_steps: masses is NULL");
     MZ_CHECK(n_steps >= 0, "couette_steps: negative step count");
     // uploads only of what changed since the last call (the device copies
-    // are written by nothing else than these uploads)
+    // are written by nothing else than these uploads), after queued kernels
     if (!h->masses_valid || h->masses_up[0] != masses[0]) {
+        MZ_HIP(hipStreamSynchronize(h->stream));
         MZ_HIP(hipMemcpy(h->d_masses, masses, sizeof(double), hipMemcpyHostToDevice));
         h->masses_up[0] = masses[0];
         h->masses_valid = true;
@@ -95,6 +96,7 @@ static int couette_run(mz_store *h, int32_t n_steps, uint64_t step0, double dt, 
         double *v = (double *)mz_scratch(h, "step_V", h->n_cells * sizeof(double));
         MZ_CHECK(v != nullptr, "couette_steps: scratch allocation failed");
         if (h->V_up.size() != (size_t)h->n_cells || std::memcmp(h->V_up.data(), V, h->n_cells * sizeof(double))) {
+            MZ_HIP(hipStreamSynchronize(h->stream));
             MZ_HIP(hipMemcpy(v, V, h->n_cells * sizeof(double), hipMemcpyHostToDevice));
             h->V_up.assign(V, V + h->n_cells);
         }

@@ -217,7 +217,8 @@ extern "C" int mz_create(int32_t n_cells, int32_t n_species, const int64_t *capa
     MZ_HIP(hipMalloc(&h->d_pavg, pavg_bytes));
     MZ_HIP(hipMemset(h->d_pavg, 0, pavg_bytes));
     h->inter.resize(nss);
-    MZ_HIP(hipStreamSynchronize(h->stream));
+    // the clears above run on the null stream, which the store's stream does not wait for
+    MZ_HIP(hipStreamSynchronize(nullptr));
     // the fixed scratch array of mz_sort_noalloc: its address on this device
     int rs = mz_noalloc_scratch_init(nullptr);
     if (rs) return rs;
@@ -303,7 +304,9 @@ void *mz_scratch(mz_store *h, const char *name, size_t bytes) {
 }
 
 // ===========================================================================
-// upload / download
+// upload / download.  The store's stream does not wait for hipMemcpy, nor
+// hipMemcpy for it: an upload over values that queued kernels may still read
+// first waits for the stream.
 extern "C" int mz_upload_species(mz_store *h, int32_t species, int64_t n_pos, const double *x,
                                  const double *v, const double *w, const int64_t *ids,
                                  const int64_t *pia, int64_t n_total, int32_t contiguous,
@@ -320,8 +323,8 @@ extern "C" int mz_upload_species(mz_store *h, int32_t species, int64_t n_pos, co
     // the free-id LIFO holds at most `length` ids; creations can grow length up
     // to the slot capacity plus one resize! chunk
     int64_t need = std::max<int64_t>(length, s.cap) + 2 * MZ_DELTA_PARTICLES;
+    MZ_HIP(hipStreamSynchronize(h->stream));
     if (need > s.bufcap) {
-        MZ_HIP(hipStreamSynchronize(h->stream));
         hipFree(s.buffer);
         s.bufcap = need;
         MZ_HIP(hipMalloc(&s.buffer, s.bufcap * sizeof(int32_t)));
@@ -397,6 +400,7 @@ extern "C" int mz_upload_cell_keys(mz_store *h, int32_t species, int64_t n, cons
         MZ_CHECK(cells[i] >= 1 && cells[i] <= h->n_cells, "upload_cell_keys: cell out of range");
         k[i] = (int32_t)cells[i];
     }
+    MZ_HIP(hipStreamSynchronize(h->stream));
     if (n > 0) MZ_HIP(hipMemcpy(s.key, k.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
     return 0;
 }
@@ -484,6 +488,7 @@ extern "C" int mz_set_grid_1d(mz_store *h, double L, int64_t nx, double wall_off
     h->has_grid = true;
     // Cell1D(xlo, xhi, V): V = dx, inv_V = 1/V (grid_uniform1D.jl:20-31, 76-82)
     std::vector<double> V(nx, dx), iV(nx, 1.0 / dx);
+    MZ_HIP(hipStreamSynchronize(h->stream));
     MZ_HIP(hipMemcpy(h->d_V, V.data(), nx * sizeof(double), hipMemcpyHostToDevice));
     MZ_HIP(hipMemcpy(h->d_invV, iV.data(), nx * sizeof(double), hipMemcpyHostToDevice));
     return 0;
@@ -516,6 +521,7 @@ extern "C" int mz_set_interaction(mz_store *h, int32_t s1, int32_t s2, double mu
 extern "C" int mz_set_sigma_g_w_max(mz_store *h, int32_t s1, int32_t s2, const double *sgwm) {
     MZ_CHECK(s1 >= 1 && s1 <= h->n_species && s2 >= 1 && s2 <= h->n_species, "set_sgwm: bad species");
     size_t off = ((size_t)(s1 - 1) * h->n_species + (s2 - 1)) * h->n_cells;
+    MZ_HIP(hipStreamSynchronize(h->stream));
     MZ_HIP(hipMemcpy(h->d_sgwm + off, sgwm, h->n_cells * sizeof(double), hipMemcpyHostToDevice));
     return 0;
 }
