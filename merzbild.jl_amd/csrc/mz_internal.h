@@ -75,6 +75,7 @@ struct mz_store {
     int32_t *d_err = nullptr;
     // of the count-matrix sort: the cells' totals (left at 0 by every sort) and starts
     int32_t *d_ccount = nullptr, *d_cstart = nullptr;
+    uint64_t *d_ntc_left = nullptr;   // NTC, SWPM: a bit per cell of a call that its lanes leave
     double *d_np = nullptr, *d_n = nullptr, *d_v = nullptr, *d_T = nullptr;
     double *d_V = nullptr, *d_invV = nullptr;
     double *d_masses = nullptr;

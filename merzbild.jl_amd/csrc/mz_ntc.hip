@@ -362,16 +362,16 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
     const int32_t st1a = A.a.pia.start1[c] - 1, st2a = A.a.pia.start2[c] - 1;
     const int32_t st1b = A.b.pia.start1[c] - 1, st2b = A.b.pia.start2[c] - 1;
     const int64_t sc_b = !CREATES || single ? 0 : A.sc_cap;   // species half 1 of the scratch
-    int T = 4;
+    int lt = 2;   // log2 of the number of tracks T: 0 .. 3
     int32_t inc = SWPM ? 2 : (CREATES && single ? 1 : 0);
     int64_t cc = 0;
     uint64_t o = dr.k;
     while (cc < C.n_coll) {
         const uint64_t D = o;
-        const int M = T == 1 ? NTC_T1_LEN : 64 / T;
+        const int T = 1 << lt, M = lt == 0 ? NTC_T1_LEN : 64 >> lt;
         dr.cover(D, 5 * (T - 1) + 3 * (M - 1) + 5);
         const int32_t na0 = S.na, nb0 = single ? S.na : S.nb;
-        const int a_l = T == 1 ? 0 : lane / M;
+        const int a_l = lt == 0 ? 0 : lane >> (6 - lt);
         const int j_l = lane - a_l * M;
         const int64_t cand = cc + a_l + j_l;
         const bool live = j_l < M && cand < C.n_coll;
@@ -434,7 +434,7 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
             }
         }
         const uint64_t samem = __ballot(live && same && !fresh), slowm = __ballot(slow);
-        const uint64_t stop = __ballot(!live || fresh) | samem | slowm, ends = mz_window_ends(T, M);
+        const uint64_t stop = __ballot(!live || fresh) | samem | slowm, ends = mz_window_ends(lt, NTC_T1_LEN);
         // collisions after which the particle count is not the predicted one
         const uint64_t eqm = __ballot(eq), last = KIND != NTC_SPLIT ? 0 : __ballot(eq == (inc > 0));
         uint64_t accm = __ballot(acc), maxm = __ballot(sg > sgwm);
@@ -515,8 +515,8 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
         }
         cc += a + j;
         o = D + (uint64_t)(5 * a + 3 * j);
-        if (why == MZ_WALK_TRACKS) T = min(8, 2 * T);
-        else if (why == MZ_WALK_TRACK && 2 * a < T) T = max(1, T / 2);
+        if (why == MZ_WALK_TRACKS) lt = min(3, lt + 1);
+        else if (why == MZ_WALK_TRACK && 2 * a < T) lt = max(0, lt - 1);
         bool direct = false;
         if (why == MZ_WALK_STOP) {
             direct = ((samem >> pos) & 1) || pos == 0;   // pos 0: a pick out of range by rounding
@@ -541,50 +541,128 @@ __device__ __forceinline__ void ntc_windows(const NtcArgs &A, const int c, const
     }
 }
 
-// Calls over more cells than this first run the cells of at most
-// NTC_LANE_MAX candidates one lane each (k_ntc), then the others one wavefront
-// each; calls over fewer run every cell on a wavefront.  A window costs about
-// 4 us however few of its lanes hold a candidate, and some 3,000 wavefronts
-// run at once: 16,000 cells of one candidate take 45 us on wavefronts and
-// 16 us on lanes, 2,000 cells of seven 21 us on wavefronts against 4 us per
-// candidate on lanes; 65,536 cells of 20 to 20,000 particles 14.0 ms on lanes
-// and 9.4 ms on wavefronts.
+// Calls over at most NTC_WAVE_MAX_CELLS cells run every cell on a wavefront.
+// Calls over more run a pass of one lane per cell, which leaves some cells to
+// a second pass of one wavefront per cell.  A lane takes lane_us per candidate,
+// one after another, however many cells there are (until the gathers of all
+// lanes fill the memory: NTC_LANE_FILL us per candidate and cell).  The second
+// pass has a latency of its own (NTC_LEFT_US), and a cell takes window_ns of the
+// whole chip for its start and for each window, which reaches as far as its
+// tracks do or until a particle is met again, after about sqrt(particles)
+// candidates.  So each group of 64 cells picks the number of candidates up to
+// which its cells run on lanes that makes the sum of its longest lane and of the
+// second pass, were all groups like it, the least.
+//
+// us a call, all on lanes / all on wavefronts / this rule.  No particles created,
+// cells of 60 particles and c candidates: 8,192 cells, c = 6 23 / 39 / 28, c = 25 75
+// / 85 / 80, c = 100 276 / 246 / 234; 16,384, c = 12 45 / 84 / 50, c = 200 610 / 840
+// / 624; 65,536, c = 12 127 / 278 / 135.  Splitting: 8,192, c = 100 653 / 392 / 356;
+// 32,768, c = 50 631 / 720 / 564.  Cells of 2 to 125 candidates, evenly over the
+// logarithm: 16,384 cells 364 / 150 / 174, splitting 911 / 394 / 415.  What the
+// rule costs where lanes are right is the second launch: 9 -> 12 us for 4,097 cells
+// of one candidate, 12 -> 17 us for 65,536.
 #define NTC_WAVE_MAX_CELLS 4096
-#define NTC_LANE_MAX 4
+#define NTC_LANE_MIN 4            // candidates that always run on a lane
+#define NTC_LANE_FILL 1.2e-4
+#define NTC_LEFT_US 12.0
+struct NtcCost {
+    double lane_us, window_ns;
+};
+#define NTC_COST_PLAIN NtcCost{2.75, 1.8}
+#define NTC_COST_SPLIT NtcCost{5.0, 2.5}
+#define NTC_COST_SWPM NtcCost{5.0, 1.8}
+
+// Whether this lane's cell (in: there is one), of n candidates among np
+// particles, runs on the lane; `cells` in the call.  All 64 lanes take part.
+__device__ __forceinline__ bool ntc_on_lane(bool in, int64_t n, int32_t np, int cells, const NtcCost &k) {
+    const double x = in ? (double)n : 0.0, top = mz_wave_max(x);
+    if (!(top > NTC_LANE_MIN)) return true;
+    const double share = k.window_ns * 1e-3 * cells / __popcll(__ballot(in));
+    const double wave_us = share * (1.0 + x / fmin(18.0, sqrt((double)np)));
+    const double c = fmax(k.lane_us, NTC_LANE_FILL * cells);
+    double best = 1e300, most = NTC_LANE_MIN;
+    for (double t = NTC_LANE_MIN;; t *= 2.0) {
+        const bool all = t >= top;
+        const double cost = c * mz_wave_max(x <= t ? x : 0.0) +
+                            (all ? 0.0 : NTC_LEFT_US + mz_wave_sum(x <= t ? 0.0 : wave_us));
+        // a bound between the least and all has to be clearly better: the
+        // longest lane of any group holds up the call
+        if (cost < (all ? best : 0.8 * best)) {
+            best = cost;
+            most = t;
+        }
+        if (all) break;
+    }
+    return x <= most;
+}
+
+// Whether this lane runs its cell (in: there is one); left gets a bit for each
+// cell that is left.
+__device__ __forceinline__ bool ntc_stays(const NtcArgs &A, bool in, int64_t n, int32_t np, const NtcCost &k,
+                                          uint64_t *left) {
+    if (left) {
+        const bool on = ntc_on_lane(in, n, np, A.cell_hi - A.cell_lo + 1, k);
+        const uint64_t m = __ballot(!on);
+        if (threadIdx.x == 0) left[blockIdx.x] = m;
+        if (!on) return false;
+    }
+    return in;
+}
 
 // One lane per cell; cells run in parallel (64-lane workgroups, so the loop
-// keeps its state in registers).  Cells of more than max_coll candidates are
-// left, their count noted, for k_ntc_wave.
-__global__ void __launch_bounds__(64) k_ntc(NtcArgs A, int64_t max_coll) {
+// keeps its state in registers).  left == nullptr: every cell.
+__global__ void __launch_bounds__(64) k_ntc(NtcArgs A, uint64_t *left) {
     const int c = A.cell_lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c > A.cell_hi) return;
+    const bool in = c <= A.cell_hi;
     A.rp = mz_rng_resolve(A.rp);
     NtcLaneDraw dr{A.rp, mz_stream((uint64_t)c)};
     NtcCell C;
     NtcState S;
-    ntc_setup(A, c, dr, C, S);
-    if (C.n_coll > max_coll) {
-        A.cnt[(int64_t)c * 5 + 2] = (int32_t)C.n_coll;
-        return;
-    }
+    C.n_coll = C.nla = C.nlb = 0;
+    if (in) ntc_setup(A, c, dr, C, S);
+    if (!ntc_stays(A, in, C.n_coll, min(C.nla, C.nlb), A.may_split ? NTC_COST_SPLIT : NTC_COST_PLAIN, left)) return;
     for (int64_t cc = 0; cc < C.n_coll; ++cc)
         if (!ntc_candidate(A, c, C, S, dr)) return;
     ntc_finish_cell(A, c, C, S);
 }
 
-// One wavefront per cell (Philox draws), candidates a window at a time; cells
-// of at most min_coll candidates (after k_ntc) are done already.
+// The cells left by the lanes: wavefront k of the launch looks after cells
+// per k .. per k + per - 1 (per divides 64).  Up to 8,192 cells a workgroup is one
+// wavefront and one cell; in larger calls, where mostly none is left, it is four,
+// of several cells each, since a workgroup's start costs more than its look
+// (65,536 of them 16 us).  One queue for all wavefronts costs 20 ns a cell, its
+// counter's atomics one after another: 80 us for 4,096 cells.
+template <class Run>
+__device__ __forceinline__ void ntc_left_cells(const NtcArgs &A, const uint64_t *left, int per, Run run) {
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c0 = per * (blockIdx.x * (blockDim.x >> 6) + wv);   // from A.cell_lo
+    if (A.cell_lo + c0 > A.cell_hi) return;
+    uint64_t m = left[c0 >> 6] >> (c0 & 63);
+    if (per < 64) m &= (1ull << per) - 1;
+    for (; m; m &= m - 1) run(A.cell_lo + c0 + (int)__builtin_ctzll(m));
+}
+
+// Cell c on this wavefront (Philox draws), candidates a window at a time.
 template <int KIND>
-__global__ void __launch_bounds__(64) k_ntc_wave(NtcArgs A, int32_t min_coll) {
-    const int c = A.cell_lo + blockIdx.x;
-    if (c > A.cell_hi || (min_coll > 0 && A.cnt[(int64_t)c * 5 + 2] <= min_coll)) return;
-    A.rp = mz_rng_resolve(A.rp);
+__device__ __forceinline__ void ntc_wave_cell(const NtcArgs &A, const int c) {
     NtcWaveDraw dr{A.rp, (uint64_t)c, 0, ~(uint64_t)0, 0.0, 0.0};
     NtcCell C;
     NtcState S;
     ntc_setup(A, c, dr, C, S);
     ntc_windows<KIND>(A, c, C, S, dr, 0.0, 0.0);
     if ((threadIdx.x & 63) == 0) ntc_finish_cell(A, c, C, S);
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(64) k_ntc_wave(NtcArgs A) {
+    A.rp = mz_rng_resolve(A.rp);
+    ntc_wave_cell<KIND>(A, A.cell_lo + blockIdx.x);
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(256) k_ntc_left(NtcArgs A, const uint64_t *left, int per) {
+    A.rp = mz_rng_resolve(A.rp);
+    ntc_left_cells(A, left, per, [&](int c) { ntc_wave_cell<KIND>(A, c); });
 }
 
 // Count pass of the split path: n_coll of every cell (draw 0 of its stream).
@@ -707,16 +785,33 @@ static NtcArgs base_args(mz_store *h, int s1, int s2, double dt, const double *d
     return A;
 }
 
+// the launch shape of ntc_left_cells
+struct NtcLeftShape {
+    dim3 grid, block;
+    int per;
+};
+static NtcLeftShape ntc_left_shape(int ncells) {
+    const int waves = ncells <= 8192 ? 1 : 4;
+    int per = 1;
+    while (per < 64 && ncells > 16384 * per) per *= 2;
+    return NtcLeftShape{dim3((ncells + waves * per - 1) / (waves * per)), dim3(64 * waves), per};
+}
+
 // The candidate loops over ncells cells; replayed draws run one lane per cell.
 static void launch_k_ntc(mz_store *h, const NtcArgs &A, int ncells) {
-    const bool wave = A.rp.mode == 0, few = ncells <= NTC_WAVE_MAX_CELLS;
-    if (!wave || !few)
-        hipLaunchKernelGGL(k_ntc, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A,
-                           wave ? (int64_t)NTC_LANE_MAX : INT64_MAX);
-    if (wave && A.may_split)
-        hipLaunchKernelGGL(k_ntc_wave<NTC_SPLIT>, dim3(ncells), dim3(64), 0, h->stream, A, few ? 0 : NTC_LANE_MAX);
-    else if (wave)
-        hipLaunchKernelGGL(k_ntc_wave<NTC_PLAIN>, dim3(ncells), dim3(64), 0, h->stream, A, few ? 0 : NTC_LANE_MAX);
+    const dim3 lanes((ncells + 63) / 64);
+    uint64_t *const left = h->d_ntc_left;
+    if (A.rp.mode != 0) {
+        hipLaunchKernelGGL(k_ntc, lanes, dim3(64), 0, h->stream, A, (uint64_t *)nullptr);
+    } else if (ncells <= NTC_WAVE_MAX_CELLS) {
+        hipLaunchKernelGGL(A.may_split ? k_ntc_wave<NTC_SPLIT> : k_ntc_wave<NTC_PLAIN>, dim3(ncells), dim3(64), 0,
+                           h->stream, A);
+    } else {
+        hipLaunchKernelGGL(k_ntc, lanes, dim3(64), 0, h->stream, A, left);
+        const NtcLeftShape ls = ntc_left_shape(ncells);
+        hipLaunchKernelGGL(A.may_split ? k_ntc_left<NTC_SPLIT> : k_ntc_left<NTC_PLAIN>, ls.grid, ls.block, 0, h->stream,
+                           A, (const uint64_t *)left, ls.per);
+    }
 }
 
 int mz_launch_ntc_equal(mz_store *h, int s1, int s2, double dt, const double *dV, double dw_tol, int equal_weight,
@@ -913,10 +1008,11 @@ __device__ __forceinline__ void swpm_finish(const NtcArgs &A, const int c, const
     A.created[c] = S.ca;
 }
 
-// One lane per cell, for replayed draws.
-__global__ void __launch_bounds__(64) k_swpm(NtcArgs A, double G, const double *__restrict__ wmax) {
+// One lane per cell (k_ntc's rule).
+__global__ void __launch_bounds__(64) k_swpm(NtcArgs A, double G, const double *__restrict__ wmax, uint64_t *left) {
     const int c = A.cell_lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c > A.cell_hi) return;
+    const bool in = c <= A.cell_hi;
+    if (!ntc_stays(A, in, in ? A.ncoll_in[c] : 0, in ? A.a.pia.nloc[c] : 0, NTC_COST_SWPM, left)) return;
     A.rp = mz_rng_resolve(A.rp);
     NtcLaneDraw dr{A.rp, mz_stream((uint64_t)c)};
     dr.seek(1);
@@ -929,17 +1025,25 @@ __global__ void __launch_bounds__(64) k_swpm(NtcArgs A, double G, const double *
     swpm_finish(A, c, C, S);
 }
 
-// One wavefront per cell (Philox draws), candidates a window at a time.
-__global__ void __launch_bounds__(64) k_swpm_wave(NtcArgs A, double G, const double *__restrict__ wmax) {
-    const int c = A.cell_lo + blockIdx.x;
-    if (c > A.cell_hi) return;
-    A.rp = mz_rng_resolve(A.rp);
+// Cell c on this wavefront (Philox draws), candidates a window at a time.
+__device__ __forceinline__ void swpm_wave_cell(const NtcArgs &A, const int c, double G, const double *wmax) {
     NtcWaveDraw dr{A.rp, (uint64_t)c, 1, ~(uint64_t)0, 0.0, 0.0};
     NtcCell C;
     NtcState S;
     swpm_setup(A, c, C, S);
     ntc_windows<NTC_SWPM>(A, c, C, S, dr, 1.0 / (1.0 + G), 1.0 / wmax[c]);
     if ((threadIdx.x & 63) == 0) swpm_finish(A, c, C, S);
+}
+
+__global__ void __launch_bounds__(64) k_swpm_wave(NtcArgs A, double G, const double *__restrict__ wmax) {
+    A.rp = mz_rng_resolve(A.rp);
+    swpm_wave_cell(A, A.cell_lo + blockIdx.x, G, wmax);
+}
+
+__global__ void __launch_bounds__(256) k_swpm_left(NtcArgs A, double G, const double *__restrict__ wmax,
+                                                   const uint64_t *left, int per) {
+    A.rp = mz_rng_resolve(A.rp);
+    ntc_left_cells(A, left, per, [&](int c) { swpm_wave_cell(A, c, G, wmax); });
 }
 
 extern "C" int mz_swpm(mz_store *h, int32_t species, double G, double dt, const double *V, uint64_t tag,
@@ -985,10 +1089,19 @@ extern "C" int mz_swpm(mz_store *h, int32_t species, double G, double dt, const 
         A.ncoll_in = ncoll;
         A.soff = soff;
         A.created = created;
-        if (rng_mode == 0)
-            hipLaunchKernelGGL(k_swpm_wave, dim3(ncells), dim3(64), 0, h->stream, A, G, (const double *)wmax);
-        else
-            hipLaunchKernelGGL(k_swpm, dim3((ncells + 63) / 64), dim3(64), 0, h->stream, A, G, (const double *)wmax);
+        // the rule of launch_k_ntc
+        const double *const wm = wmax;
+        const dim3 lanes((ncells + 63) / 64);
+        uint64_t *const left = h->d_ntc_left;
+        if (rng_mode != 0) {
+            hipLaunchKernelGGL(k_swpm, lanes, dim3(64), 0, h->stream, A, G, wm, (uint64_t *)nullptr);
+        } else if (ncells <= NTC_WAVE_MAX_CELLS) {
+            hipLaunchKernelGGL(k_swpm_wave, dim3(ncells), dim3(64), 0, h->stream, A, G, wm);
+        } else {
+            hipLaunchKernelGGL(k_swpm, lanes, dim3(64), 0, h->stream, A, G, wm, left);
+            const NtcLeftShape ls = ntc_left_shape(ncells);
+            hipLaunchKernelGGL(k_swpm_left, ls.grid, ls.block, 0, h->stream, A, G, wm, (const uint64_t *)left, ls.per);
+        }
         MZ_HIP(hipGetLastError());
         double **scp = (double **)mz_scratch(h, "ntc_scp", 7 * sizeof(double *));
         MZ_CHECK(scp != nullptr, "swpm: scratch allocation failed");

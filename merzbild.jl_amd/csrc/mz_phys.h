@@ -135,11 +135,13 @@ __device__ __forceinline__ int mz_window_walk(uint64_t acc, uint64_t stop, uint6
     }
 }
 
-// The last lane of each track.
-__device__ __forceinline__ uint64_t mz_window_ends(int T, int M) {
-    uint64_t e = 0;
-    for (int a = 1; a <= T; ++a) e |= 1ull << (a * M - 1);
-    return e;
+// The last lane of each of 1 << lt tracks of 64 >> lt lanes; a single track has
+// t1_len lanes.
+__device__ __forceinline__ uint64_t mz_window_ends(int lt, int t1_len) {
+    return lt == 0   ? 1ull << (t1_len - 1)
+           : lt == 1 ? 0x8000000080000000ull
+           : lt == 2 ? 0x8000800080008000ull
+                     : 0x8080808080808080ull;
 }
 
 // Diffuse re-emission from a wall: three draws (normal, tangential speed

@@ -207,12 +207,12 @@ __device__ inline void slab_ntc_cell(const SlabArgs &A, const MzRngParams &rp, i
 // mz_ntc.hip, without created particles): the candidate reached after a
 // collisions and r rejections starts at draw D + 5 a + 3 r, point a M + j is the
 // one after a collisions and j rejections, a lane each, and the wave
-// walks them in order with ballots; the number T of tracks is kept from step
-// to step.  nd draws are ready in pre; a window past them computes its own.
+// walks them in order with ballots; the number of tracks, 1 << lt, is kept from
+// step to step.  nd draws are ready in pre; a window past them computes its own.
 // All lanes return the same values.
 __device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &rp, int c, double Vc, int32_t base,
                                           int32_t nla, double *sv0, double *sv1, double *sv2, const double *sw,
-                                          const double *pre, int nd, int &T, double &sgwm, int32_t &n_coll_out,
+                                          const double *pre, int nd, int &lt, double &sgwm, int32_t &n_coll_out,
                                           int32_t &performed, int32_t &eqw) {
     const int lane = threadIdx.x & 63;
     int64_t est = (int64_t)floor(mz_ncoll_est(true, A.dt, nla, nla, sgwm, Vc, pre[0]));
@@ -227,8 +227,8 @@ __device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &
     uint32_t o = 1;   // the next draw: at most 2^32 / 5 candidates' draws
     while (cc < n_coll) {
         const uint32_t D = o;
-        const int M = 64 / T;   // T = 1, 2, 4 or 8
-        const int a_l = lane / M, j_l = lane - a_l * M;
+        const int T = 1 << lt, M = 64 >> lt;   // 1, 2, 4 or 8 tracks
+        const int a_l = lane >> (6 - lt), j_l = lane - a_l * M;
         const bool live = cc + a_l + j_l < n_coll;
         const uint32_t sL = D + (uint32_t)(5 * a_l + 3 * j_l);
         double d0, d1, d2, d3, d4;
@@ -253,7 +253,7 @@ __device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &
         const double sg = live && !same && !slow ? mz_vhs_sgw(A.factor, A.expo, g, sw[pi], sw[pk]) : 0.0;
         mz_vhs_dir(d3, d4, e0, e1, e2);
         const uint64_t samem = __ballot(live && same), slowm = __ballot(slow);
-        const uint64_t stop = __ballot(!live) | samem | slowm, ends = mz_window_ends(T, M);
+        const uint64_t stop = __ballot(!live) | samem | slowm, ends = mz_window_ends(lt, 64);
         uint64_t accm = __ballot(d2 < sg / sgwm), maxm = __ballot(sg > sgwm);
         uint64_t taken = 0, seen = 0, dirty = 0, checked = 0;
         int pos = 0, why;
@@ -288,8 +288,8 @@ __device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &
         performed += a;
         cc += a + j;
         o = D + (uint32_t)(5 * a + 3 * j);
-        if (why == MZ_WALK_TRACKS) T = min(8, 2 * T);
-        else if (why == MZ_WALK_TRACK && 2 * a < T) T = max(1, T / 2);
+        if (why == MZ_WALK_TRACKS) lt = min(3, lt + 1);
+        else if (why == MZ_WALK_TRACK && 2 * a < T) lt = max(0, lt - 1);
         bool direct = false;
         if (why == MZ_WALK_STOP) {
             direct = (samem >> pos) & 1;
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(Slab
     double my_sgwm = ntc_lane ? A.sgwm[clo + my_k] : 0.0;
     const double my_V = ntc_lane ? A.V[clo + my_k] : 1.0;
     int32_t my_nla = 0, my_ncoll = 0, my_perf = 0, my_eqw = 0;
-    int ntc_tracks = 8;   // of slab_ntc_cell_wave
+    int ntc_tracks = 3;   // of slab_ntc_cell_wave: log2
 
     double px0[R], px1[R], px2[R], pv0[R], pv1[R], pv2[R], pw[R];
     int32_t pid[R], pkey[R], prank[R], pcell[R];

@@ -193,6 +193,7 @@ extern "C" int mz_create(int32_t n_cells, int32_t n_species, const int64_t *capa
     MZ_HIP(hipMalloc(&h->d_ccount, (2 * ncp + 16) * sizeof(int32_t)));
     MZ_HIP(hipMemset(h->d_ccount, 0, ncp * sizeof(int32_t)));
     h->d_cstart = h->d_ccount + ncp;
+    MZ_HIP(hipMalloc(&h->d_ntc_left, (size_t)(n_cells + 63) / 64 * sizeof(uint64_t)));
     size_t pn = (size_t)n_species * n_cells;
     MZ_HIP(hipMalloc(&h->d_np, pn * sizeof(double)));
     MZ_HIP(hipMalloc(&h->d_n, pn * sizeof(double)));
@@ -265,7 +266,7 @@ extern "C" int mz_destroy(mz_store *h) {
     if (h->h_report) hipHostFree(h->h_report);
     mz_graph_release(h);
     for (auto &s : h->sp) free_species(s);
-    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ccount);
+    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ccount); hipFree(h->d_ntc_left);
     hipFree(h->d_np); hipFree(h->d_n); hipFree(h->d_T); hipFree(h->d_v); hipFree(h->d_V);
     hipFree(h->d_invV);
     hipFree(h->d_masses);

@@ -156,3 +156,49 @@ def test_equal_weights_without_tolerance_vs_oracle(hip, mzo, two):
         assert g["err"] == 0
         helpers.assert_state_matches(mzo, g, pvs[s - 1], pia, species=s, rtol=RTOL)
     st.close()
+
+
+@pytest.mark.parametrize("method", ["equal", "split", "swpm"])
+@pytest.mark.parametrize("nc", [4097, 8200, 17000])
+def test_lanes_and_wavefronts_of_one_call_vs_oracle(hip, mzo, method, nc):
+    """Calls of a pass of lanes and a pass of wavefronts over the cells it
+    leaves, where those passes' shapes change: groups of 64 cells with no, some and
+    only long candidate loops, a last group of one cell, groups of empty cells."""
+    rng = np.random.default_rng(nc)
+    counts = rng.integers(2, 7, nc)
+    counts[64:128] = 30
+    counts[128:1024:7] = 60
+    counts[2000:2100] = 1
+    counts[-1] = 50
+    b = _batched_0d(hip, mzo, nc, 0, seed=31, counts=counts, cap_mult=12)
+    st, pv, pia, it = b["st"], b["pv"], b["pia"], b["it"]
+    sg = np.array([b["cfs"][c].sigma_g_w_max for c in range(nc)]) * 2.0
+    if method == "swpm":
+        sg /= 1e23 / counts
+    st.set_sigma_g_w_max(1, 1, sg)
+    cfs = (mzo.CFSwpm * nc)() if method == "swpm" else b["cfs"]
+    for c in range(nc):
+        if method == "swpm":
+            cfs[c].sigma_g_max = sg[c]
+        else:
+            cfs[c].sigma_g_w_max = sg[c]
+    V = counts / np.where(counts > 6, 250.0, 12.0)   # about 40 candidates in the large cells, one in the others
+    dt, tag = (1.2 if method == "swpm" else 4.0) * b["dt"], (5 << 4) | 1
+    r = mzo.RNG(seed=7, tag=tag)
+    if method == "swpm":
+        hip.swpm(st, 1, 1.0, dt, V=V, tag=tag)
+        for c in range(1, nc + 1):
+            mzo.lib().mzo_swpm(r.ref, C.byref(cfs[c - 1]), C.byref(it), pv.p, pia.p, c, 1, 1.0, dt, V[c - 1])
+    else:
+        hip.ntc(st, 1, 1, dt, V=V, equal_weight=method == "equal", tag=tag)
+        for c in range(1, nc + 1):
+            mzo.lib().mzo_ntc_single(r.ref, C.byref(cfs[c - 1]), C.byref(it), pv.p, pia.p, c, 1, dt, V[c - 1], 1e-16,
+                                     1 if method == "equal" else 0)
+    cf = st.collision_factors(1, 1)
+    assert np.array_equal(cf["n_coll"], [cfs[c].n_coll for c in range(nc)])
+    assert np.array_equal(cf["n_coll_performed"], [cfs[c].n_coll_performed for c in range(nc)])
+    assert cf["n_coll"].max() > 20 and np.median(cf["n_coll"]) <= 4
+    got = st.download_species(1)
+    assert got["err"] == 0
+    helpers.assert_state_matches(mzo, got, pv, pia, rtol=RTOL)
+    st.close()
