@@ -2015,11 +2015,16 @@ extern "C" int mz_get_flux(mz_store *h, int32_t which, double *kinetic_energy_fl
 // workgroup per (cell, species); the mean is reduced first, then the centred sums.
 //
 // What bounds it: the powers (a pow of each particle's speed per moment) on
-// the one wave of the largest cell.  With cells few enough that their
-// workgroups are resident together, a workgroup takes a cell (1,024 uneven
-// cells of up to 30,000 particles, three moments: 13.9 -> 12.7 ms for a pass
-// of two calls among splitting steps; 4,096 cells of about 1,150: no change).
-#define MOMENTS_JOINT_CELLS 4096
+// the one wave of the largest cell.  With cells so few that their workgroups run
+// together, a workgroup takes a cell: all of its waves where it has more than
+// MOMENTS_JOINT_NP particles, else one, since the sums across the waves then cost
+// more than they save.  us a call with three moments, wave / workgroup a cell: 1
+// cell of 100 particles 9.1 / 9.5, of 300 13.8 / 10.6, of 20,000 511 / 136; 500
+// cells of 20 8.5 / 8.8, of 300 15.8 / 12.7, of 5,000 173 / 79.  4,096 cells of 3
+// 14.0 / 16.4, of 300 39 / 51, of 1,200 134 / 129: they fill the chip with a wave
+// each.
+#define MOMENTS_JOINT_CELLS 1024
+#define MOMENTS_JOINT_NP 256
 template <int WAVES>
 __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_cells, int32_t n_mom,
                                                        const int32_t *__restrict__ powers,
@@ -2030,12 +2035,19 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
     const int sidx = blockIdx.y;
     const MzSpView &sp = views.v[sidx];
     const int c = WAVES > 1 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
-    const int lane = WAVES > 1 ? (int)threadIdx.x : (int)(threadIdx.x & 63);   // among the cell's threads
+    if (c >= n_cells) return;
+    const int32_t st1 = sp.pia.start1[c] - 1, n1 = sp.pia.n1[c];
+    const int32_t st2 = sp.pia.start2[c] - 1, n2 = sp.pia.n2[c] > 0 ? sp.pia.n2[c] : 0;
+    const int32_t tot = n1 + n2;
+    const bool joint = WAVES > 1 && tot > MOMENTS_JOINT_NP;
+    if (WAVES > 1 && !joint && threadIdx.x >= 64) return;
+    const int lane = joint ? (int)threadIdx.x : (int)(threadIdx.x & 63);   // among the cell's threads
+    const int step = joint ? 64 * WAVES : 64;
     __shared__ double part[WAVES];
     // the sum over the cell's threads, on every one of them
     auto total = [&](double x) {
         x = mz_wave_sum(x);
-        if (WAVES == 1) return x;
+        if (!joint) return x;
         __syncthreads();
         if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
         __syncthreads();
@@ -2043,12 +2055,8 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
         for (int k = 1; k < WAVES; ++k) x += part[k];
         return x;
     };
-    if (c >= n_cells) return;
-    const int32_t st1 = sp.pia.start1[c] - 1, n1 = sp.pia.n1[c];
-    const int32_t st2 = sp.pia.start2[c] - 1, n2 = sp.pia.n2[c] > 0 ? sp.pia.n2[c] : 0;
-    const int32_t tot = n1 + n2;
     double n = 0.0, a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int32_t i = lane; i < tot; i += 64 * WAVES) {
+    for (int32_t i = lane; i < tot; i += step) {
         const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
         const double w = sp.w[p];
         n += w;
@@ -2066,7 +2074,7 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
     for (int j = 0; j < MZ_MAX_MOMENTS; ++j) mom[j] = 0.0;
     if (n > 0.0) {
         m0 = a0 / n; m1 = a1 / n; m2 = a2 / n;
-        for (int32_t i = lane; i < tot; i += 64 * WAVES) {
+        for (int32_t i = lane; i < tot; i += step) {
             const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
             const double w = sp.w[p];
             const double d0 = sp.v0[p] - m0, d1 = sp.v1[p] - m1, d2 = sp.v2[p] - m2;

@@ -61,3 +61,36 @@ def test_moments_wave_and_workgroup_per_cell(hip):
         st.close()
     for a, b, atol in zip(*out, (0.0, 1e-12 * 1500.0, 0.0, 0.0)):
         assert np.allclose(a, b, rtol=1e-12, atol=atol, equal_nan=True)
+
+
+def test_moments_of_cells_on_one_and_all_waves_of_a_workgroup(hip):
+    """1,020 cells, a workgroup each, of which those of more than 256 particles use
+    all its waves, against numpy in long double: sums of up to 1,500 positive
+    terms, and a power of a ulp or two each."""
+    counts = np.array([256, 257, 1500, 0, 1, 255, 320, 2] + [9] * 1012)
+    nc, n = len(counts), int(counts.sum())
+    rng = np.random.default_rng(6)
+    v, w = rng.normal(50.0, 300.0, size=(n, 3)), rng.uniform(0.5, 2.0, n)
+    first = np.cumsum(counts) - counts
+    pia = np.zeros((nc, 7), dtype=np.int64)
+    pia[:, 0] = pia[:, 3] = counts
+    pia[:, 1], pia[:, 2], pia[:, 5] = first + 1, first + counts, -1
+    st = hip.DeviceStore(nc, 1, n)
+    st.upload_species(1, np.full((n, 3), 0.5), v, w, np.arange(1, n + 1), pia, n, True, None, n)
+    pp = hip.PhysProps(nc, 1, [4, 6], Tref=300.0)
+    hip.compute_props_with_total_moments(st, [hip.Species("Ar", helpers.MASS_AR)], pp)
+    ratio = []
+    for c in range(nc):
+        s = slice(first[c], first[c] + counts[c])
+        wl, vl = w[s].astype(np.longdouble), v[s].astype(np.longdouble)
+        assert pp.np[0, c] == counts[c]
+        if counts[c] < 3:
+            continue
+        mean = (wl[:, None] * vl).sum(0) / wl.sum()
+        speed = np.sqrt(((vl - mean) ** 2).sum(1))
+        assert abs(pp.n[0, c] / wl.sum() - 1) < 1e-13
+        assert np.all(np.abs(pp.v[0, c] - mean) < 1e-12 * 1500.0)
+        assert abs(pp.T[0, c] / ((wl * speed ** 2).sum() * helpers.MASS_AR / (3 * wl.sum() * helpers.KB)) - 1) < 1e-12
+        ratio.append([pp.moments[0, c, j] / ((wl * speed ** p).sum() / wl.sum()) for j, p in enumerate((4, 6))])
+    assert np.allclose(ratio, ratio[0], rtol=1e-12, atol=0)   # the scaling is the same for every cell
+    st.close()
