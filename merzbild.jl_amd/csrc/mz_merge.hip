@@ -20,7 +20,7 @@
 // A cell of more than OCT_MAX_N particles, or one whose split loop would
 // need more than OCT_MAX_BINS bins, is handed on: the LDS kernel lists it and
 // a second kernel merges the listed cells with the same code on arrays in
-// device memory (one slice per workgroup, one wavefront per workgroup, the
+// device memory (one slice per workgroup, four or eight wavefronts each, the
 // workgroups taking the listed cells in turn).  The split loop keeps its
 // state in LDS either way; the cell's arrays are then read through L2.
 #include "mz_internal.h"
@@ -84,7 +84,9 @@ using OctBin = OctBinT<int16_t>;
 // output slots and draw offsets.
 template <class IdxT>
 struct OctWork {
-    IdxT *pis, *psort;        // LDS path: the order of parity 0 and 1
+    // LDS path: the order of parity 0, then that of parity 1 (one array and an
+    // offset: a choice between two pointers would hide that both are in LDS)
+    IdxT *ord;
     uint8_t *poct;
     OctBinT<IdxT> *bins;
     IdxT *bslot, *bdraw;
@@ -159,73 +161,56 @@ __device__ __forceinline__ double *oct_stg(const OctWork<IdxT> &W, int q, int k)
 // The values of the particle at tree position i of a bin of depth parity par:
 // through the particle order (LDS path) or from the staged buffer.
 template <class IdxT, bool BIG>
-__device__ __forceinline__ void oct_ld(const OctArgs &A, const OctWork<IdxT> &W, const IdxT *pis, int32_t s1,
+__device__ __forceinline__ void oct_ld(const OctArgs &A, const OctWork<IdxT> &W, int32_t s1,
                                        int32_t n1, int32_t s2, int par, int i, double &w, double &a0, double &a1,
                                        double &a2) {
     if constexpr (BIG) {
         w = oct_stg(W, par, 0)[i]; a0 = oct_stg(W, par, 1)[i]; a1 = oct_stg(W, par, 2)[i]; a2 = oct_stg(W, par, 3)[i];
     } else {
-        const int64_t p = oct_slot((par ? W.psort : W.pis)[i], s1, n1, s2);
+        const int64_t p = oct_slot(W.ord[par * OCT_MAX_N + i], s1, n1, s2);
         w = A.sp.w[p]; a0 = A.sp.v0[p]; a1 = A.sp.v1[p]; a2 = A.sp.v2[p];
     }
 }
 
 // The id (place in the cell) of the particle at tree position i.
 template <class IdxT, bool BIG>
-__device__ __forceinline__ int oct_id(const OctWork<IdxT> &W, const IdxT *pis, int par, int i) {
+__device__ __forceinline__ int oct_id(const OctWork<IdxT> &W, int par, int i) {
     if constexpr (BIG) return oct_sid(W, par)[i];
-    else return (par ? W.psort : W.pis)[i];
+    else return W.ord[par * OCT_MAX_N + i];
 }
 
-__device__ inline double blk_min(double v, double *red) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = red[0];
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmin(r, red[k]);
-    __syncthreads();
-    return r;
-}
-__device__ inline double blk_max(double v, double *red) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = red[0];
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, red[k]);
-    __syncthreads();
-    return r;
-}
-__device__ inline double blk_sum(double v, double *red) {
-    v = mz_wave_sum(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = (red[0] + red[1]) + (red[2] + red[3]);
-    __syncthreads();
-    return r;
-}
-
-// min/max of v over pis[bs..be] (bin_bounds_recompute!, merging_octree_N2.jl:382-418)
-template <class IdxT, int NW>
-__device__ void oct_bounds(const OctArgs &A, const IdxT *pis, int bs, int be, int32_t s1, int32_t n1, int32_t s2,
-                           double *mn, double *mx, double *red) {
-    for (int d = 0; d < 3; ++d) {
-        const double *vv = d == 0 ? A.sp.v0 : (d == 1 ? A.sp.v1 : A.sp.v2);
-        double a = 9299792458.0, b = -9299792458.0;
-        for (int i = bs + threadIdx.x; i <= be; i += blockDim.x) {
-            double x = vv[oct_slot(pis[i], s1, n1, s2)];
-            a = fmin(a, x);
-            b = fmax(b, x);
-        }
-        if (NW == 1) {
-            mn[d] = mz_wave_min(a);
-            mx[d] = mz_wave_max(b);
-        } else {
-            mn[d] = blk_min(a, red);
-            mx[d] = blk_max(b, red);
-        }
+// min/max of v over the N particles of a cell (bin_bounds_recompute!,
+// merging_octree_N2.jl:382-418), on every thread; red holds 6 NW values
+template <int NW>
+__device__ __forceinline__ void oct_bounds(const OctArgs &A, int N, int32_t s1, int32_t n1, int32_t s2, double mn[3],
+                                           double mx[3], double *red) {
+    const double top = 9299792458.0;
+    double r[6] = {top, top, top, top, top, top};   // min of v, then of -v
+    for (int i = threadIdx.x; i < N; i += NW * 64) {
+        const int64_t p = oct_slot(i, s1, n1, s2);
+        const double x0 = A.sp.v0[p], x1 = A.sp.v1[p], x2 = A.sp.v2[p];
+        r[0] = fmin(r[0], x0); r[1] = fmin(r[1], x1); r[2] = fmin(r[2], x2);
+        r[3] = fmin(r[3], -x0); r[4] = fmin(r[4], -x1); r[5] = fmin(r[5], -x2);
     }
+    const int wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        const double m = mz_wave_min(r[q]);
+        if ((threadIdx.x & 63) == 0) red[6 * wv + q] = m;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        double lo = red[d], hi = red[3 + d];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) {
+            lo = fmin(lo, red[6 * k + d]);
+            hi = fmin(hi, red[6 * k + 3 + d]);
+        }
+        mn[d] = lo;
+        mx[d] = -hi;
+    }
+    __syncthreads();
 }
 
 // The end of an N:2 merge of cell c (compute_new_particles!,
@@ -286,13 +271,19 @@ __device__ inline void oct_emit(const OctArgs &A, int c, int32_t draw, int slot,
                                 int32_t s2) {
     MzStream st = mz_stream((uint64_t)c);
     st.k = 6 * (uint64_t)draw;
+    double u[6];
+    if (A.rp.mode == 0) {   // six draws from an even place: three blocks
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            mz_philox_pair(A.rp, st.stream, 3 * (uint64_t)draw + d, u[2 * d], u[2 * d + 1]);
+    } else {
+#pragma unroll
+        for (int d = 0; d < 6; ++d) u[d] = mz_rand(A.rp, st);
+    }
     double dv[3], dx[3];
-    uint32_t neg = 0;   // bit d: draw d below 1/2 (one copy of the draw's code)
-#pragma unroll 1
-    for (int d = 0; d < 6; ++d) neg |= (mz_rand(A.rp, st) < 0.5 ? 1u : 0u) << d;
     for (int d = 0; d < 3; ++d) {
-        dv[d] = (neg >> d) & 1 ? -1.0 : 1.0;
-        dx[d] = (neg >> (3 + d)) & 1 ? -1.0 : 1.0;
+        dv[d] = u[d] < 0.5 ? -1.0 : 1.0;
+        dx[d] = u[3 + d] < 0.5 ? -1.0 : 1.0;
     }
     const double w1 = 0.5 * Wb;
     for (int k = 0; k < 2; ++k) {
@@ -326,8 +317,6 @@ __device__ inline void oct_defer(const OctArgs &A, int c, int32_t N) {
 template <class IdxT, int NW, bool BIG, int PRE>
 __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, const int32_t N,
                                                const int32_t target_np, const OctWork<IdxT> &W, OctShared<PRE> &S) {
-    IdxT *const pis = W.pis;
-    IdxT *const psort = W.psort;
     uint8_t *const poct = W.poct;
     OctBinT<IdxT> *const bins = W.bins;
     double *const red = S.red;
@@ -348,14 +337,14 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             W.stg[3 * W.n_stg + i] = A.sp.v2[p];
         }
     } else {
-        for (int i = threadIdx.x; i < N; i += blockDim.x) pis[i] = (IdxT)i;
+        for (int i = threadIdx.x; i < N; i += blockDim.x) W.ord[i] = (IdxT)i;
     }
     double mn[3], mx[3];
     if (A.init_bounds == 3) {
         for (int d = 0; d < 3; ++d) { mn[d] = -299792458.0; mx[d] = 299792458.0; }
     } else {
-        __syncthreads();
-        oct_bounds<IdxT, NW>(A, pis, 0, N - 1, s1, n1, s2, mn, mx, red);
+        static_assert(sizeof(S.pre) >= 6 * NW * sizeof(double), "the bounds fit the splits' place");
+        oct_bounds<NW>(A, N, s1, n1, s2, mn, mx, reinterpret_cast<double *>(S.pre));
         if (A.init_bounds == 2) {
             for (int d = 0; d < 3; ++d) {
                 double m = fmax(fabs(mn[d]), fabs(mx[d]));
@@ -417,20 +406,19 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         const int bs = bins[b].start, be = bins[b].end;
         const int par = bins[b].depth & 1;
         if (A.bounds_mode == 2) {
-            double bmn[3], bmx[3];
-            for (int d = 0; d < 3; ++d) {
-                double lo = 9299792458.0, hi = -9299792458.0;
-                for (int i = bs + lane; i <= be; i += 64) {
-                    double w, x[3];
-                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, x[0], x[1], x[2]);
-                    lo = fmin(lo, x[d]);
-                    hi = fmax(hi, x[d]);
-                }
-                bmn[d] = mz_wave_min(lo);
-                bmx[d] = mz_wave_max(hi);
+            double lo0 = 9299792458.0, lo1 = lo0, lo2 = lo0, hi0 = -lo0, hi1 = -lo0, hi2 = -lo0;
+            for (int i = bs + lane; i <= be; i += 64) {
+                double w, x0, x1, x2;
+                oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, i, w, x0, x1, x2);
+                lo0 = fmin(lo0, x0); lo1 = fmin(lo1, x1); lo2 = fmin(lo2, x2);
+                hi0 = fmax(hi0, x0); hi1 = fmax(hi1, x1); hi2 = fmax(hi2, x2);
             }
-            if (lane == 0 && be >= bs)
-                for (int d = 0; d < 3; ++d) { bins[b].vmin[d] = bmn[d]; bins[b].vmax[d] = bmx[d]; }
+            lo0 = mz_wave_min(lo0); lo1 = mz_wave_min(lo1); lo2 = mz_wave_min(lo2);
+            hi0 = mz_wave_max(hi0); hi1 = mz_wave_max(hi1); hi2 = mz_wave_max(hi2);
+            if (lane == 0 && be >= bs) {
+                bins[b].vmin[0] = lo0; bins[b].vmin[1] = lo1; bins[b].vmin[2] = lo2;
+                bins[b].vmax[0] = hi0; bins[b].vmax[1] = hi1; bins[b].vmax[2] = hi2;
+            }
             oct_wave_sync();
         }
         if (lane < 3) {
@@ -453,7 +441,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
                 double nt = 0.0;
                 for (int i = bs; i <= be; ++i) {
                     double w, a0, a1, a2;
-                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, a0, a1, a2);
+                    oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, i, w, a0, a1, a2);
                     nt += w;
                     vel_mid[0] = vel_mid[0] + w * a0;
                     vel_mid[1] = vel_mid[1] + w * a1;
@@ -479,13 +467,13 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         double nw = 0.0, nv0 = 0.0, nv1 = 0.0, nv2 = 0.0;
         IdxT pi1 = 0;
         if (bs + lane <= be) {
-            pi1 = oct_id<IdxT, BIG>(W, pis, par, bs + lane);
-            oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, nw, nv0, nv1, nv2);
+            pi1 = oct_id<IdxT, BIG>(W, par, bs + lane);
+            oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, bs + lane, nw, nv0, nv1, nv2);
         }
         // the next chunk's ids, loaded a chunk ahead of its values (the
         // staged values need no ids)
         IdxT pin = 0;
-        if (!BIG && bs + 64 + lane <= be) pin = oct_id<IdxT, BIG>(W, pis, par, bs + 64 + lane);
+        if (!BIG && bs + 64 + lane <= be) pin = oct_id<IdxT, BIG>(W, par, bs + 64 + lane);
         int o1 = 0;
         for (int i0 = bs; i0 <= be; i0 += 64) {
             const int i = i0 + lane;
@@ -499,7 +487,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
                     nw = A.sp.w[p]; nv0 = A.sp.v0[p]; nv1 = A.sp.v1[p]; nv2 = A.sp.v2[p];
                 }
             }
-            if (!BIG && i + 128 <= be) pin = oct_id<IdxT, BIG>(W, pis, par, i + 128);
+            if (!BIG && i + 128 <= be) pin = oct_id<IdxT, BIG>(W, par, i + 128);
             int o = 0;
             if (i <= be) {
                 o = 1;
@@ -553,7 +541,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         // (earlier chunks, then earlier lanes of its chunk).
         const uint64_t lt = mz_lanemask_lt();
         const int oq = par ^ 1;
-        IdxT *const dsto = oq ? psort : pis;   // LDS path
+        IdxT *const dsto = BIG ? nullptr : W.ord + oq * OCT_MAX_N;   // LDS path
         if (one) {
             int dst = 0;
 #pragma unroll
@@ -574,9 +562,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             int rq[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
             // each chunk's octants and ids are loaded a chunk ahead
             int on = bs + lane <= be ? poct[bs + lane] : 0;
-            IdxT pn = bs + lane <= be ? oct_id<IdxT, BIG>(W, pis, par, bs + lane) : (IdxT)0;
+            IdxT pn = bs + lane <= be ? oct_id<IdxT, BIG>(W, par, bs + lane) : (IdxT)0;
             double qw = 0.0, qa = 0.0, qb = 0.0, qc = 0.0;
-            if (BIG && bs + lane <= be) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, qw, qa, qb, qc);
+            if (BIG && bs + lane <= be) oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, bs + lane, qw, qa, qb, qc);
             for (int i0 = bs; i0 <= be; i0 += 64) {
                 const int i = i0 + lane;
                 const bool valid = i <= be;
@@ -585,8 +573,8 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
                 const double vw = qw, va = qa, vb = qb, vc = qc;
                 const bool vn = i + 64 <= be;
                 on = vn ? poct[i + 64] : 0;
-                pn = vn ? oct_id<IdxT, BIG>(W, pis, par, i + 64) : (IdxT)0;
-                if (BIG && vn) oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i + 64, qw, qa, qb, qc);
+                pn = vn ? oct_id<IdxT, BIG>(W, par, i + 64) : (IdxT)0;
+                if (BIG && vn) oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, i + 64, qw, qa, qb, qc);
                 int dst = 0;
 #pragma unroll
                 for (int q = 1; q <= 8; ++q) {
@@ -658,8 +646,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         if (lane >= K0) ne_r = ref_r = add_r = 0;
         int sn = ne_r, sa = add_r, sr = ref_r;
         double sc = lane < K0 ? cr : -1.0;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
+        for (int o = 1; o < K0; o <<= 1) {
             const int y0 = __shfl_up(sn, o, 64), y1 = __shfl_up(sa, o, 64), y2 = __shfl_up(sr, o, 64);
             const double y3 = __shfl_up(sc, o, 64);
             if (lane >= o) { sn += y0; sa += y1; sr += y2; sc = fmax(sc, y3); }
@@ -767,68 +754,80 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
     for (;;) {
         const int n_ent = S.n_ent;
         if (n_ent == 0 || total_post_s + 14 > target_np) break;
-        // the heaviest bin, the lowest id on ties
-        double bw = -1.0;
-        int bid = 0x7FFFFFFF, ent = 0;
-        for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
-            const double kw = W.hkey[i];
-            const int ki = W.hid[i];
-            if (kw > bw || (kw == bw && ki < bid)) { bw = kw; bid = ki; ent = i; }
-        }
-        {
-            const double mw = mz_wave_max(bw);
-            const int mi = mz_wave_min_i32(bw == mw ? bid : 0x7FFFFFFF);
-            const uint64_t m = __ballot(bw == mw && bid == mi);
-            const int me = __builtin_amdgcn_readlane(ent, m ? __builtin_ctzll(m) : 0);
-            if (lane == 0) { red[wv] = mw; S.rid[wv] = mi; S.rent[wv] = me; }
-        }
-        __syncthreads();
-        double mw = red[0];
-        int mi = S.rid[0], e_pick = S.rent[0];
-#pragma unroll
-        for (int k = 1; k < NW; ++k)
-            if (red[k] > mw || (red[k] == mw && S.rid[k] < mi)) { mw = red[k]; mi = S.rid[k]; e_pick = S.rent[k]; }
-        if (!(mw > -1.0)) break;   // weights that do not compare
-        const bool fresh = W.hst[e_pick] == 0;   // not split yet
-        if (threadIdx.x == 0) {
-            S.list[0] = e_pick;
-            S.n_list = fresh ? 1 : 0;
-            S.dropped = 0;
-        }
-        __syncthreads();
-        // the list; one entry of pre is kept free for the next heaviest bin
         const uint64_t free = S.pre_free;
-        const int room = A.split != 1 ? (fresh ? 1 : 0)
-                                      : min(__popcll(free) - 1, (target_np - total_post_s) / 6 + 1);
-        const double thr = share * mw;
-        for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
-            const double kw = W.hkey[i];
-            if (kw >= thr && i != e_pick && W.hst[i] == 0) {
-                const int at = atomicAdd(&S.n_list, 1);
-                if (at < room) S.list[at] = i;
-                else atomicMax(&S.dropped, (unsigned long long)__double_as_longlong(kw));
+        double mw;
+        int e_pick = 0, n_all, n_list;
+        bool fresh;
+        if (n_ent == 1) {   // the first split of every cell: no search, no list
+            mw = W.hkey[0];
+            if (!(mw > -1.0)) break;   // weights that do not compare
+            fresh = W.hst[0] == 0;
+            n_all = n_list = fresh ? 1 : 0;
+            __syncthreads();   // every wave has read before wave 0 writes
+        } else {
+            // the heaviest bin, the lowest id on ties
+            double bw = -1.0;
+            int bid = 0x7FFFFFFF, ent = 0;
+            for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
+                const double kw = W.hkey[i];
+                const int ki = W.hid[i];
+                if (kw > bw || (kw == bw && ki < bid)) { bw = kw; bid = ki; ent = i; }
             }
+            {
+                const double wm = mz_wave_max(bw);
+                const int wi = mz_wave_min_i32(bw == wm ? bid : 0x7FFFFFFF);
+                const uint64_t m = __ballot(bw == wm && bid == wi);
+                const int we = __builtin_amdgcn_readlane(ent, m ? __builtin_ctzll(m) : 0);
+                if (lane == 0) { red[wv] = wm; S.rid[wv] = wi; S.rent[wv] = we; }
+            }
+            if (threadIdx.x == 0) {
+                S.n_list = 0;
+                S.dropped = 0;
+            }
+            __syncthreads();
+            mw = red[0];
+            int mi = S.rid[0];
+            e_pick = S.rent[0];
+#pragma unroll
+            for (int k = 1; k < NW; ++k)
+                if (red[k] > mw || (red[k] == mw && S.rid[k] < mi)) { mw = red[k]; mi = S.rid[k]; e_pick = S.rent[k]; }
+            if (!(mw > -1.0)) break;
+            fresh = W.hst[e_pick] == 0;   // not split yet
+            // the list of the others; one entry of pre is kept free for the next heaviest bin
+            const int first = fresh ? 1 : 0;
+            const int room = A.split != 1 ? first : min(__popcll(free) - 1, (target_np - total_post_s) / 6 + 1);
+            const double thr = share * mw;
+            for (int i = threadIdx.x; i < n_ent; i += NW * 64) {
+                const double kw = W.hkey[i];
+                if (kw >= thr && i != e_pick && W.hst[i] == 0) {
+                    const int at = first + atomicAdd(&S.n_list, 1);
+                    if (at < room) S.list[at] = i;
+                    else atomicMax(&S.dropped, (unsigned long long)__double_as_longlong(kw));
+                }
+            }
+            __syncthreads();
+            n_all = first + S.n_list;
+            n_list = max(first, min(n_all, room));
         }
-        __syncthreads();
-        const int n_all = S.n_list, n_list = max(fresh ? 1 : 0, min(n_all, room));
-        const double dropped = __longlong_as_double((long long)S.dropped);
+        const bool over = n_all > n_list;
+        const double bound = over ? __longlong_as_double((long long)S.dropped) : share * mw;
         for (int k = wv; k < n_list; k += NW) {
             uint64_t f = free;   // the k-th free entry
             for (int j = 0; j < k; ++j) f &= f - 1;
-            split(__builtin_amdgcn_readfirstlane(S.list[k]), __builtin_ctzll(f));
+            split(k == 0 && fresh ? e_pick : __builtin_amdgcn_readfirstlane(S.list[k]), __builtin_ctzll(f));
         }
-        __syncthreads();
+        if (n_list > 1) __syncthreads();   // one split is wave 0's own
         if (wv == 0) {
             uint64_t f = free;
             for (int j = 0; j < n_list; ++j) f &= f - 1;
             if (lane == 0) S.pre_free = f;
             oct_wave_sync();
             // bins not split: lighter than thr, or at most as heavy as `dropped`
-            take(e_pick, n_all > n_list ? dropped : thr, n_all <= n_list);
+            take(e_pick, bound, !over);
         }
         // a list that overflows leaves bins out that come before listed ones: a
         // narrower share then, a wider one while half the places stay empty
-        share = n_all > n_list ? 1.0 - 0.7 * (1.0 - share) : (2 * n_all < PRE ? fmax(0.25, 1.0 - 1.2 * (1.0 - share)) : share);
+        share = over ? 1.0 - 0.7 * (1.0 - share) : (2 * n_all < PRE ? fmax(0.25, 1.0 - 1.2 * (1.0 - share)) : share);
         __syncthreads();
         if (stop_s) break;
     }
@@ -848,7 +847,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
     if (Nbins == 1 && threadIdx.x == 0) {
         double s = 0.0;
         const int par0 = bins[0].depth & 1;
-        for (int i = 0; i < N; ++i) s += A.sp.w[oct_slot(oct_id<IdxT, BIG>(W, pis, par0, i), s1, n1, s2)];
+        for (int i = 0; i < N; ++i) s += A.sp.w[oct_slot(oct_id<IdxT, BIG>(W, par0, i), s1, n1, s2)];
         bins[0].w = s;
     }
     __syncthreads();
@@ -919,8 +918,8 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             const bool on = bs + lane <= be;
             double w = 0.0, u0 = 0.0, u1 = 0.0, u2 = 0.0, y0 = 0.0, y1 = 0.0, y2 = 0.0;
             if (on) {
-                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, pis, par, bs + lane), s1, n1, s2);
-                oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + lane, w, u0, u1, u2);
+                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, par, bs + lane), s1, n1, s2);
+                oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, bs + lane, w, u0, u1, u2);
                 y0 = A.sp.x0[p]; y1 = A.sp.x1[p]; y2 = A.sp.x2[p];
             }
             vm[0] = mz_wave_sum(on ? w * u0 : 0.0) * inv_w;
@@ -949,9 +948,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             for (int i = bs + lane + 64 * q; i <= be; i += 256) {
-                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, pis, par, i), s1, n1, s2);
+                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, par, i), s1, n1, s2);
                 double w, u0, u1, u2;
-                oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, u0, u1, u2);
+                oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, i, w, u0, u1, u2);
                 sv[q][0] = fma(w, u0, sv[q][0]); sv[q][1] = fma(w, u1, sv[q][1]);
                 sv[q][2] = fma(w, u2, sv[q][2]);
                 sx[q][0] = fma(w, A.sp.x0[p], sx[q][0]); sx[q][1] = fma(w, A.sp.x1[p], sx[q][1]);
@@ -972,9 +971,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             for (int i = bs + lane + 64 * q; i <= be; i += 256) {
-                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, pis, par, i), s1, n1, s2);
+                const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, par, i), s1, n1, s2);
                 double w, u0, u1, u2;
-                oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, i, w, u0, u1, u2);
+                oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, i, w, u0, u1, u2);
                 const double a0 = u0 - vm[0], a1 = u1 - vm[1], a2 = u2 - vm[2];
                 const double e0 = A.sp.x0[p] - xm[0], e1 = A.sp.x1[p] - xm[1], e2 = A.sp.x2[p] - xm[2];
                 sv[q][0] = fma(w, a0 * a0, sv[q][0]); sv[q][1] = fma(w, a1 * a1, sv[q][1]);
@@ -993,9 +992,10 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         if (lane == 0) oct_emit(A, c, bdraw[b], bslot[b], Wb, vm, xm, sdv, sdx, s1, n1, s2);
     };
     // compute_bin_props! and compute_new_particles! per bin.  With at least
-    // LANE_BINS bins (whatever the number of waves, so the sums are the same) a bin of at most OCT_LANE_NP particles takes one lane, its
-    // sums in particle order (the reference's order), and a larger bin the whole
-    // wavefront; with fewer bins the waves take the bins in turn.
+    // LANE_BINS bins (whatever the number of waves, so the sums are the same) a
+    // bin of at most OCT_LANE_NP particles takes one lane, its sums in particle
+    // order (the reference's order), and a larger bin the whole wavefront; with
+    // fewer bins the waves take the bins in turn.
     if (Nbins < LANE_BINS) {
         for (int b = wv; b < Nbins; b += NW) {
             const int32_t bnp = bins[b].w == 0.0 ? 0 : (int32_t)bins[b].np;
@@ -1003,7 +1003,7 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             if (bnp <= 2) {
                 const int bs = bins[b].start, par = bins[b].depth & 1;
                 if (lane < bnp)
-                    oct_copy(A, oct_slot(oct_id<IdxT, BIG>(W, pis, par, bs + lane), s1, n1, s2),
+                    oct_copy(A, oct_slot(oct_id<IdxT, BIG>(W, par, bs + lane), s1, n1, s2),
                              oct_slot(bslot[b] + lane, s1, n1, s2));
                 continue;
             }
@@ -1025,16 +1025,16 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
         const int slot = lone ? bslot[bl] : 0;
         if (lone && bnp <= 2)
             for (int j = 0; j < bnp; ++j)
-                oct_copy(A, oct_slot(oct_id<IdxT, BIG>(W, pis, par, bs + j), s1, n1, s2), oct_slot(slot + j, s1, n1, s2));
+                oct_copy(A, oct_slot(oct_id<IdxT, BIG>(W, par, bs + j), s1, n1, s2), oct_slot(slot + j, s1, n1, s2));
         const bool sums = lone && bnp > 2;
         const int jn = (int)mz_wave_max(sums ? (double)bnp : 0.0);
         if (jn > 0) {
             double vm[3] = {0.0, 0.0, 0.0}, xm[3] = {0.0, 0.0, 0.0};
             for (int j = 0; j < jn; ++j) {
                 if (sums && j < bnp) {
-                    const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, pis, par, bs + j), s1, n1, s2);
+                    const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, par, bs + j), s1, n1, s2);
                     double w, a0, a1, a2;
-                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + j, w, a0, a1, a2);
+                    oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, bs + j, w, a0, a1, a2);
                     vm[0] = vm[0] + w * a0; vm[1] = vm[1] + w * a1; vm[2] = vm[2] + w * a2;
                     xm[0] = xm[0] + w * A.sp.x0[p]; xm[1] = xm[1] + w * A.sp.x1[p]; xm[2] = xm[2] + w * A.sp.x2[p];
                 }
@@ -1044,9 +1044,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
             double vs[3] = {0.0, 0.0, 0.0}, xs[3] = {0.0, 0.0, 0.0};
             for (int j = 0; j < jn; ++j) {
                 if (sums && j < bnp) {
-                    const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, pis, par, bs + j), s1, n1, s2);
+                    const int64_t p = oct_slot(oct_id<IdxT, BIG>(W, par, bs + j), s1, n1, s2);
                     double w, u0, u1, u2;
-                    oct_ld<IdxT, BIG>(A, W, pis, s1, n1, s2, par, bs + j, w, u0, u1, u2);
+                    oct_ld<IdxT, BIG>(A, W, s1, n1, s2, par, bs + j, w, u0, u1, u2);
                     const double a0 = u0 - vm[0], a1 = u1 - vm[1], a2 = u2 - vm[2];
                     const double e0 = A.sp.x0[p] - xm[0], e1 = A.sp.x1[p] - xm[1], e2 = A.sp.x2[p] - xm[2];
                     vs[0] = vs[0] + w * (a0 * a0); vs[1] = vs[1] + w * (a1 * a1); vs[2] = vs[2] + w * (a2 * a2);
@@ -1084,8 +1084,7 @@ __device__ inline bool oct_pick(const OctArgs &A, int c, int32_t &N, int32_t &ta
 
 // One workgroup per cell, the working arrays in LDS.
 __global__ void __launch_bounds__(256) k_octree_merge(OctArgs A) {
-    __shared__ int16_t pis[OCT_MAX_N];
-    __shared__ int16_t psort[OCT_MAX_N];
+    __shared__ int16_t ord[2 * OCT_MAX_N];
     __shared__ __align__(16) uint8_t poct[OCT_MAX_N];   // after the splits: per-bin slots and draws
     __shared__ OctBin bins[OCT_MAX_BINS];
     __shared__ double hkey[OCT_MAX_BINS];
@@ -1104,7 +1103,7 @@ __global__ void __launch_bounds__(256) k_octree_merge(OctArgs A) {
         return;
     }
     OctWork<int16_t> W;
-    W.pis = pis; W.psort = psort; W.poct = poct; W.bins = bins;
+    W.ord = ord; W.poct = poct; W.bins = bins;
     W.hkey = hkey; W.hid = hid; W.hst = hst;
     static_assert(2 * OCT_MAX_BINS * sizeof(int16_t) <= OCT_MAX_N, "the slots and draws fit the octants");
     W.bslot = reinterpret_cast<int16_t *>(poct);
@@ -1136,10 +1135,9 @@ __global__ void __launch_bounds__(WAVES * 64) k_octree_merge_big(OctArgs A) {
     const int32_t n_list = A.big_info[0];
     const size_t g = blockIdx.x;
     OctWork<int32_t> W;
-    W.pis = A.big_pis + g * (size_t)A.big_ncap;
-    W.psort = A.big_psort + g * (size_t)A.big_ncap;
-    W.sid0 = W.pis;
-    W.sid_q = W.psort - W.pis;
+    W.ord = nullptr;
+    W.sid0 = A.big_pis + g * (size_t)A.big_ncap;
+    W.sid_q = A.big_psort - A.big_pis;
     W.stg = A.big_stage + g * (size_t)A.big_ncap * 8;
     W.n_stg = A.big_ncap;
     W.poct = A.big_poct + g * (size_t)A.big_ncap;
