@@ -581,25 +581,36 @@ __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(Slab
         if (tid < SLAB_MAXC) { runL[tid] = 0; runR[tid] = 0; }
         if (HIT_LIST && tid == 0) s_hits = 0;
         if (SNAP && t > 0 && props_due(t - 1)) props_cells();
-        if (WAVE_NTC) {
-            MzRngParams rp = A.rp;
-            rp.tag = (step << 4) | 1u;
+        MzRngParams rpn = A.rp;
+        rpn.tag = (step << 4) | 1u;
+        // Large averaging slabs have four waves for up to 32 cells, and their
+        // cells often a candidate or none: a wave whose cells have at most twice
+        // as many candidates as it has cells with any takes them on lanes, side by
+        // side (us per step, waves / lanes: 10 cells of 60 particles, a quarter
+        // of a candidate each, 14.0 / 11.7; one cell of 500, 11 candidates, 14.1 /
+        // 20.8).
+        bool on_lanes = !WAVE_NTC;
+        if (WAVE_NTC && AVG) {
+            double e = 0.0;
+            if (ntc_lane)
+                e = floor(mz_ncoll_est(true, A.dt, ccn[my_k], ccn[my_k], my_sgwm, my_V, sdraw[my_k * nd]));
+            on_lanes = !__ballot(e > 2.0 * __popcll(__ballot(e > 0.0)));
+        }
+        if (WAVE_NTC && !on_lanes) {
             for (int k = wave, l = 0; k < ncl; k += NW, ++l) {   // its values on lane l
                 const int32_t nla = ccn[k];
                 double sg = mz_readlane_d(my_sgwm, l);
                 int32_t nc_, pf_, eq_;
-                slab_ntc_cell_wave(A, rp, clo + k, mz_readlane_d(my_V, l), cst[k], nla, sv0, sv1, sv2, sw,
+                slab_ntc_cell_wave(A, rpn, clo + k, mz_readlane_d(my_V, l), cst[k], nla, sv0, sv1, sv2, sw,
                                    sdraw + k * nd, nd, ntc_tracks, sg, nc_, pf_, eq_);
                 if (lane == l) {
                     my_sgwm = sg;
                     my_nla = nla; my_ncoll = nc_; my_perf = pf_; my_eqw = eq_;
                 }
             }
-        } else if (ntc_lane) {
-            MzRngParams rp = A.rp;
-            rp.tag = (step << 4) | 1u;
+        } else if (on_lanes && ntc_lane) {
             my_nla = ccn[my_k];
-            slab_ntc_cell(A, rp, clo + my_k, my_V, cst[my_k], my_nla, sv0, sv1, sv2, sw, sdraw + my_k * nd, my_sgwm,
+            slab_ntc_cell(A, rpn, clo + my_k, my_V, cst[my_k], my_nla, sv0, sv1, sv2, sw, sdraw + my_k * nd, my_sgwm,
                           my_ncoll, my_perf, my_eqw);
         }
         if (wall_side >= 0 && wave >= wall_w0) wall_draws(step);

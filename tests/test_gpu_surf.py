@@ -348,3 +348,45 @@ def test_couette_avg_steps_vs_oracle(hip, mzo, mode):
     assert avg.np.sum() > 0
     _compare(sa, avg.q, np.array([0.0, flux, flux] + [mom] * 7 + [ke]))
     st.close()
+
+
+@pytest.mark.parametrize("n_cells,ppc,dt,sgwm_mult,shape", [
+    (6, 250, 1e-9, 1.0, (1, 4)), (6, 600, 1e-9, 4.0, (1, 8)), (40, 60, 5e-10, 1.0, (10, 4)), (40, 60, 5e-10, 30.0, (10, 4)),
+    (50, 50, 5e-10, 8.0, (20, 8)), (5, 400, 1e-9, 0.3, (2, 8))])
+def test_large_avg_slabs_equal_graph(hip, mzo, n_cells, ppc, dt, sgwm_mult, shape):
+    """Averaging slabs of more than 512 particles (candidates in windows of a
+    wavefront, or cells of few of them on lanes; wall draws ahead, wall records)
+    against the step graph: particles, collision factors and averaged properties
+    bit for bit, wall averages equal to rounding."""
+    steps = 60
+    case = helpers.couette_case(mzo, n_cells=n_cells, ppc=ppc, seed=n_cells, dt=dt, sgwm_mult=sgwm_mult, dx=1e-5)
+    a, b = helpers.store_from_case(hip, case), helpers.store_from_case(hip, case)
+    b.set_slab_shape(*shape)
+    for st, mode in ((a, "graph"), (b, "slab")):
+        st.surf_clear(1)
+        st.props_avg_clear()
+        path = hip.couette_avg_steps(st, steps, 3, dt, steps, species_data=case["species"], mode=mode)
+        assert path == mode, st.slab_info()
+    assert b.slab_info()[0] >= 4
+    da, db = a.download_species(1), b.download_species(1)
+    n = da["n_total"]
+    assert da["err"] == 0 and db["err"] == 0
+    assert np.array_equal(da["pia"], db["pia"]) and np.array_equal(da["index"][:n], db["index"][:n])
+    for k in ("x", "v", "w"):
+        assert np.array_equal(da[k][:n], db[k][:n]), k
+    ca, cb = a.collision_factors(1, 1), b.collision_factors(1, 1)
+    for k in ca:
+        assert np.array_equal(ca[k], cb[k]), k
+    assert ca["n_coll"].sum() > 0
+    pa, pb = hip.PhysProps(n_cells, 1).fetch_avg(a), hip.PhysProps(n_cells, 1).fetch_avg(b)
+    for k in ("lpa", "np", "n", "v", "T"):
+        assert np.array_equal(getattr(pa, k), getattr(pb, k)), k
+    sa = hip.SurfProps.grid1d(1).fetch(a, 1)._to_device()[0]
+    sb = hip.SurfProps.grid1d(1).fetch(b, 1)._to_device()[0]
+    assert np.array_equal(sa[:, 0], sb[:, 0]) and sa[:, 0].min() > 0
+    for e in range(2):
+        mom = np.abs(sa[e, 3:10]).sum()
+        bound = np.array([0.0, sa[e, 1], sa[e, 1]] + [mom] * 7 + [np.abs(sa[e, 10]) + sa[e, 6] * 1000.0])
+        assert np.all(np.abs(sa[e] - sb[e]) <= 1e-10 * bound), (e, sa[e], sb[e])
+    a.close()
+    b.close()
