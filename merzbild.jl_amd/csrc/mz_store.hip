@@ -1104,8 +1104,8 @@ static bool sort_uses_radix(const mz_store *h, const MzSpecies &s) {
 // bounds its interface states.
 static bool sort_noalloc_fits(const mz_store *h, const MzSpecies &s) {
     const int64_t nchunks = (s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK;
-    return h->sort_path != 2 && (h->sort_path == 1 || (h->n_cells <= MZ_SORT_MAX_CELLS &&
-                                                       (int64_t)h->n_cells * nchunks <= 8 * s.cap));
+    return h->sort_path != 2 && h->n_cells <= MZ_SORT_MAX_CELLS &&
+           (h->sort_path == 1 || (int64_t)h->n_cells * nchunks <= 8 * s.cap);
 }
 
 struct RsScratch {
@@ -1300,6 +1300,8 @@ extern "C" int mz_sort_noalloc(mz_store *h, int32_t species, int32_t compute_cel
              "chunks <= 8 x capacity, sort path not radix)");
     const int64_t nc = h->n_cells;
     const int64_t nchunks = (s.cap + MZ_SORT_CHUNK - 1) / MZ_SORT_CHUNK;
+    // the matrix alone takes nc * nchunks; the bound keeps the nc words more that
+    // the interface states
     const int64_t need = std::max<int64_t>(nc * nchunks + nc, 2 * nc);
     MZ_CHECK(need <= MZ_NOALLOC_SCRATCH_WORDS,
              "sort_noalloc: n_cells x (chunks + 1) exceeds the fixed scratch of 2^21 int32 words (8 MiB); "

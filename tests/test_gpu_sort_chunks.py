@@ -43,3 +43,25 @@ def test_sort_chunks_vs_oracle(hip, mzo, n, nc, cap, nearly):
         helpers.assert_state_matches(mzo, got, pv, pia, rtol=0.0, check_buffer=False)
         assert np.array_equal(got["cell"], pv.cell[:n])
     st.close()
+
+
+def test_forced_matrix_refuses_more_cells_than_it_states(hip):
+    """14,336 cells at most where a caller asks for the count matrix, with and
+    without allocating."""
+    for nc in (14336, 14337):
+        st = hip.DeviceStore(nc, 1, 64)
+        pia = np.zeros((nc, 7), dtype=np.int64)
+        pia[:, 2] = pia[:, 5] = -1
+        pia[0] = [3, 1, 3, 3, 0, -1, 0]
+        x = np.array([[nc - 0.5, 0, 0], [0.5, 0, 0], [7.5, 0, 0]])
+        st.upload_species(1, x, np.zeros((3, 3)), np.ones(3), np.arange(1, 4), pia, 3, True, None, 3)
+        st.set_grid(hip.Grid1DUniform(float(nc), nc))
+        st.set_sort_path("matrix")
+        for sort in (hip.sort_particles, hip.sort_particles_noalloc):
+            if nc > 14336:
+                with pytest.raises(hip.MzError):
+                    sort(st, 1)
+            else:
+                sort(st, 1)
+                assert list(st.download_species(1)["index"]) == [2, 3, 1]
+        st.close()
