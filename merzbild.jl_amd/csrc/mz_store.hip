@@ -190,10 +190,10 @@ extern "C" int mz_create(int32_t n_cells, int32_t n_species, const int64_t *capa
     MZ_HIP(hipMalloc(&h->d_err, sizeof(int32_t)));
     MZ_HIP(hipMemset(h->d_err, 0, sizeof(int32_t)));
     const size_t ncp = ((size_t)n_cells + 15) & ~(size_t)15;
-    MZ_HIP(hipMalloc(&h->d_ccount, (2 * ncp + 16) * sizeof(int32_t)));
+    MZ_HIP(hipMalloc(&h->d_ccount, (2 * ncp + 16) * sizeof(int32_t) + (size_t)(n_cells + 63) / 64 * sizeof(uint64_t)));
     MZ_HIP(hipMemset(h->d_ccount, 0, ncp * sizeof(int32_t)));
     h->d_cstart = h->d_ccount + ncp;
-    MZ_HIP(hipMalloc(&h->d_ntc_left, (size_t)(n_cells + 63) / 64 * sizeof(uint64_t)));
+    h->d_ntc_left = (uint64_t *)(h->d_cstart + ncp + 16);
     size_t pn = (size_t)n_species * n_cells;
     MZ_HIP(hipMalloc(&h->d_np, pn * sizeof(double)));
     MZ_HIP(hipMalloc(&h->d_n, pn * sizeof(double)));
@@ -266,7 +266,7 @@ extern "C" int mz_destroy(mz_store *h) {
     if (h->h_report) hipHostFree(h->h_report);
     mz_graph_release(h);
     for (auto &s : h->sp) free_species(s);
-    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ccount); hipFree(h->d_ntc_left);
+    hipFree(h->d_sgwm); hipFree(h->d_cfcnt); hipFree(h->d_err); hipFree(h->d_ccount);
     hipFree(h->d_np); hipFree(h->d_n); hipFree(h->d_T); hipFree(h->d_v); hipFree(h->d_V);
     hipFree(h->d_invV);
     hipFree(h->d_masses);
@@ -2019,16 +2019,17 @@ extern "C" int mz_get_flux(mz_store *h, int32_t which, double *kinetic_energy_fl
 // What bounds it: the powers (a pow of each particle's speed per moment) on
 // the one wave of the largest cell.  With cells so few that their workgroups run
 // together, a workgroup takes a cell: all of its waves where it has more than
-// MOMENTS_JOINT_NP particles, else one, since the sums across the waves then cost
-// more than they save.  us a call with three moments, wave / workgroup a cell: 1
-// cell of 100 particles 9.1 / 9.5, of 300 13.8 / 10.6, of 20,000 511 / 136; 500
-// cells of 20 8.5 / 8.8, of 300 15.8 / 12.7, of 5,000 173 / 79.  4,096 cells of 3
-// 14.0 / 16.4, of 300 39 / 51, of 1,200 134 / 129: they fill the chip with a wave
-// each.
+// joint_np particles, else one, since the sums across the waves then cost more
+// than they save.  us a call with three moments, a wave a cell / this rule's two
+// ways: 1 cell of 100 particles 9.1 / 9.5, of 300 13.8 / 10.6, of 20,000 511 / 136;
+// 500 cells of 20 8.5 / 8.8, of 300 15.8 / 12.7, of 5,000 173 / 79; 1,024 cells of
+// 300 16.2, on all waves 17.5, of 600 25.6 / 24.6, of 5,000 182 / 142.  Past 1,024
+// cells a wave each fills the chip: 2,048 of 20 9.8 / 11.8, of 300 23 / 29, of
+// 1,200 75 / 71; 4,096 of 300 39 / 51, of 1,200 135 / 132.
 #define MOMENTS_JOINT_CELLS 1024
-#define MOMENTS_JOINT_NP 256
+static int32_t moments_joint_np(int64_t cells) { return cells <= 512 ? 256 : 512; }
 template <int WAVES>
-__global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_cells, int32_t n_mom,
+__global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_cells, int32_t joint_np, int32_t n_mom,
                                                        const int32_t *__restrict__ powers,
                                                        const double *__restrict__ scale,   // [species][n_mom]
                                                        const double *__restrict__ masses, double *__restrict__ out_np,
@@ -2041,7 +2042,7 @@ __global__ void __launch_bounds__(256) k_props_moments(MzViews views, int32_t n_
     const int32_t st1 = sp.pia.start1[c] - 1, n1 = sp.pia.n1[c];
     const int32_t st2 = sp.pia.start2[c] - 1, n2 = sp.pia.n2[c] > 0 ? sp.pia.n2[c] : 0;
     const int32_t tot = n1 + n2;
-    const bool joint = WAVES > 1 && tot > MOMENTS_JOINT_NP;
+    const bool joint = WAVES > 1 && tot > joint_np;
     if (WAVES > 1 && !joint && threadIdx.x >= 64) return;
     const int lane = joint ? (int)threadIdx.x : (int)(threadIdx.x & 63);   // among the cell's threads
     const int step = joint ? 64 * WAVES : 64;
@@ -2130,13 +2131,14 @@ extern "C" int mz_compute_props_moments(mz_store *h, const int32_t *powers, int3
     h->masses_valid = false;   // the couette drivers upload their mass again
     {
         MzTimed tm(h, "props");
-        if ((int64_t)h->n_cells * ns <= MOMENTS_JOINT_CELLS)
+        const int64_t cells = (int64_t)h->n_cells * ns;
+        if (cells <= MOMENTS_JOINT_CELLS)
             hipLaunchKernelGGL(k_props_moments<4>, dim3(h->n_cells, ns), dim3(256), 0, h->stream, mz_views(h),
-                               h->n_cells, n_moments, d_pow, d_sc, h->d_masses, h->d_np, h->d_n, h->d_v, h->d_T,
-                               d_m);
+                               h->n_cells, moments_joint_np(cells), n_moments, d_pow, d_sc, h->d_masses, h->d_np,
+                               h->d_n, h->d_v, h->d_T, d_m);
         else
             hipLaunchKernelGGL(k_props_moments<1>, dim3((h->n_cells + 3) / 4, ns), dim3(256), 0, h->stream,
-                               mz_views(h), h->n_cells, n_moments, d_pow, d_sc, h->d_masses, h->d_np, h->d_n,
+                               mz_views(h), h->n_cells, 0, n_moments, d_pow, d_sc, h->d_masses, h->d_np, h->d_n,
                                h->d_v, h->d_T, d_m);
         MZ_HIP(hipGetLastError());
     }

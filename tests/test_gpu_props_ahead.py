@@ -63,11 +63,12 @@ def test_moments_wave_and_workgroup_per_cell(hip):
         assert np.allclose(a, b, rtol=1e-12, atol=atol, equal_nan=True)
 
 
-def test_moments_of_cells_on_one_and_all_waves_of_a_workgroup(hip):
-    """1,020 cells, a workgroup each, of which those of more than 256 particles use
-    all its waves, against numpy in long double: sums of up to 1,500 positive
-    terms, and a power of a ulp or two each."""
-    counts = np.array([256, 257, 1500, 0, 1, 255, 320, 2] + [9] * 1012)
+@pytest.mark.parametrize("more", [0, 1012])
+def test_moments_of_cells_on_one_and_all_waves_of_a_workgroup(hip, more):
+    """1,020 cells, and 8, a workgroup each, of which those of more than 512 (256)
+    particles use all its waves, against numpy in long double: sums of up to 1,500
+    positive terms, and a power of a ulp or two each."""
+    counts = np.array([256, 257, 1500, 512, 513, 0, 1, 255] + [9] * more)
     nc, n = len(counts), int(counts.sum())
     rng = np.random.default_rng(6)
     v, w = rng.normal(50.0, 300.0, size=(n, 3)), rng.uniform(0.5, 2.0, n)
