@@ -374,8 +374,9 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
     // compute_octree! (merging_octree_N2.jl:998-1039): the heaviest bin that
     // may be refined (the lowest id on ties) is split until the target is met.
     // What a split makes of a bin does not depend on the splits of other bins,
-    // and no child is heavier than its parent, so the order's weights only
-    // fall.  The bins are therefore split ahead of the order, in rounds:
+    // and no child is heavier than its parent (but for the rounding of its sum,
+    // which the comparison with the children below covers), so the order's
+    // weights only fall.  The bins are therefore split ahead of the order, in rounds:
     //   - all waves find the heaviest bin, and list it and the other bins of
     //     at least a share f of its weight that are not split yet;
     //   - all waves split the listed bins, one bin a wave at a time, into
@@ -394,7 +395,8 @@ __device__ __forceinline__ void oct_merge_cell(const OctArgs &A, const int c, co
     // against one wave splitting each bin as it is picked: 1,024 cells of 20 to
     // 30,000 particles, about 120 merged (the largest in 2,194 splits, 66 rounds,
     // 3.6 ms), 14.9 -> 3.5 ms a call with eight waves a cell for one; 1,850
-    // boxes of 1,300 particles to 1,000 (89 splits, 16 rounds) 1.02 -> 0.72 ms.
+    // boxes of 1,300 particles to 1,000 (89 splits, 16 rounds) 1.02 -> 0.61 ms;
+    // 5,000 cells of 60 to 20 (one split) 195 -> 186 us, of 300 to 64 529 -> 482.
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 

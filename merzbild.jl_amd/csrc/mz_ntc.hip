@@ -342,13 +342,13 @@ struct NtcWaveDraw {
 // What bounds it: the latency of one window (draw exchange, the two gathers,
 // the power chain; about 4 us) times the windows of the cell with the most.
 // Few acceptances make windows of 40 candidates, many make eight tracks of
-// eight.  Measured against one lane per cell, and against windows that ended
-// at every split: 8,192 boxes of 90 particles with 130 candidates, 8% accepted,
-// 4,030 -> 300 us a call; 2,048 boxes with 580 candidates (up to 3,500), 4%
-// accepted, SWPM, 5,560 -> 200 us; 4,096 boxes with 150 candidates, 39%
-// accepted, SWPM, 1,220 -> 190 us; 1,024 cells of up to 30,000 particles, 290
-// candidates (up to 2,900), 40% accepted, 3,250 -> 1,320 us; 500 cells of 35
-// candidates, 5% accepted, 46 -> 22 us.
+// eight.  Measured against one lane per cell, and (the last two) against windows
+// that ended at every split, in states of 50 passes and more: 8,192 boxes of 90
+// particles with 130 candidates, 8% accepted, 4,030 -> 310 us a call; 2,048 boxes
+// with 580 candidates (up to 3,500), 4% accepted, SWPM, 5,560 -> 270 us; 4,096
+// boxes with 150 candidates, 39% accepted, SWPM, 1,220 -> 270 us; 1,024 cells of up
+// to 30,000 particles, 290 candidates (up to 2,900), 40% accepted, 3,250 -> 710 us;
+// 500 cells of 35 candidates, 5% accepted, 46 -> 19 us.
 #define NTC_T1_LEN 40   // candidates of a single track (its draws fit the 128 held)
 
 enum { NTC_PLAIN = 0, NTC_SPLIT = 1, NTC_SWPM = 2 };   // no particles created; ntc! with splitting; swpm!
@@ -947,9 +947,9 @@ extern "C" int mz_ntc_cells(mz_store *h, int32_t s1, int32_t s2, double dt, cons
 
 // ===========================================================================
 // swpm! (collision_swpm.jl:201-288): single-species collisions of
-// variable-weight particles.  One lane per cell, as NTC: the loop is
-// sequential (the running (sigma g)_max, and particles created by the loop
-// are candidates of the same loop).  An accepted pair gives up
+// variable-weight particles.  A cell's loop is sequential (the running
+// (sigma g)_max, and particles created by the loop are candidates of the same
+// loop) and runs as NTC's do: in windows of a wavefront, or on a lane.  An accepted pair gives up
 // min(w_i, w_k) / (1 + G) of each weight to two new particles at the pair's
 // positions, which then take the pair's post-collision velocities
 // (scatter_vhs!); the pair keeps its velocities.  Created particles go to

@@ -324,7 +324,7 @@ __device__ inline void slab_ntc_cell_wave(const SlabArgs &A, const MzRngParams &
 // threads, two workgroups per CU; larger ones 512 (256 in the averaging
 // phase), one workgroup per CU (50 cells of 1,000 particles, us per step of a
 // slab: convection and ranking 5.6 -> 1.7, mailbox 2.7 -> 1.8, scatter 1.4 ->
-// 0.9; the whole step 65 -> 22 with the windows and the list of wall hits).
+// 0.9; the whole step 65 -> 20 with the windows and the list of wall hits).
 template <int R, bool AVG, int NT>
 __global__ void __launch_bounds__(NT, R * NT <= 512 ? 2 : 1) k_slab_couette(SlabArgs A) {
     constexpr int P = R * NT;             // LDS particle capacity
