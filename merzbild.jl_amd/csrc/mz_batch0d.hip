@@ -352,7 +352,7 @@ __global__ void __launch_bounds__(256, 2) k_batch0d(B0Args A) {
                         const int64_t p = i < jn1 ? (int64_t)jst1 + i : (int64_t)jst2 + (i - jn1);
                         b0_get(A.aos, p, v0, v1, v2, w);
                     };
-                    const MzPropsOut o = mz_props_wave<MZ_PROPS_AHEAD>(get, jtot, A.mass);
+                    const MzPropsOut o = mz_props_wave<4>(get, jtot, A.mass);
                     if (lane == 0) {
                         const int64_t ix = (int64_t)A.sidx * A.n_cells + cj;
                         A.out_np[ix] = (double)jtot;

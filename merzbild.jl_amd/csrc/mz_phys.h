@@ -332,10 +332,12 @@ struct MzPropsOut {
 };
 
 // One load a pass left a wave waiting on memory: a cell of 20,000 particles took
-// 100 us a step, about 35 us with eight loads of a lane in flight (k_batch0d, one
-// wave on the cell; 2,048 uneven cells, 50 steps: 29.3 -> 25.7 ms).  Kernels
-// that are short of registers, with cells of a few hundred particles, keep 1.
-#define MZ_PROPS_AHEAD 8
+// 59 us a call, 26 us with eight loads of a lane in flight (mz_props).
+// The batched pass takes four: 64 cells of 20 to 20,000 particles 161 -> 131 us
+// a step (eight: 128), cells of up to 300 particles no slower than with one
+// (eight: 2 to 3 percent slower, the loop's code beside the collisions').
+// Kernels that are short of registers, with cells of a few hundred particles,
+// keep 1.
 template <int AHEAD = 1, class Get>
 __device__ inline MzPropsOut mz_props_wave(const Get &get, int32_t tot, double mass) {
     const int lane = threadIdx.x & 63;
@@ -355,7 +357,9 @@ __device__ inline MzPropsOut mz_props_wave(const Get &get, int32_t tot, double m
     };
     int32_t i = lane;
     if (AHEAD > 1) {
-        for (; i + 64 * (AHEAD - 1) < tot; i += 64 * AHEAD) {
+        // blocks that every lane is in (one that some are in would run beside
+        // the others' single loads)
+        for (; i - lane + 64 * AHEAD <= tot; i += 64 * AHEAD) {
             double w[AHEAD], v0[AHEAD], v1[AHEAD], v2[AHEAD];
 #pragma unroll
             for (int k = 0; k < AHEAD; ++k) get(i + 64 * k, w[k], v0[k], v1[k], v2[k]);

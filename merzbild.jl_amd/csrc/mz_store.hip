@@ -1873,7 +1873,7 @@ __global__ void __launch_bounds__(256) k_props(MzViews views, int32_t n_cells, i
         const int64_t p = i < n1 ? (int64_t)st1 + i : (int64_t)st2 + (i - n1);
         w = sp.w[p]; v0 = sp.v0[p]; v1 = sp.v1[p]; v2 = sp.v2[p];
     };
-    const MzPropsOut o = mz_props_wave<MZ_PROPS_AHEAD>(get, tot, masses[sidx]);
+    const MzPropsOut o = mz_props_wave<8>(get, tot, masses[sidx]);
     if (lane == 0) {
         const int64_t ix = (int64_t)sidx * n_cells + c;
         out_np[ix] = (double)tot;
